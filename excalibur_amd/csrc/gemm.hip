@@ -1,13 +1,17 @@
 // Dense GEMM on the gfx950 matrix cores: C = alpha * op(A) op(B) + beta * C, row-major, FP64
 // (v_mfma_f64_16x16x4_f64) and FP32 (v_mfma_f32_16x16x4_f32).
 //
-// Workgroup tile 128 x 128, four wavefronts in a 2 x 2 arrangement, each wavefront a 64 x 64
-// block of 4 x 4 MFMA tiles; K is staged through LDS in chunks of 16 with register
-// double-buffering of the next chunk. Options used by the factorizations: split-K (partial tiles
-// summed in a fixed order by a second kernel, so results do not depend on scheduling), skipping
-// the zero K range of a triangular operand, and computing only the lower tiles of a symmetric
-// product (mirrored into the upper half by the reduction).
+// Workgroup tiles of 128 x 128 and 64 x 64, chosen per product (gemm_plan); K is staged through
+// registers into LDS in steps of 16, one step ahead of the one being multiplied and two ahead of the
+// loads. Bound by the MFMAs: FP64 67.9 TFLOP/s at order 4096 and 61.4 on 1000 x 50000 x 1000 (the
+// MFMA loop alone 78, the vendor library 71 and 59), FP32 134 at order 8192 and 130 on 2000 x 100000
+// x 2000 (156 alone, 149 the library); with scalar loads behind branches, whose merged registers
+// waited for every load at once, 55 and 46.6, 111 and 105. Options used by the factorizations: split-K
+// (partial tiles summed in a fixed order by a second kernel, so results do not depend on
+// scheduling), skipping the zero K range of a triangular operand, and computing only the lower
+// tiles of a symmetric product (mirrored into the upper half by the reduction).
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -42,7 +46,6 @@ struct Mfma<float> {
   __device__ static inline int row(int lk, int v) { return 4 * lk + v; }
 };
 
-constexpr int BM = 128, BN = 128, BK = 16, NT = 256;
 
 struct GemmArgs {
   int ta, tb;
@@ -56,10 +59,12 @@ struct GemmArgs {
   double alpha, beta;
   int tri;        // EXC_TRI_* restriction of the K range per tile
   int lower_only; // compute only tiles with tile_row >= tile_col
-  long kchunk;    // split-K chunk (multiple of BK); 0 = no split
+  long kchunk;    // split-K chunk (multiple of the K step); 0 = no split
   void* part;     // split-K partials: splits x M x N (type T)
+  int bm, bn;     // tile sizes
   long tm;        // tile rows
   long ntile;     // tiles per split (tm x tn, or the lower tiles tm (tm + 1) / 2)
+  int pair;       // a workgroup takes the tile rows r and tm - 1 - r (op(A) triangular)
   long total;     // ntile x splits = the 1-D grid
 };
 
@@ -87,191 +92,426 @@ __device__ inline void tile_of(const GemmArgs& g, long& tile_m, long& tile_n, lo
     tile_n = n;
     tile_m = n + u;
   } else {
-    tile_n = u / g.tm;
-    tile_m = u - tile_n * g.tm;
+    const long rows = g.pair ? (g.tm + 1) / 2 : g.tm;
+    tile_n = u / rows;
+    tile_m = u - tile_n * rows;
   }
 }
 
-// K range [k0, k1) that can contribute to output rows [i0, i0+BM) / columns [j0, j0+BN).
-__device__ inline void k_range(const GemmArgs& g, long i0, long j0, long& k0, long& k1) {
+// K range [k0, k1) that can contribute to output rows [i0, i0+bm) / columns [j0, j0+bn).
+__device__ inline void k_range(const GemmArgs& g, long i0, long j0, int bm, int bn, long& k0, long& k1) {
   k0 = 0;
   k1 = g.K;
   switch (g.tri) {
-    case EXC_TRI_A_LOWER: k1 = min(k1, i0 + BM); break;  // op(A)[i][k] = 0 for k > i
+    case EXC_TRI_A_LOWER: k1 = min(k1, i0 + bm); break;  // op(A)[i][k] = 0 for k > i
     case EXC_TRI_A_UPPER: k0 = max(k0, i0); break;       // op(A)[i][k] = 0 for k < i
     case EXC_TRI_B_LOWER: k0 = max(k0, j0); break;       // op(B)[k][j] = 0 for k < j
-    case EXC_TRI_B_UPPER: k1 = min(k1, j0 + BN); break;  // op(B)[k][j] = 0 for k > j
+    case EXC_TRI_B_UPPER: k1 = min(k1, j0 + bn); break;  // op(B)[k][j] = 0 for k > j
     default: break;
   }
 }
 
-// One k-chunk of A and B (BM x BK and BK x BN) staged through registers into LDS. The per-thread
-// element coordinates do not change between chunks: for a non-transposed A every thread owns one
-// k column (tid % 16) of 8 rows 16 apart; for a transposed A one row (tid % 128) of 8 k steps 2
-// apart (and likewise for B), so each chunk is 8 loads at a fixed stride from one base pointer.
-template <typename T, int TA, int TB>
-struct Stager {
-  const T* pa;  // base of this thread's A elements at k = 0
-  const T* pb;
-  long sa, sb;  // stride between the thread's 8 elements
-  long ka, kb;  // stride of one k step
-  int ai, ak, bj, bk;  // LDS coordinates of element q = 0 (q advances ai or ak by 16 / 2)
-  __device__ Stager(const GemmArgs& g, long i0, long j0, int tid) {
-    if (!TA) { ai = tid >> 4; ak = tid & 15; pa = (const T*)g.A + (i0 + ai) * g.lda + ak; sa = 16 * g.lda; ka = 1; }
-    else { ak = tid >> 7; ai = tid & 127; pa = (const T*)g.A + (long)ak * g.lda + i0 + ai; sa = 2 * g.lda; ka = g.lda; }
-    if (!TB) { bk = tid >> 7; bj = tid & 127; pb = (const T*)g.B + (long)bk * g.ldb + j0 + bj; sb = 2 * g.ldb; kb = g.ldb; }
-    else { bj = tid >> 4; bk = tid & 15; pb = (const T*)g.B + (j0 + bj) * g.ldb + bk; sb = 16 * g.ldb; kb = 1; }
-  }
-  __device__ inline int a_i(int q) const { return TA ? ai : ai + 16 * q; }
-  __device__ inline int a_k(int q) const { return TA ? ak + 2 * q : ak; }
-  __device__ inline int b_j(int q) const { return TB ? bj + 16 * q : bj; }
-  __device__ inline int b_k(int q) const { return TB ? bk : bk + 2 * q; }
+// 16 bytes of one operand, in registers and in LDS; in global memory only the elements' own
+// alignment is assumed (gfx950 loads unaligned 16-byte words).
+template <typename T>
+struct Unit;
+template <>
+struct Unit<double> {
+  typedef double lds_t __attribute__((ext_vector_type(2)));
+  typedef double glb_t __attribute__((ext_vector_type(2), aligned(8)));
+};
+template <>
+struct Unit<float> {
+  typedef float lds_t __attribute__((ext_vector_type(4)));
+  typedef float glb_t __attribute__((ext_vector_type(4), aligned(4)));
 };
 
-// One output tile [i0, i0+BM) x [j0, j0+BN) over the K range [k0, k1). The result element (gi, gj)
+// Shape of the kernel: WM x WN wavefronts, each MT x NT MFMA tiles, K staged in steps of kRow bytes'
+// worth of elements per operand row.
+template <typename T, int WM_, int WN_, int MT_, int NT_, int PER, bool FIRST, int KV_>
+struct Shape {
+  using elem = T;
+  static constexpr int WM = WM_, WN = WN_, MT = MT_, NT = NT_;
+  static constexpr int BM = 16 * WM * MT, BN = 16 * WN * NT;
+  static constexpr int kThreads = 64 * WM * WN;
+  static constexpr bool FRAGS_FIRST = FIRST;  // a step's first fragments are read before its stores
+  static constexpr int V = 16 / (int)sizeof(T);        // elements of a 16-byte unit
+  static constexpr int kRow = sizeof(T) == 8 ? 128 : 64;  // bytes of K per row and step
+  static constexpr int UNITS = kRow / 16;
+  static constexpr int BK = kRow / (int)sizeof(T);
+  static constexpr int KV = KV_;                        // consecutive k of a lane in a fragment (1 or V)
+  static constexpr int GROUPS = BK / (4 * KV);          // a group: KV MFMA steps of 4 k each
+  static constexpr int kPerCu = PER;  // resident workgroups (registers and LDS)
+};
+
+// One operand's slab of a step, E rows (or columns) by BK, staged through registers into
+// LDS as 16-byte units. KMAJ: the operand is contiguous along k in memory (A, or B transposed); LDS
+// holds [row][unit of k] with the unit index XORed by the row, so the 16 rows a fragment read
+// touches fall into different banks. Otherwise it is contiguous along the rows (A transposed, or
+// B) and LDS holds [k][unit of rows], whose fragment reads are whole 256-byte lines.
+//
+// The contraction may run over k in any order that both operands share. With KV = V the lane group
+// lk = lane / 16 takes the V consecutive k of unit lk + 4 g, one per MFMA step, so that one 16-byte
+// LDS read feeds V steps; with KV = 1 it takes k = lk + 4 g, which sums in ascending order as
+// LAPACK's reference does (the 64 x 64 FP64 tile, the one of small matrices: 2 % slower). Where the
+// operand is not KMAJ a read feeds up to V MFMA tiles, whose rows interleave (row_of).
+//
+// A load is branch-free: its coordinates are clamped into the operand, and what that shifted or
+// repeated is put right when the registers are stored (fix). A branch around a load merges two
+// definitions of its registers, and the copies that takes wait for the load on the spot.
+template <typename T, bool KMAJ, int E, int TT, int UNITS, int KV, int kThreads>
+struct Slab {
+  typedef typename Unit<T>::lds_t lv;
+  typedef typename Unit<T>::glb_t gv;
+  static constexpr int V = 16 / (int)sizeof(T);
+  static constexpr int Q = E * UNITS / kThreads;    // units per thread
+  static constexpr int UPR = KMAJ ? UNITS : E / V;  // units of one LDS row
+  static constexpr int STEP = kThreads / UPR;       // rows between a thread's units
+  static constexpr int VT = TT < V ? TT : V;        // interleaved MFMA tiles (not KMAJ)
+  static constexpr int NP = KMAJ ? Q : 1;
+  const T* p[NP];  // KMAJ: this thread's rows at k = 0; else its column at k = 0
+  long ld;
+  long e0, ext;    // first row of the slab, rows of the operand
+  int r0, u;       // first LDS row and unit of this thread
+  int sh;          // not KMAJ: elements the clamp moved the unit down by
+  lv reg[Q];
+
+  __device__ Slab(const void* P, long ld_, long e0_, long ext_, int tid) : ld(ld_), e0(e0_), ext(ext_) {
+    r0 = tid / UPR;
+    u = tid % UPR;
+    sh = 0;
+    if (KMAJ) {
+#pragma unroll
+      for (int q = 0; q < NP; q++) p[q] = (const T*)P + min(e0 + r0 + q * STEP, ext - 1) * ld;
+    } else {
+      const long c = e0 + (long)u * V, last = max(ext - V, 0L);
+      p[0] = (const T*)P + min(c, last);
+      sh = (int)min(max(c - last, 0L), (long)V);
+    }
+  }
+  // The step at kb of the range that ends at k1 (k1 >= V; not KMAJ: ext >= V). What depends on the
+  // thread is kept in 32 bits, relative to the step: the registers decide how many workgroups
+  // are resident.
+  __device__ __forceinline__ void load(long kb, long k1) {
+    if (KMAJ) {
+      const int k = min(u * V, near(k1 - V - kb));
+#pragma unroll
+      for (int q = 0; q < Q; q++) reg[q] = *(const gv*)(p[q % NP] + kb + k);
+    } else {
+      const int last = near(k1 - 1 - kb);
+      const T* s = p[0] + kb * ld;
+#pragma unroll
+      for (int q = 0; q < Q; q++) reg[q] = *(const gv*)(s + min(r0 + q * STEP, last) * ld);
+    }
+  }
+  // a (uniform) distance, saturated far beyond any step
+  __device__ static __forceinline__ int near(long d) { return (int)max(min(d, 1L << 24), -(1L << 24)); }
+  // The same step element by element, for operands too small for a unit.
+  __device__ __forceinline__ void load_checked(long kb, long k1) {
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      lv x;
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        const long row = KMAJ ? e0 + r0 + q * STEP : e0 + (long)u * V + v;
+        const long k = KMAJ ? kb + u * V + v : kb + r0 + q * STEP;
+        T e = T(0);
+        if (row < ext && k < k1) e = KMAJ ? p[q % NP][k] : p[0][k * ld + (row - min(e0 + (long)u * V, max(ext - V, 0L)))];
+        x[v] = e;
+      }
+      reg[q] = x;
+    }
+  }
+  // Elements moved down by s places, zeros behind them (s >= V: all zero).
+  __device__ static __forceinline__ lv shifted(lv x, int s) {
+    lv y;
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      T e = T(0);
+#pragma unroll
+      for (int w = v; w < V; w++) e = w - v == s ? x[w] : e;
+      y[v] = e;
+    }
+    return y;
+  }
+  // Puts right what the clamps of load did: the step's elements at or beyond k1 become zero.
+  __device__ __forceinline__ void fix(long kb, long k1) {
+    const int left = near(k1 - kb);
+    const int s = KMAJ ? min(max(u * V + V - left, 0), V) : sh;
+#pragma unroll
+    for (int q = 0; q < Q; q++) reg[q] = shifted(reg[q], !KMAJ && r0 + q * STEP >= left ? V : s);
+  }
+  // Whether every step needs fix (a unit straddles the end of the rows).
+  __device__ __forceinline__ bool ragged() const { return !KMAJ && e0 + E > ext && ext % V != 0; }
+  // Zeroes the elements on the far side of the diagonal: k > row (lower) or k < row (upper).
+  __device__ __forceinline__ void mask(long kb, bool lower) {
+    const int d = near(e0 - kb);
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      lv x = reg[q];
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        const int row = d + (KMAJ ? r0 + q * STEP : u * V + v);
+        const int k = KMAJ ? u * V + v : r0 + q * STEP;
+        const bool zero = lower ? k > row : k < row;
+        x[v] = zero ? T(0) : x[v];
+      }
+      reg[q] = x;
+    }
+  }
+  __device__ static inline int swz(int row) { return KMAJ ? (row / (16 / UNITS)) & (UNITS - 1) : 0; }
+  __device__ __forceinline__ void store(lv* lds) const {
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      const int r = r0 + q * STEP;
+      lds[r * UPR + (u ^ swz(r))] = reg[q];
+    }
+  }
+  // The wavefront's fragments of group g: f[v][t] is MFMA step v's element for tile t; w0 is the
+  // wavefront's first row of the slab.
+  __device__ static __forceinline__ void frag(const lv* lds, int w0, int g, int li, int lk, T (*f)[TT]) {
+    const int k0 = (lk + 4 * g) * KV;
+    const T* l = (const T*)lds;
+    if (KMAJ) {
+#pragma unroll
+      for (int t = 0; t < TT; t++) {
+        const int r = w0 + t * 16 + li;
+        const int at = r * UPR + ((k0 / V) ^ swz(r));
+        if (KV == V) {
+          const lv x = lds[at];
+#pragma unroll
+          for (int v = 0; v < KV; v++) f[v][t] = x[v];
+        } else {
+          f[0][t] = l[at * V + k0 % V];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int v = 0; v < KV; v++) {
+        const T* line = l + (k0 + v) * E + w0;
+#pragma unroll
+        for (int t = 0; t < TT; t += VT) {
+          if (VT == V) {
+            const lv x = *(const lv*)(line + t * 16 + li * VT);
+#pragma unroll
+            for (int z = 0; z < VT; z++) f[v][t + z] = x[z];
+          } else {
+#pragma unroll
+            for (int z = 0; z < VT; z++) f[v][t + z] = line[t * 16 + li * VT + z];
+          }
+        }
+      }
+    }
+  }
+  // Row of the wavefront's block that element r of MFMA tile t stands for.
+  __device__ static __forceinline__ int row_of(int t, int r) {
+    return KMAJ ? t * 16 + r : (t / VT) * 16 * VT + r * VT + t % VT;
+  }
+};
+
+// The 128 x 128 and 64 x 64 workgroup tiles. kStep: measured time of a step on a CU with its
+// resident workgroups (us per workgroup), kAlone: with one workgroup on the CU. The MFMAs alone take
+// 1.73 / 0.43 us in FP64 and 0.86 / 0.22 us in FP32. The FP64 tile is split over eight wavefronts
+// (65.9 TFLOP/s at order 4096, 63.7 with four of 64 x 64, whose 256 registers leave two wavefronts
+// per SIMD); in FP32 four reach 129.5 at order 8192, eight 122.4. kMaxSum: terms of one running sum
+// (its rounding error grows with them) beyond which K is split as far as the workspace allows and,
+// in FP64 (kMaxSumFills), as far as two workgroups per CU (and a plan that stays above it counts 10 % more).
+template <typename T>
+struct Shapes;
+template <>
+struct Shapes<double> {
+  using Big = Shape<double, 4, 2, 2, 4, 2, false, 2>;
+  using Small = Shape<double, 2, 2, 2, 2, 4, true, 1>;
+  static constexpr double kStep[2] = {1.98, 0.54}, kAlone[2] = {2.09, 0.73};
+  static constexpr long kMaxSum = 256;
+  static constexpr bool kMaxSumFills = true;
+};
+template <>
+struct Shapes<float> {
+  using Big = Shape<float, 2, 2, 4, 4, 3, true, 4>;
+  using Small = Shape<float, 2, 2, 2, 2, 4, true, 4>;
+  static constexpr double kStep[2] = {1.00, 0.287}, kAlone[2] = {1.18, 0.52};
+  static constexpr long kMaxSum = 2048;
+  static constexpr bool kMaxSumFills = false;
+};
+
+template <class S>
+struct Tiles {
+  typename Unit<typename S::elem>::lds_t a[2][S::BM * S::UNITS];
+  typename Unit<typename S::elem>::lds_t b[2][S::BN * S::UNITS];
+};
+
+// One output tile [i0, i0+BM) x [j0, j0+BN) over the K range [k0, k1), k0 a multiple of BK. The result element (gi, gj)
 // goes to Cb[(gi - ci0) * ldc + (gj - cj0)]: scaled by alpha (plus beta times the old value) when
 // direct, else stored as it is (a split-K partial).
-template <typename T, int TA, int TB>
+//
+// Step c's products read one LDS buffer while the registers, loaded during step c - 1, are stored
+// into the other and refilled with step c + 2's loads: a load has a whole step to arrive, and the
+// barrier that ends a step waits for no memory. (The stores and loads past the last step, of
+// clamped addresses, are not read.)
+template <typename T, int TA, int TB, bool TRI, class S>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, long i0, long j0, long k0, long k1, T* Cb, long ldc,
-                                          long ci0, long cj0, bool direct, T (*As)[BK][BM + 1],
-                                          T (*Bs)[BK][BN + 1]) {
+                                          long ci0, long cj0, bool direct, Tiles<S>& lds) {
   using acc_t = typename Mfma<T>::acc_t;
+  constexpr int BK = S::BK, V = S::V, MT = S::MT, NT = S::NT;
+  using SA = Slab<T, !TA, S::BM, MT, S::UNITS, S::KV, S::kThreads>;
+  using SB = Slab<T, (bool)TB, S::BN, NT, S::UNITS, S::KV, S::kThreads>;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
-  const Stager<T, TA, TB> st(g, i0, j0, tid);
-  // interior tile: no row or column bounds, chunks aligned to BK. A whole chunk of it then loads
-  // without checks unless it crosses the diagonal of a triangular operand (the k range already
-  // excludes the chunks wholly on the zero side), so only such chunks and a last partial chunk
-  // check their elements.
-  const bool interior = i0 + BM <= g.M && j0 + BN <= g.N && (k0 % BK) == 0;
-  auto fast = [&](long kb) {
-    if (!interior || kb + BK > k1) return false;
-    switch (g.tri) {
-      case EXC_TRI_A_LOWER: return kb + BK <= i0 + 1;       // every k <= i0 <= row
-      case EXC_TRI_A_UPPER: return kb >= i0 + BM - 1;       // every k >= last row
-      case EXC_TRI_B_LOWER: return kb >= j0 + BN - 1;       // every k >= last column
-      case EXC_TRI_B_UPPER: return kb + BK <= j0 + 1;       // every k <= j0 <= column
-      default: return true;
-    }
-  };
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  acc_t acc[4][4];
-#pragma unroll
-  for (int a = 0; a < 4; a++)
-#pragma unroll
-    for (int b = 0; b < 4; b++) acc[a][b] = acc_t{0, 0, 0, 0};
-  T ra[8], rb[8];
-  auto load_fast = [&](long kbase) {
-    const T* pa = st.pa + kbase * st.ka;
-    const T* pb = st.pb + kbase * st.kb;
-#pragma unroll
-    for (int q = 0; q < 8; q++) ra[q] = pa[q * st.sa];
-#pragma unroll
-    for (int q = 0; q < 8; q++) rb[q] = pb[q * st.sb];
-  };
-  auto load_checked = [&](long kbase) {
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const long gi = i0 + st.a_i(q), gk = kbase + st.a_k(q);
-      T v = T(0);
-      if (gi < g.M && gk >= k0 && gk < k1) v = st.pa[kbase * st.ka + q * st.sa];
-      if ((g.tri == EXC_TRI_A_LOWER && gk > gi) || (g.tri == EXC_TRI_A_UPPER && gk < gi)) v = T(0);
-      ra[q] = v;
-      const long gj = j0 + st.b_j(q), gk2 = kbase + st.b_k(q);
-      T w = T(0);
-      if (gj < g.N && gk2 >= k0 && gk2 < k1) w = st.pb[kbase * st.kb + q * st.sb];
-      if ((g.tri == EXC_TRI_B_LOWER && gk2 < gj) || (g.tri == EXC_TRI_B_UPPER && gk2 > gj)) w = T(0);
-      rb[q] = w;
-    }
-  };
-  auto store_chunk = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < 8; q++) As[buf][st.a_k(q)][st.a_i(q)] = ra[q];
-#pragma unroll
-    for (int q = 0; q < 8; q++) Bs[buf][st.b_k(q)][st.b_j(q)] = rb[q];
-  };
-  const long kstart = (k0 / BK) * BK;
-  int buf = 0;
-  if (kstart < k1) {
-    if (fast(kstart)) load_fast(kstart);
-    else load_checked(kstart);
-    store_chunk(0);
-  }
-  __syncthreads();
   const int li = lane & 15, lk = lane >> 4;
-  for (long kb = kstart; kb < k1; kb += BK) {
-    const bool more = kb + BK < k1;
-    if (more) {
-      if (fast(kb + BK)) load_fast(kb + BK);
-      else load_checked(kb + BK);
+  const int wm = (wave / S::WN) * 16 * MT, wn = (wave % S::WN) * 16 * NT;
+  SA sa(g.A, g.lda, i0, g.M, tid);
+  SB sb(g.B, g.ldb, j0, g.N, tid);
+  acc_t acc[MT][NT];
+#pragma unroll
+  for (int a = 0; a < MT; a++)
+#pragma unroll
+    for (int b = 0; b < NT; b++) acc[a][b] = acc_t{0, 0, 0, 0};
+  // the last step of a range that ends inside it, operands whose rows end inside a unit, and a
+  // triangular operand's steps that cross its diagonal (the k range already excludes the steps
+  // wholly on the zero side) are put right between their load and their store
+  const bool ragged_a = sa.ragged(), ragged_b = sb.ragged();
+  auto store = [&](long kb, int buf, bool fix) __attribute__((always_inline)) {
+    if (fix) {
+      const bool tail = kb + BK > k1;
+      if (tail || ragged_a) sa.fix(kb, k1);
+      if (tail || ragged_b) sb.fix(kb, k1);
     }
-#pragma unroll
-    for (int ks = 0; ks < BK; ks += 4) {
-      T af[4], bf[4];
-#pragma unroll
-      for (int a = 0; a < 4; a++) af[a] = As[buf][ks + lk][wm + a * 16 + li];
-#pragma unroll
-      for (int b = 0; b < 4; b++) bf[b] = Bs[buf][ks + lk][wn + b * 16 + li];
-#pragma unroll
-      for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = Mfma<T>::step(af[a], bf[b], acc[a][b]);
+    if (TRI) {
+      switch (g.tri) {
+        case EXC_TRI_A_LOWER: if (kb + BK > i0 + 1) sa.mask(kb, true); break;
+        case EXC_TRI_A_UPPER: if (kb < i0 + S::BM - 1) sa.mask(kb, false); break;
+        case EXC_TRI_B_LOWER: if (kb < j0 + S::BN - 1) sb.mask(kb, false); break;
+        case EXC_TRI_B_UPPER: if (kb + BK > j0 + 1) sb.mask(kb, true); break;
+        default: break;
+      }
     }
-    if (more) {
-      store_chunk(buf ^ 1);
-      __syncthreads();
+    sa.store(lds.a[buf]);
+    sb.store(lds.b[buf]);
+  };
+  T fa[S::KV][MT], fb[S::KV][NT];
+  auto frags = [&](int buf, int gr) __attribute__((always_inline)) {
+    SA::frag(lds.a[buf], wm, gr, li, lk, fa);
+    SB::frag(lds.b[buf], wn, gr, li, lk, fb);
+  };
+  auto products = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int v = 0; v < S::KV; v++)
+#pragma unroll
+      for (int a = 0; a < MT; a++)
+#pragma unroll
+        for (int b = 0; b < NT; b++) acc[a][b] = Mfma<T>::step(fa[v][a], fb[v][b], acc[a][b]);
+  };
+  if (g.K < V || (TA && g.M < V) || (!TB && g.N < V)) {
+    for (long kb = k0; kb < k1; kb += BK) {
+      sa.load_checked(kb, k1);
+      sb.load_checked(kb, k1);
+      store(kb, 0, false);
+      lds_barrier();
+#pragma unroll
+      for (int gr = 0; gr < S::GROUPS; gr++) {
+        frags(0, gr);
+        products();
+      }
+      lds_barrier();
+    }
+  } else if (k0 < k1) {
+    sa.load(k0, k1);
+    sb.load(k0, k1);
+    store(k0, 0, true);
+    sa.load(k0 + BK, k1);
+    sb.load(k0 + BK, k1);
+    lds_barrier();
+    int buf = 0;
+    for (long kb = k0; kb < k1; kb += BK) {
+      if (S::FRAGS_FIRST) frags(buf, 0);
+      store(kb + BK, buf ^ 1, true);
+      sa.load(kb + 2 * BK, k1);
+      sb.load(kb + 2 * BK, k1);
+      if (!S::FRAGS_FIRST) frags(buf, 0);
+      products();
+#pragma unroll
+      for (int gr = 1; gr < S::GROUPS; gr++) {
+        frags(buf, gr);
+        products();
+      }
+      lds_barrier();
       buf ^= 1;
     }
   }
-  // epilogue: operands were supplied as A[lane%16][lane/16], B[lane/16][lane%16]
-  T* C = Cb;
+  // epilogue: operands were supplied as A[lane%16][lane/16], B[lane/16][lane%16]. The VN
+  // interleaved tiles of a B that is contiguous along n hold consecutive columns: one store.
   const T alpha = (T)g.alpha, beta = (T)g.beta;
+  constexpr int VN = TB ? 1 : SB::VT;
+  typedef T cv __attribute__((ext_vector_type(VN == 1 ? 2 : VN), aligned(sizeof(T))));
 #pragma unroll
-  for (int a = 0; a < 4; a++)
+  for (int a = 0; a < MT; a++)
 #pragma unroll
-    for (int b = 0; b < 4; b++)
+    for (int b = 0; b < NT; b += VN)
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        const long gi = i0 + wm + a * 16 + Mfma<T>::row(lk, v);
-        const long gj = j0 + wn + b * 16 + li;
-        if (gi < g.M && gj < g.N) {
-          const T val = acc[a][b][v];
-          T* cp = C + (gi - ci0) * ldc + (gj - cj0);
-          if (direct) {
-            T out = alpha * val;
-            if (g.beta != 0.0) out += beta * *cp;
-            *cp = out;
-          } else {
-            *cp = val;
+        const long gi = i0 + wm + SA::row_of(a, Mfma<T>::row(lk, v));
+        const long gj = j0 + wn + SB::row_of(b, li);
+        if (gi >= g.M || gj >= g.N) continue;
+        T* cp = Cb + (gi - ci0) * ldc + (gj - cj0);
+        if (VN > 1 && gj + VN <= g.N) {
+          cv out;
+#pragma unroll
+          for (int z = 0; z < VN; z++) out[z] = direct ? alpha * acc[a][b + z][v] : acc[a][b + z][v];
+          if (direct && g.beta != 0.0) {
+            const cv old = *(const cv*)cp;
+#pragma unroll
+            for (int z = 0; z < VN; z++) out[z] += beta * old[z];
           }
+          *(cv*)cp = out;
+        } else {
+#pragma unroll
+          for (int z = 0; z < VN; z++)
+            if (gj + z < g.N) {
+              T out = direct ? alpha * acc[a][b + z][v] : acc[a][b + z][v];
+              if (direct && g.beta != 0.0) out += beta * cp[z];
+              cp[z] = out;
+            }
         }
       }
 }
 
-template <typename T, int TA, int TB>
-__global__ __launch_bounds__(NT, 2) void k_gemm(GemmArgs g) {
-  __shared__ T As[2][BK][BM + 1];
-  __shared__ T Bs[2][BK][BN + 1];
+// TRI: one operand is triangular. The general products are a kernel of their own: the triangle's
+// code in their loop costs registers, and with them 5 % of their rate.
+template <typename T, int TA, int TB, bool TRI, class S>
+__global__ __launch_bounds__(S::kThreads, S::kPerCu * S::kThreads / 256) void k_gemm(GemmArgs g) {
+  __shared__ Tiles<S> lds;
   long tile_m, tile_n, split;
   tile_of(g, tile_m, tile_n, split);
-  const long i0 = tile_m * BM, j0 = tile_n * BN;
-  long k0, k1;
-  k_range(g, i0, j0, k0, k1);
-  if (g.kchunk > 0) {
-    const long ks = split * g.kchunk;
-    k0 = max(k0, ks);
-    k1 = min(k1, ks + g.kchunk);
-  }
+  const long j0 = tile_n * S::BN;
   T* Cb = g.kchunk > 0 ? (T*)g.part + (size_t)split * g.M * g.N : (T*)g.C;
   const long ldc = g.kchunk > 0 ? g.N : g.ldc;
-  gemm_tile<T, TA, TB>(g, i0, j0, k0, k1, Cb, ldc, 0, 0, g.kchunk == 0, As, Bs);
+  const long ks = split * g.kchunk, ke = g.kchunk > 0 ? min(g.K, ks + g.kchunk) : g.K;
+  if (!TRI) {
+    gemm_tile<T, TA, TB, false, S>(g, tile_m * S::BM, j0, ks, ke, Cb, ldc, 0, 0, g.kchunk == 0, lds);
+    return;
+  }
+  for (;;) {
+    long k0, k1;
+    k_range(g, tile_m * S::BM, j0, S::BM, S::BN, k0, k1);
+    k0 = max(k0, ks);
+    k1 = min(k1, ke);
+    gemm_tile<T, TA, TB, true, S>(g, tile_m * S::BM, j0, k0, k1, Cb, ldc, 0, 0, g.kchunk == 0, lds);
+    // a triangular op(A) gives row r of the tiles a K range that grows or shrinks with r: rows r and
+    // tm - 1 - r together are the same work for every workgroup
+    if (!g.pair || 2 * tile_m >= g.tm - 1) break;  // the second of a pair, or the middle row
+    tile_m = g.tm - 1 - tile_m;
+    lds_barrier();  // the next tile restages the slabs
+  }
 }
 
 // Grouped products: many independent problems of one transposition pattern in one launch. The
-// host lays out work items (problem, tile, K range, partial slot); a persistent grid strides over
-// them, each item running the same tile code as k_gemm. Items of a tile split over K (or of a
-// mirrored symmetric product) store partial tiles; k_grouped_reduce then sums each tile's
-// partials in slot order (deterministic), applies alpha and beta, and mirrors lower tiles.
+// host lays out work items (problem, tile or pair of tiles, K range, partial slot), one workgroup
+// each, running the same tile code as k_gemm; the dispatcher balances them over the CUs (a grid that
+// strode over them by itself gave every workgroup a fixed share, whatever its items' lengths).
+// Items of a tile split over K (or of a mirrored symmetric product) store partial tiles;
+// k_grouped_reduce then sums each tile's partials in slot order (deterministic), applies alpha
+// and beta, and mirrors lower tiles.
 struct GroupProb {
   const void* A;
   const void* B;
@@ -281,32 +521,46 @@ struct GroupProb {
 };
 struct GroupItem {
   int p, tile_m, tile_n, slot;  // slot < 0: the item owns its whole tile and stores it directly
+  int other_m, pad;             // >= 0: tile row it takes as well (a triangular op(A), see k_gemm)
   long k0, k1;
 };
 struct GroupRed {
   int p, tile_m, tile_n, first_slot, nslots, pad;
 };
 
-template <typename T, int TA, int TB>
-__global__ __launch_bounds__(NT, 2) void k_gemm_grouped(const GroupProb* __restrict__ probs,
-                                                        const GroupItem* __restrict__ items, long nitems,
-                                                        T* __restrict__ part, double alpha, double beta) {
-  __shared__ T As[2][BK][BM + 1];
-  __shared__ T Bs[2][BK][BN + 1];
-  for (long it = blockIdx.x; it < nitems; it += gridDim.x) {
-    const GroupItem w = items[it];
-    const GroupProb pr = probs[w.p];
-    GemmArgs g{};
-    g.A = pr.A; g.lda = pr.lda; g.B = pr.B; g.ldb = pr.ldb; g.M = pr.M; g.N = pr.N; g.K = pr.K;
-    g.tri = pr.tri; g.alpha = alpha; g.beta = beta;
-    const long i0 = (long)w.tile_m * BM, j0 = (long)w.tile_n * BN;
-    long k0, k1;
-    k_range(g, i0, j0, k0, k1);
-    k0 = max(k0, w.k0);
-    k1 = min(k1, w.k1);
-    if (w.slot < 0) gemm_tile<T, TA, TB>(g, i0, j0, k0, k1, (T*)pr.C, pr.ldc, 0, 0, true, As, Bs);
-    else gemm_tile<T, TA, TB>(g, i0, j0, k0, k1, part + (size_t)w.slot * BM * BN, BN, i0, j0, false, As, Bs);
-    __syncthreads();  // the next item restages the LDS tiles
+template <typename T>
+using GroupShape = typename Shapes<T>::Big;
+constexpr int kGroupBM = 128, kGroupBN = 128;
+
+template <typename T, int TA, int TB, bool TRI>
+__global__ __launch_bounds__(GroupShape<T>::kThreads, GroupShape<T>::kPerCu * GroupShape<T>::kThreads / 256) void k_gemm_grouped(
+    const GroupProb* __restrict__ probs, const GroupItem* __restrict__ items, long nitems, T* __restrict__ part,
+    double alpha, double beta) {
+  constexpr int BM = kGroupBM, BN = kGroupBN;
+  __shared__ Tiles<GroupShape<T>> lds;
+  // each die takes a contiguous range of the items, as in tile_of
+  const long L = blockIdx.x, q = nitems / kXcds, r = nitems % kXcds;
+  const GroupItem w = items[(L % kXcds) * q + min(L % kXcds, r) + L / kXcds];
+  const GroupProb pr = probs[w.p];
+  GemmArgs g{};
+  g.A = pr.A; g.lda = pr.lda; g.B = pr.B; g.ldb = pr.ldb; g.M = pr.M; g.N = pr.N; g.K = pr.K;
+  g.tri = pr.tri; g.alpha = alpha; g.beta = beta;
+  const bool direct = w.slot < 0;
+  const long j0 = (long)w.tile_n * BN;
+  T* Cb = direct ? (T*)pr.C : part + (size_t)w.slot * BM * BN;
+  for (int tile_m = w.tile_m;;) {
+    const long i0 = (long)tile_m * BM;
+    long k0 = w.k0, k1 = w.k1;
+    if (TRI) {
+      k_range(g, i0, j0, BM, BN, k0, k1);
+      k0 = max(k0, w.k0);
+      k1 = min(k1, w.k1);
+    }
+    gemm_tile<T, TA, TB, TRI, GroupShape<T>>(g, i0, j0, k0, k1, Cb, direct ? pr.ldc : BN, direct ? 0 : i0,
+                                             direct ? 0 : j0, direct, lds);
+    if (!TRI || w.other_m < 0 || tile_m == w.other_m) break;
+    tile_m = w.other_m;
+    lds_barrier();  // the next tile restages the slabs
   }
 }
 
@@ -317,13 +571,13 @@ __global__ __launch_bounds__(256) void k_grouped_reduce(const GroupProb* __restr
   const GroupRed r = reds[blockIdx.x];
   const GroupProb pr = probs[r.p];
   T* C = (T*)pr.C;
-  for (int e = threadIdx.x; e < BM * BN; e += blockDim.x) {
-    const int li = e / BN, lj = e - li * BN;
-    const long gi = (long)r.tile_m * BM + li, gj = (long)r.tile_n * BN + lj;
+  for (int e = threadIdx.x; e < kGroupBM * kGroupBN; e += blockDim.x) {
+    const int li = e / kGroupBN, lj = e - li * kGroupBN;
+    const long gi = (long)r.tile_m * kGroupBM + li, gj = (long)r.tile_n * kGroupBN + lj;
     if (gi >= pr.M || gj >= pr.N) continue;
     if (pr.lower_only && gj > gi) continue;  // the upper part of a diagonal tile comes by mirroring
     T s = T(0);
-    for (int q = 0; q < r.nslots; q++) s += part[(size_t)(r.first_slot + q) * BM * BN + e];
+    for (int q = 0; q < r.nslots; q++) s += part[(size_t)(r.first_slot + q) * kGroupBM * kGroupBN + e];
     T out = (T)alpha * s;
     if (beta != 0.0) out += (T)beta * C[gi * pr.ldc + gj];
     C[gi * pr.ldc + gj] = out;
@@ -338,7 +592,7 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs g, int splits) {
   const long total = g.M * g.N;
   if (idx >= total) return;
   const long i = idx / g.N, j = idx - i * g.N;
-  if (g.lower_only && (j / BN) > (i / BM)) return;
+  if (g.lower_only && (j / g.bn) > (i / g.bm)) return;
   const T* P = (const T*)g.part;
   T s = T(0);
   for (int z = 0; z < splits; z++) s += P[(size_t)z * total + idx];
@@ -357,18 +611,71 @@ __global__ __launch_bounds__(256) void k_mirror_lower(long n, T* C, long ldc) {
   if (j > i) C[i * ldc + j] = C[j * ldc + i];
 }
 
-// Workgroups of k_gemm resident at once on the current device: per_cu per CU (two for the FP64
-// kernel's 256 VGPRs and 64 KB of LDS, three for FP32), times the CU count (cached per device).
-long resident_slots(int per_cu) {
-  static int cus[64] = {0};
+// Compute units of the current device (cached per device).
+long compute_units() {
+  static std::atomic<int> cus[64];
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256L * per_cu;
-  if (cus[dev] <= 0) {
-    int n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cus[dev].load();
+  if (n <= 0) {
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev] = n;
+    cus[dev].store(n);
   }
-  return (long)cus[dev] * per_cu;
+  return n;
+}
+
+struct GemmPlan {
+  int tile;    // 128 or 64
+  int splits;  // of K
+};
+
+// Tile and split of one product: the pair with the least estimated time. A CU with w workgroups
+// takes max(w kStep, kAlone) per step; a split adds the write and the fixed-order sum of its partials
+// (about 5 TB/s, they stay in the caches) and 5 us for its launch. Splits need a workspace and keep
+// at least two steps each (a lone step is all latency); near ties go to the larger tile and fewer
+// splits.
+template <typename T>
+GemmPlan gemm_plan(long M, long N, long K, const ExcGemmOpts& o) {
+  constexpr int BK = Shapes<T>::Big::BK;
+  constexpr long kMaxSum = Shapes<T>::kMaxSum;
+  const long cus = compute_units();
+  GemmPlan best{128, 1};
+  double best_us = -1.0;
+  for (int c = 0; c < 2; c++) {
+    const long tile = c == 0 ? 128 : 64;
+    const long tm = (M + tile - 1) / tile, tn = (N + tile - 1) / tile;
+    const long tiles = o.lower_only ? tm * (tm + 1) / 2 : tm * tn;
+    // a triangular operand leaves the tiles about half of K on average
+    const double share = o.tri != EXC_TRI_NONE ? 0.5 + 0.5 / (double)(o.tri <= EXC_TRI_A_UPPER ? tm : tn) : 1.0;
+    const long slots = cus * (c == 0 ? Shapes<T>::Big::kPerCu : Shapes<T>::Small::kPerCu);
+    const double out = (double)sizeof(T) * M * N * (o.lower_only ? 0.5 : 1.0);
+    const long room = o.work && K > 4 * BK ? (long)std::min<size_t>(K / (2 * BK), o.work_bytes / ((size_t)M * N * sizeof(T))) : 1;
+    const long most = std::max(1L, std::min(room, 2 * ((slots + tiles - 1) / tiles)));
+    long least = std::min(room, (K + kMaxSum - 1) / kMaxSum);
+    if (Shapes<T>::kMaxSumFills) least = std::min(least, 2 * cus / tiles);
+    least = std::max(1L, least);
+    for (long sp = least; sp <= std::max(least, most); sp++) {
+      const long depth = ((K + sp - 1) / sp + BK - 1) / BK;
+      const long per_cu = (tiles * sp + cus - 1) / cus;
+      double us = 6.0 + depth * std::max(per_cu * Shapes<T>::kStep[c] * share, Shapes<T>::kAlone[c]);
+      if (sp > 1) us += 5.0 + (2 * sp + 1) * out / 5.0e6;
+      if (Shapes<T>::kMaxSumFills && K > sp * kMaxSum) us *= 1.1;
+      if (best_us < 0.0 || us < 0.99 * best_us) {
+        best_us = us;
+        best = GemmPlan{(int)tile, (int)sp};
+      }
+    }
+  }
+  return best;
+}
+
+template <typename T, bool TRI, class S>
+void gemm_launch(int ta, int tb, const GemmArgs& g, hipStream_t s) {
+  const dim3 grid((unsigned)g.total), block(S::kThreads);
+  if (!ta && !tb) hipLaunchKernelGGL((k_gemm<T, 0, 0, TRI, S>), grid, block, 0, s, g);
+  else if (!ta && tb) hipLaunchKernelGGL((k_gemm<T, 0, 1, TRI, S>), grid, block, 0, s, g);
+  else if (ta && !tb) hipLaunchKernelGGL((k_gemm<T, 1, 0, TRI, S>), grid, block, 0, s, g);
+  else hipLaunchKernelGGL((k_gemm<T, 1, 1, TRI, S>), grid, block, 0, s, g);
 }
 
 template <typename T>
@@ -380,31 +687,14 @@ int gemm_impl(int ta, int tb, long M, long N, long K, double alpha, const T* A, 
   g.ta = ta; g.tb = tb; g.M = M; g.N = N; g.K = K;
   g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc;
   g.alpha = alpha; g.beta = beta; g.tri = o.tri; g.lower_only = o.lower_only;
-  const long tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
-  long tiles = o.lower_only ? tm * (tm + 1) / 2 : tm * tn;
-  int splits = 1;
-  const long slots = resident_slots(sizeof(T) == 8 ? 2 : 3);
-  if (o.work && K > 4 * BK && tiles < slots) {
-    // Split K (only while the tiles alone leave resident slots idle) into the number of
-    // chunks that minimizes an estimate of the time: (rounds of resident workgroups) x (chunk
-    // depth) x ~3 us per 16-deep chunk (a workgroup alone on its CU waits on its loads), plus,
-    // when split, the fixed-order reduction: ~5 us and a read of every partial at ~3 TB/s. A grid
-    // just above the resident slots would run a second, nearly empty round; a large output
-    // would spend more summing partials than the split saves. Ties go to fewer splits.
-    const long maxs = std::min<long>(K / BK, 4 * ((slots + tiles - 1) / tiles));
-    long best = 1;
-    double best_cost = -1.0;
-    for (long sp = 1; sp <= std::max(1L, maxs); sp++) {
-      if (sp > 1 && (size_t)sp * M * N * sizeof(T) > o.work_bytes) break;
-      const long rounds = (tiles * sp + slots - 1) / slots;
-      const long depth = ((K + sp - 1) / sp + BK - 1) / BK;
-      double cost = 3.0 * (double)(rounds * depth);
-      if (sp > 1) cost += 5.0 + (double)sp * M * N * sizeof(T) / 3.0e6;
-      if (best_cost < 0.0 || cost < best_cost) { best = sp; best_cost = cost; }
-    }
-    splits = (int)best;
-  }
-  if (K == 0) splits = 1;
+  constexpr int BK = Shapes<T>::Big::BK;
+  const GemmPlan p = gemm_plan<T>(M, N, K, o);
+  g.bm = g.bn = p.tile;
+  g.tm = (M + p.tile - 1) / p.tile;
+  const long tn = (N + p.tile - 1) / p.tile;
+  g.pair = !o.lower_only && (o.tri == EXC_TRI_A_LOWER || o.tri == EXC_TRI_A_UPPER) ;
+  g.ntile = o.lower_only ? g.tm * (g.tm + 1) / 2 : (g.pair ? (g.tm + 1) / 2 : g.tm) * tn;
+  int splits = p.splits;
   if (splits > 1) {
     long chunk = (K + splits - 1) / splits;
     chunk = ((chunk + BK - 1) / BK) * BK;
@@ -412,16 +702,17 @@ int gemm_impl(int ta, int tb, long M, long N, long K, double alpha, const T* A, 
     g.kchunk = chunk;
     g.part = o.work;
   }
-  g.tm = tm;
-  g.ntile = tiles;
-  g.total = tiles * splits;
+  g.total = g.ntile * splits;
   EXC_REQUIRE(g.total < (1L << 31), EXC_ERR_ARG, "exc_gemm: too many tiles");
-  dim3 grid((unsigned)g.total);
   hipEvent_t e0 = exc_prof::mark(s);
-  if (!ta && !tb) hipLaunchKernelGGL((k_gemm<T, 0, 0>), grid, dim3(NT), 0, s, g);
-  else if (!ta && tb) hipLaunchKernelGGL((k_gemm<T, 0, 1>), grid, dim3(NT), 0, s, g);
-  else if (ta && !tb) hipLaunchKernelGGL((k_gemm<T, 1, 0>), grid, dim3(NT), 0, s, g);
-  else hipLaunchKernelGGL((k_gemm<T, 1, 1>), grid, dim3(NT), 0, s, g);
+  const bool tri = o.tri != EXC_TRI_NONE;
+  if (p.tile == 128) {
+    if (tri) gemm_launch<T, true, typename Shapes<T>::Big>(ta, tb, g, s);
+    else gemm_launch<T, false, typename Shapes<T>::Big>(ta, tb, g, s);
+  } else {
+    if (tri) gemm_launch<T, true, typename Shapes<T>::Small>(ta, tb, g, s);
+    else gemm_launch<T, false, typename Shapes<T>::Small>(ta, tb, g, s);
+  }
   EXC_CHECK_HIP(hipGetLastError());
   if (e0) {
     // useful flops: a triangular operand halves the products, a symmetric (lower-only) result too
@@ -452,6 +743,8 @@ struct GroupPlan {
 };
 
 GroupPlan group_plan(int nprob, const ExcGemmProblem* P, long kchunk) {
+  constexpr int BM = kGroupBM, BN = kGroupBN, BK = Shapes<double>::Big::BK;
+  static_assert(BK == Shapes<float>::Big::BK, "one chunk length for both types");
   GroupPlan g;
   if (kchunk > 0) kchunk = ((kchunk + BK - 1) / BK) * BK;
   for (int p = 0; p < nprob; p++) {
@@ -464,21 +757,22 @@ GroupPlan group_plan(int nprob, const ExcGemmProblem* P, long kchunk) {
     if (q.lower_only) f *= 0.5;
     g.flops += f;
     const long tm = (q.M + BM - 1) / BM, tn = (q.N + BN - 1) / BN;
+    // chunks of about kchunk, of equal length within a problem
     const long splits = (kchunk > 0 && q.K > kchunk) ? (q.K + kchunk - 1) / kchunk : 1;
+    const long chunk = splits == 1 ? q.K : ((q.K + splits - 1) / splits + BK - 1) / BK * BK;
+    const bool pair = splits == 1 && !q.lower_only && (q.tri == EXC_TRI_A_LOWER || q.tri == EXC_TRI_A_UPPER);
     for (long b = 0; b < tn; b++)
-      for (long a = 0; a < tm; a++) {
+      for (long a = 0; a < (pair ? (tm + 1) / 2 : tm); a++) {
         if (q.lower_only && a < b) continue;
         if (splits == 1 && !q.mirror) {
-          g.items.push_back(GroupItem{p, (int)a, (int)b, -1, 0, q.K});
+          const long other = pair && 2 * a < tm - 1 ? tm - 1 - a : -1;
+          g.items.push_back(GroupItem{p, (int)a, (int)b, -1, (int)other, 0, 0, q.K});
           continue;
         }
         const long first = g.slots;
-        for (long sp = 0; sp < splits; sp++) {
-          const long k0 = splits == 1 ? 0 : sp * kchunk;
-          const long k1 = splits == 1 ? q.K : std::min(q.K, (sp + 1) * kchunk);
-          g.items.push_back(GroupItem{p, (int)a, (int)b, (int)(g.slots++), k0, k1});
-        }
-        g.reds.push_back(GroupRed{p, (int)a, (int)b, (int)first, (int)splits, 0});
+        for (long k0 = 0; k0 < q.K || k0 == 0; k0 += chunk)
+          g.items.push_back(GroupItem{p, (int)a, (int)b, (int)(g.slots++), -1, 0, k0, std::min(q.K, k0 + chunk)});
+        g.reds.push_back(GroupRed{p, (int)a, (int)b, (int)first, (int)(g.slots - first), 0});
       }
   }
   return g;
@@ -487,11 +781,11 @@ GroupPlan group_plan(int nprob, const ExcGemmProblem* P, long kchunk) {
 size_t group_bytes(const GroupPlan& g, size_t tsize) {
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   return up(g.probs.size() * sizeof(GroupProb)) + up(g.items.size() * sizeof(GroupItem)) +
-         up(std::max<size_t>(1, g.reds.size()) * sizeof(GroupRed)) + (size_t)g.slots * BM * BN * tsize;
+         up(std::max<size_t>(1, g.reds.size()) * sizeof(GroupRed)) + (size_t)g.slots * kGroupBM * kGroupBN * tsize;
 }
 
 template <typename T>
-int group_run(int ta, int tb, const GroupPlan& g, double alpha, double beta, int grid, void* work, size_t wb,
+int group_run(int ta, int tb, const GroupPlan& g, double alpha, double beta, void* work, size_t wb,
               hipStream_t s) {
   EXC_REQUIRE(group_bytes(g, sizeof(T)) <= wb, EXC_ERR_SPACE, "exc_gemm_grouped: workspace too small");
   if (g.items.empty()) return EXC_OK;
@@ -511,13 +805,16 @@ int group_run(int ta, int tb, const GroupPlan& g, double alpha, double beta, int
     EXC_CHECK_HIP(hipMemcpyAsync(dr, g.reds.data(), g.reds.size() * sizeof(GroupRed), hipMemcpyHostToDevice, s));
   EXC_CHECK_HIP(hipStreamSynchronize(s));
   const long nitems = (long)g.items.size();
-  if (grid <= 0) grid = (int)std::min<long>(nitems, resident_slots(sizeof(T) == 8 ? 2 : 3));
-  grid = (int)std::min<long>(grid, nitems);
+  EXC_REQUIRE(nitems < (1L << 31), EXC_ERR_ARG, "exc_gemm_grouped: too many tiles");
+  const dim3 grid((unsigned)nitems), block(GroupShape<T>::kThreads);
   hipEvent_t e0 = exc_prof::mark(s);
-  if (!ta && !tb) hipLaunchKernelGGL((k_gemm_grouped<T, 0, 0>), dim3(grid), dim3(NT), 0, s, dp, di, nitems, part, alpha, beta);
-  else if (!ta && tb) hipLaunchKernelGGL((k_gemm_grouped<T, 0, 1>), dim3(grid), dim3(NT), 0, s, dp, di, nitems, part, alpha, beta);
-  else if (ta && !tb) hipLaunchKernelGGL((k_gemm_grouped<T, 1, 0>), dim3(grid), dim3(NT), 0, s, dp, di, nitems, part, alpha, beta);
-  else hipLaunchKernelGGL((k_gemm_grouped<T, 1, 1>), dim3(grid), dim3(NT), 0, s, dp, di, nitems, part, alpha, beta);
+  // one transposition pattern per call; a set with any triangular problem takes the kernel for both
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, dp, di, nitems, part, alpha, beta); };
+  const bool tri = std::any_of(g.probs.begin(), g.probs.end(), [](const GroupProb& p) { return p.tri != EXC_TRI_NONE; });
+  if (!ta && !tb) tri ? launch(k_gemm_grouped<T, 0, 0, true>) : launch(k_gemm_grouped<T, 0, 0, false>);
+  else if (!ta && tb) tri ? launch(k_gemm_grouped<T, 0, 1, true>) : launch(k_gemm_grouped<T, 0, 1, false>);
+  else if (ta && !tb) tri ? launch(k_gemm_grouped<T, 1, 0, true>) : launch(k_gemm_grouped<T, 1, 0, false>);
+  else tri ? launch(k_gemm_grouped<T, 1, 1, true>) : launch(k_gemm_grouped<T, 1, 1, false>);
   EXC_CHECK_HIP(hipGetLastError());
   if (!g.reds.empty()) {
     hipLaunchKernelGGL(k_grouped_reduce<T>, dim3((unsigned)g.reds.size()), dim3(256), 0, s, dp, dr, part, alpha,
@@ -528,7 +825,7 @@ int group_run(int ta, int tb, const GroupPlan& g, double alpha, double beta, int
   return EXC_OK;
 }
 
-// Tuning results per problem set: the K chunk and the persistent grid that ran fastest.
+// Tuning results per problem set: the K chunk that ran fastest and its number of workgroups.
 struct TuneEntry {
   long key[8];
   long kchunk;
@@ -539,10 +836,10 @@ std::vector<TuneEntry> g_tune;
 std::mutex g_tune_mu;
 
 template <typename T>
-int grouped_impl(int ta, int tb, int nprob, const ExcGemmProblem* P, double alpha, double beta, long kchunk, int grid,
+int grouped_impl(int ta, int tb, int nprob, const ExcGemmProblem* P, double alpha, double beta, long kchunk,
                  void* work, size_t wb, hipStream_t s) {
   EXC_REQUIRE(nprob >= 0 && (nprob == 0 || P), EXC_ERR_ARG, "exc_gemm_grouped: bad arguments");
-  if (kchunk >= 0) return group_run<T>(ta, tb, group_plan(nprob, P, kchunk), alpha, beta, grid, work, wb, s);
+  if (kchunk >= 0) return group_run<T>(ta, tb, group_plan(nprob, P, kchunk), alpha, beta, work, wb, s);
   // autotune: one timed run per candidate on the caller's data (each run overwrites the outputs
   // completely, so the last one leaves the result), the fastest kept per problem-set key
   long key[8] = {(long)sizeof(T), ta, tb, nprob, 0, 0, 0, 0};
@@ -556,12 +853,10 @@ int grouped_impl(int ta, int tb, int nprob, const ExcGemmProblem* P, double alph
     std::lock_guard<std::mutex> lock(g_tune_mu);
     for (const TuneEntry& e : g_tune)
       if (std::equal(e.key, e.key + 8, key))
-        return group_run<T>(ta, tb, group_plan(nprob, P, e.kchunk), alpha, beta, e.grid, work, wb, s);
+        return group_run<T>(ta, tb, group_plan(nprob, P, e.kchunk), alpha, beta, work, wb, s);
   }
   EXC_REQUIRE(beta == 0.0, EXC_ERR_ARG, "exc_gemm_grouped: tuning runs need beta = 0 (each run overwrites C)");
-  const long slots = resident_slots(sizeof(T) == 8 ? 2 : 3);
   const long chunks[] = {0, 16384, 8192, 4096, 2048};
-  const int mults[] = {1, 2};
   hipEvent_t a, b;
   EXC_CHECK_HIP(hipEventCreate(&a));
   EXC_CHECK_HIP(hipEventCreate(&b));
@@ -570,22 +865,19 @@ int grouped_impl(int ta, int tb, int nprob, const ExcGemmProblem* P, double alph
   for (long kc : chunks) {
     const GroupPlan g = group_plan(nprob, P, kc);
     if (group_bytes(g, sizeof(T)) > wb) continue;
-    for (int mu : mults) {
-      const int gr = (int)std::min<long>((long)g.items.size(), slots * mu);
-      int rc = group_run<T>(ta, tb, g, alpha, beta, gr, work, wb, s);  // warm (and tables uploaded)
-      if (rc) return rc;
-      EXC_CHECK_HIP(hipEventRecord(a, s));
-      rc = group_run<T>(ta, tb, g, alpha, beta, gr, work, wb, s);
-      if (rc) return rc;
-      EXC_CHECK_HIP(hipEventRecord(b, s));
-      EXC_CHECK_HIP(hipEventSynchronize(b));
-      float ms = 0.f;
-      EXC_CHECK_HIP(hipEventElapsedTime(&ms, a, b));
-      if (best.ms < 0 || ms < best.ms) {
-        best.ms = ms;
-        best.kchunk = kc;
-        best.grid = gr;
-      }
+    int rc = group_run<T>(ta, tb, g, alpha, beta, work, wb, s);  // warm (and tables uploaded)
+    if (rc) return rc;
+    EXC_CHECK_HIP(hipEventRecord(a, s));
+    rc = group_run<T>(ta, tb, g, alpha, beta, work, wb, s);
+    if (rc) return rc;
+    EXC_CHECK_HIP(hipEventRecord(b, s));
+    EXC_CHECK_HIP(hipEventSynchronize(b));
+    float ms = 0.f;
+    EXC_CHECK_HIP(hipEventElapsedTime(&ms, a, b));
+    if (best.ms < 0 || ms < best.ms) {
+      best.ms = ms;
+      best.kchunk = kc;
+      best.grid = (int)g.items.size();
     }
   }
   hipEventDestroy(a);
@@ -596,16 +888,16 @@ int grouped_impl(int ta, int tb, int nprob, const ExcGemmProblem* P, double alph
     std::lock_guard<std::mutex> lock(g_tune_mu);
     g_tune.push_back(best);
   }
-  return group_run<T>(ta, tb, group_plan(nprob, P, best.kchunk), alpha, beta, best.grid, work, wb, s);
+  return group_run<T>(ta, tb, group_plan(nprob, P, best.kchunk), alpha, beta, work, wb, s);
 }
 
 }  // namespace
 
 int exc_gemm_grouped_opts(int dtype, int ta, int tb, int nprob, const ExcGemmProblem* probs, double alpha, double beta,
-                          long kchunk, int grid, void* work, size_t work_bytes, hipStream_t s) {
+                          long kchunk, void* work, size_t work_bytes, hipStream_t s) {
   EXC_REQUIRE(dtype == 4 || dtype == 8, EXC_ERR_ARG, "exc_gemm_grouped: dtype is 4 (float) or 8 (double)");
-  if (dtype == 8) return grouped_impl<double>(ta, tb, nprob, probs, alpha, beta, kchunk, grid, work, work_bytes, s);
-  return grouped_impl<float>(ta, tb, nprob, probs, alpha, beta, kchunk, grid, work, work_bytes, s);
+  if (dtype == 8) return grouped_impl<double>(ta, tb, nprob, probs, alpha, beta, kchunk, work, work_bytes, s);
+  return grouped_impl<float>(ta, tb, nprob, probs, alpha, beta, kchunk, work, work_bytes, s);
 }
 
 size_t exc_gemm_grouped_workspace(int dtype, int nprob, const ExcGemmProblem* probs, long kchunk) {

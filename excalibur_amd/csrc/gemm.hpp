@@ -39,12 +39,11 @@ struct ExcGemmProblem {
   int beta_zero_hint = 0;
 };
 // Many independent products (all FP32 when dtype = 4, all FP64 when 8; one transposition pattern)
-// in one persistent launch plus one reduction launch. kchunk: split K into chunks of this length
-// (0: no split); kchunk < 0 lets the autotuner choose the chunk and the persistent grid size by
-// timing candidates on these problems once (beta must be 0), then reuse the choice for problem
-// sets of the same shape. grid <= 0: one workgroup per resident slot.
+// in one launch plus one reduction launch. kchunk: split K into chunks of about this length (0: no
+// split); kchunk < 0 lets the autotuner choose it by timing candidates on these problems once
+// (beta must be 0), then reuse the choice for problem sets of the same shape.
 int exc_gemm_grouped_opts(int dtype, int ta, int tb, int nprob, const ExcGemmProblem* probs, double alpha, double beta,
-                          long kchunk, int grid, void* work, size_t work_bytes, hipStream_t s);
+                          long kchunk, void* work, size_t work_bytes, hipStream_t s);
 size_t exc_gemm_grouped_workspace(int dtype, int nprob, const ExcGemmProblem* probs, long kchunk);
 // The autotuner's choices so far as a JSON list (extern "C", declared in excalibur_hip.h).
 extern "C" int exc_gemm_grouped_tuning(char* buf, size_t cap);

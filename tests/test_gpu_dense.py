@@ -123,3 +123,41 @@ def test_lu_sign(hip, n):
     assert set(np.unique(s)) <= {-1.0, 1.0}
     assert np.max(np.abs(L @ U - (Q - np.diag(s)))) <= 1e-12 * n
     assert np.all(np.abs(np.diag(U)) >= 1.0 - 1e-12), "pivots have magnitude >= 1"
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+def test_gemm_edges(hip, f32, ta, tb):
+    """Sizes around the tiles, the K steps and the 16-byte units, with and without a workspace, on
+    matrices inside larger arrays that start one element off and hold NaN around them. The bound is
+    the a-priori one of a K-term dot product in any order, |err| <= (K + 2) u |A||B|."""
+    dt, u = (np.float32, 2.0 ** -24) if f32 else (np.float64, 2.0 ** -53)
+    rng = np.random.default_rng(11)
+    for (M, N, K) in ((1, 1, 1), (1, 3, 2), (2, 1, 700), (3, 200, 1000), (64, 64, 16), (65, 129, 17), (130, 1, 300),
+                      (127, 255, 31), (128, 128, 64), (257, 66, 1030), (600, 1026, 5)):
+        banner(f"gemm {M}x{N}x{K} ta={ta} tb={tb} f32={f32}")
+        A, B = rng.standard_normal((M, K)).astype(dt), rng.standard_normal((K, N)).astype(dt)
+        C = rng.standard_normal((M, N)).astype(dt)
+
+        def inside(X, pad):
+            big = np.full(1 + X.shape[0] * (X.shape[1] + pad), np.nan, dt)
+            big[1:].reshape(X.shape[0], -1)[:, :X.shape[1]] = X
+            return hip.DeviceArray.from_host(big), X.shape[1] + pad
+
+        want = 0.5 * (A.astype(np.float64) @ B.astype(np.float64)) - 2.0 * C.astype(np.float64)
+        bound = (K + 4) * u * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64) + 2.0 * np.abs(C) + 1.0)
+        dA, lda = inside(A.T if ta else A, 3)
+        dB, ldb = inside(B.T if tb else B, 5)
+        for work in (False, True):
+            dC, ldc = inside(C, 1)
+            ws = hip.workspace(hip.lib.exc_gemm_workspace(M, N, K))
+            s = np.dtype(dt).itemsize
+            hip.call("exc_sgemm" if f32 else "exc_dgemm", int(ta), int(tb), M, N, K, 0.5, dA.ptr + s, lda, dB.ptr + s,
+                     ldb, -2.0, dC.ptr + s, ldc, ws.ptr if work else None, ws.nbytes if work else 0, None)
+            hip.sync()
+            got = dC.to_host()
+            assert np.isnan(got[0])
+            got = got[1:].reshape(M, ldc)
+            assert np.isnan(got[:, N:]).all()
+            assert (np.abs(got[:, :N] - want) <= bound).all(), (M, N, K, work)
