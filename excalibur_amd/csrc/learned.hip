@@ -232,53 +232,167 @@ constexpr int kIn = 32, kHid = 256, kOut = 2;
 constexpr long kW1 = 0, kB1 = kW1 + (long)kIn * kHid, kW2 = kB1 + kHid, kB2 = kW2 + (long)kHid * kHid,
                kW3 = kB2 + kHid, kB3 = kW3 + (long)kHid * kOut, kParams = kB3 + kOut;
 
-__global__ __launch_bounds__(256) void k_bias_relu(long B, int N, float* __restrict__ Z, const float* __restrict__ bias,
+// Caller's float arrays are read 4 at a time with no more than their elements' alignment.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// H = relu(Z + bias) over the B x 256 layer, four columns per thread.
+__global__ __launch_bounds__(256) void k_bias_relu(long B, const float* __restrict__ Z, const float* __restrict__ bias,
                                                    float* __restrict__ H) {
   const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= B * N) return;
-  const float z = Z[g] + bias[g % N];
-  Z[g] = z;
-  H[g] = z > 0.f ? z : 0.f;
-}
-
-__global__ __launch_bounds__(256) void k_bias(long B, int N, float* __restrict__ Z, const float* __restrict__ bias) {
-  const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= B * N) return;
-  Z[g] = Z[g] + bias[g % N];
-}
-
-// Laplace negative log-likelihood |y - c| exp(-w) + w, averaged over B; dO its gradient.
-__global__ __launch_bounds__(256) void k_head_loss(long B, const float* __restrict__ O, const float* __restrict__ y,
-                                                   float* __restrict__ dO, float* __restrict__ loss) {
-  __shared__ float red[4];
-  const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  float l = 0.f;
-  if (g < B) {
-    const float c = O[2 * g], w = O[2 * g + 1];
-    const float r = y[g] - c;
-    const float ew = expf(-w);
-    l = fabsf(r) * ew + w;
-    dO[2 * g] = (r > 0.f ? -ew : (r < 0.f ? ew : 0.f)) / (float)B;
-    dO[2 * g + 1] = (1.f - fabsf(r) * ew) / (float)B;
+  if (g >= B * (kHid / 4)) return;
+  const int j = (int)(g % (kHid / 4)) * 4;
+  const f4u z = *(const f4u*)(Z + 4 * g);
+  f4u h;
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const float v = z[q] + bias[j + q];
+    h[q] = v > 0.f ? v : 0.f;
   }
-  l = wave_sum(l);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = l;
-  __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(loss, (red[0] + red[1] + red[2] + red[3]) / (float)B);
+  *(f4u*)(H + 4 * g) = h;
 }
 
-__global__ __launch_bounds__(256) void k_relu_back(long n, float* __restrict__ dH, const float* __restrict__ Z) {
-  const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g < n && !(Z[g] > 0.f)) dH[g] = 0.f;
+// The second hidden layer's bias and ReLU and the output layer in one pass: a wavefront per row,
+// four columns per lane. (As a matrix product the two output columns fill 1/64 of a tile.)
+constexpr int kHeadRows = 4;  // rows per wavefront
+__global__ __launch_bounds__(256) void k_bias_relu_head(long B, const float* __restrict__ Z,
+                                                        const float* __restrict__ p, float* __restrict__ H,
+                                                        float* __restrict__ O) {
+  const int lane = threadIdx.x & 63, j = 4 * lane;
+  const long r0 = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * kHeadRows;
+  float w0[4], w1[4], b2[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    w0[q] = p[kW3 + (j + q) * kOut];
+    w1[q] = p[kW3 + (j + q) * kOut + 1];
+    b2[q] = p[kB2 + j + q];
+  }
+  for (long r = r0; r < min(B, r0 + kHeadRows); r++) {
+    const f4u z = *(const f4u*)(Z + r * kHid + j);
+    f4u h;
+    float o0 = 0.f, o1 = 0.f;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const float v = z[q] + b2[q];
+      h[q] = v > 0.f ? v : 0.f;
+      o0 += h[q] * w0[q];
+      o1 += h[q] * w1[q];
+    }
+    *(f4u*)(H + r * kHid + j) = h;
+    o0 = wave_sum(o0);
+    o1 = wave_sum(o1);
+    if (lane == 0) {
+      O[2 * r] = o0 + p[kB3];
+      O[2 * r + 1] = o1 + p[kB3 + 1];
+    }
+  }
 }
 
-// out[j] = sum over the B rows of X[:, j] (fixed order: one thread per column).
-__global__ __launch_bounds__(256) void k_colsum(long B, int N, const float* __restrict__ X, float* __restrict__ out) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= N) return;
+// Head of the backward pass over a slab of rows, one column per thread: the Laplace negative
+// log-likelihood |y - c| exp(-w) + w averaged over B and its gradient dO, the gradient of the second
+// layer's sums dZ2 = (dO W3^T) where H2 > 0, and this slab's share of dW3 = H2^T dO, db2, db3 and
+// the loss. `part` holds one row of kHeadPart values per workgroup, summed by k_sum_parts in a
+// fixed order.
+constexpr int kPartW3 = 0, kPartB2 = kPartW3 + kHid * kOut, kPartB3 = kPartB2 + kHid, kPartLoss = kPartB3 + kOut,
+              kHeadPart = kPartLoss + 1;
+constexpr int kSlab = 16;  // rows whose dO a workgroup holds at a time
+__global__ __launch_bounds__(256) void k_head_back(long B, long rows, const float* __restrict__ O,
+                                                   const float* __restrict__ y, const float* __restrict__ H,
+                                                   const float* __restrict__ p, float* __restrict__ dZ,
+                                                   float* __restrict__ part, float* __restrict__ grad,
+                                                   float* __restrict__ loss) {
+  __shared__ float d0[kSlab], d1[kSlab], ls[kSlab];
+  const int j = threadIdx.x;
+  const float w0 = p[kW3 + j * kOut], w1 = p[kW3 + j * kOut + 1];
+  float g0 = 0.f, g1 = 0.f, gb = 0.f, s0 = 0.f, s1 = 0.f, sl = 0.f;
+  const long end = min(B, (blockIdx.x + 1L) * rows);
+  for (long r0 = blockIdx.x * rows; r0 < end; r0 += kSlab) {
+    const int n = (int)min((long)kSlab, end - r0);
+    float h[kSlab];
+#pragma unroll
+    for (int q = 0; q < kSlab; q++) h[q] = H[(r0 + min(q, n - 1)) * kHid + j];
+    if (j < n) {
+      const long r = r0 + j;
+      const float c = O[2 * r], w = O[2 * r + 1], e = y[r] - c, ew = expf(-w);
+      ls[j] = fabsf(e) * ew + w;
+      d0[j] = (e > 0.f ? -ew : (e < 0.f ? ew : 0.f)) / (float)B;
+      d1[j] = (1.f - fabsf(e) * ew) / (float)B;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kSlab; q++)
+      if (q < n) {
+        const float a = d0[q], b = d1[q];
+        const float dz = h[q] > 0.f ? a * w0 + b * w1 : 0.f;
+        dZ[(r0 + q) * kHid + j] = dz;
+        g0 += h[q] * a;
+        g1 += h[q] * b;
+        gb += dz;
+        s0 += a;
+        s1 += b;
+        sl += ls[q];
+      }
+    __syncthreads();
+  }
+  if (gridDim.x == 1) {  // the slab is the batch
+    grad[kW3 + j * kOut] = g0;
+    grad[kW3 + j * kOut + 1] = g1;
+    grad[kB2 + j] = gb;
+    if (j == 0) {
+      grad[kB3] = s0;
+      grad[kB3 + 1] = s1;
+      *loss = sl / (float)B;
+    }
+    return;
+  }
+  float* o = part + (long)blockIdx.x * kHeadPart;
+  o[kPartW3 + j * kOut] = g0;
+  o[kPartW3 + j * kOut + 1] = g1;
+  o[kPartB2 + j] = gb;
+  if (j == 0) {
+    o[kPartB3] = s0;
+    o[kPartB3 + 1] = s1;
+    o[kPartLoss] = sl / (float)B;
+  }
+}
+
+// dZ1 = dH1 where H1 > 0 (in place) over a slab of rows, with the slab's column sums.
+__global__ __launch_bounds__(256) void k_relu_back(long B, long rows, float* __restrict__ dH,
+                                                   const float* __restrict__ H, float* __restrict__ part) {
+  const int j = threadIdx.x;
+  const long end = min(B, (blockIdx.x + 1L) * rows);
   float s = 0.f;
-  for (long r = 0; r < B; r++) s += X[r * N + j];
-  out[j] = s;
+#pragma unroll 8
+  for (long r = blockIdx.x * rows; r < end; r++) {
+    const long e = r * kHid + j;
+    const float v = H[e] > 0.f ? dH[e] : 0.f;
+    dH[e] = v;
+    s += v;
+  }
+  part[(long)blockIdx.x * kHid + j] = s;
+}
+
+// Column sums of the n x cols partials: 16 columns per workgroup, 16 threads per column.
+// Head partials (loss given) go to the gradient's slots and the loss, others to out.
+__global__ __launch_bounds__(256) void k_sum_parts(int n, int cols, const float* __restrict__ part,
+                                                   float* __restrict__ out, float* __restrict__ grad,
+                                                   float* __restrict__ loss) {
+  __shared__ float red[16][17];
+  const int c = threadIdx.x & 15, q = threadIdx.x >> 4, col = blockIdx.x * 16 + c;
+  float s = 0.f;
+  if (col < cols)
+#pragma unroll 8
+    for (int i = q; i < n; i += 16) s += part[(long)i * cols + col];
+  red[q][c] = s;
+  __syncthreads();
+  if (q != 0 || col >= cols) return;
+  s = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; i++) s += red[i][c];
+  if (!loss) out[col] = s;
+  else if (col < kPartB2) grad[kW3 + col] = s;
+  else if (col < kPartB3) grad[kB2 + col - kPartB2] = s;
+  else if (col < kPartLoss) grad[kB3 + col - kPartB3] = s;
+  else *loss = s;
 }
 
 __global__ __launch_bounds__(256) void k_adam(long n, float* __restrict__ p, const float* __restrict__ g,
@@ -299,52 +413,121 @@ __global__ __launch_bounds__(256) void k_to_bf16(long n, const float* __restrict
   if (i < n) y[i] = __float2bfloat16(x[i]);
 }
 
-// BF16 inference: weights and activations held in bfloat16, products accumulated in FP32. One
-// sample per thread; the first hidden layer passes through LDS transposed (feature-major), so the
-// 64 lanes of a wavefront read consecutive words, and the weights are read uniformly by all lanes.
-__global__ __launch_bounds__(128) void k_mlp_infer_bf16(long B, const float* __restrict__ X,
-                                                        const __hip_bfloat16* __restrict__ P, float* __restrict__ O) {
-  __shared__ __hip_bfloat16 h[kHid][128];
-  const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool live = s < B;
-  const int me = threadIdx.x;
-  float x[kIn];
+// BF16 inference: weights and activations in bfloat16, products accumulated in FP32 on
+// v_mfma_f32_16x16x32_bf16. A workgroup runs 32 samples through both hidden layers; wavefront w owns
+// the units 64 w .. 64 w + 63. An MFMA lane wants 8 consecutive k of one unit, but the weights are
+// stored unit-fastest, so each wavefront transposes its 64 x 256 slice of W2 into LDS (8 x 8 blocks
+// in registers, 16-byte units XORed by the row against bank conflicts). 4096 samples: 797 us with
+// one sample per thread and scalar products, 11 us here.
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b8u __attribute__((ext_vector_type(8), aligned(2)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+constexpr int kInferRows = 32;
+constexpr int kUnits = kHid / 8;  // 16-byte units of a row of 256
+__global__ __launch_bounds__(256) void k_mlp_infer_bf16(long B, const float* __restrict__ X,
+                                                        const __bf16* __restrict__ P, float* __restrict__ O) {
+  __shared__ b8 w2[kHid * kUnits];       // [unit][k], 128 KB
+  __shared__ b8 h[kInferRows * kUnits];  // [sample][k] of the first layer, 16 KB
+  __shared__ float red[4][kInferRows][2];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const long s0 = (long)blockIdx.x * kInferRows;
+  const int u0 = 64 * wave;
+  // this wavefront's slice of W2: 8 unit groups x 32 k groups of 8 x 8 blocks, four per lane
 #pragma unroll
-  for (int k = 0; k < kIn; k++) x[k] = live ? __bfloat162float(__float2bfloat16(X[s * kIn + k])) : 0.f;
-  // layer 1
-  for (int j0 = 0; j0 < kHid; j0 += 32) {
-    float acc[32];
+  for (int z = 0; z < 4; z++) {
+    const int blk = lane + 64 * z, ug = blk & 7, kg = blk >> 3;
+    b8 in[8];
 #pragma unroll
-    for (int q = 0; q < 32; q++) acc[q] = __bfloat162float(P[kB1 + j0 + q]);
+    for (int k = 0; k < 8; k++) in[k] = *(const b8u*)(P + kW2 + (long)(kg * 8 + k) * kHid + u0 + ug * 8);
 #pragma unroll
-    for (int k = 0; k < kIn; k++)
+    for (int c = 0; c < 8; c++) {
+      b8 o;
 #pragma unroll
-      for (int q = 0; q < 32; q++) acc[q] += x[k] * __bfloat162float(P[kW1 + (long)k * kHid + j0 + q]);
+      for (int k = 0; k < 8; k++) o[k] = in[k][c];
+      const int r = u0 + ug * 8 + c;
+      w2[r * kUnits + (kg ^ (r & 15))] = o;
+    }
+  }
+  // layer 1: K = 32 is one step; samples are the rows of A, units the columns of B
+  b8 xa[2];
 #pragma unroll
-    for (int q = 0; q < 32; q++) h[j0 + q][me] = __float2bfloat16(acc[q] > 0.f ? acc[q] : 0.f);
+  for (int a = 0; a < 2; a++) {
+    const long s = min(s0 + a * 16 + li, B - 1);
+#pragma unroll
+    for (int k = 0; k < 8; k++) xa[a][k] = (__bf16)X[s * kIn + lk * 8 + k];
+  }
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    const int u = u0 + b * 16 + li;
+    b8 wb;
+#pragma unroll
+    for (int k = 0; k < 8; k++) wb[k] = P[kW1 + (long)(lk * 8 + k) * kHid + u];
+    const float bias = (float)P[kB1 + u];
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+      const f4 v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[a], wb, f4{bias, bias, bias, bias}, 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int s = a * 16 + 4 * lk + q;
+        ((__bf16*)h)[(s * kUnits + ((u >> 3) ^ (s & 15))) * 8 + (u & 7)] = (__bf16)(v[q] > 0.f ? v[q] : 0.f);
+      }
+    }
   }
   __syncthreads();
-  // layer 2 by chunks of 32 outputs, each chunk folded into the output layer at once
-  float o0 = __bfloat162float(P[kB3]), o1 = __bfloat162float(P[kB3 + 1]);
-  for (int j0 = 0; j0 < kHid; j0 += 32) {
-    float acc[32];
+  // layer 2
+  f4 acc[2][4];
 #pragma unroll
-    for (int q = 0; q < 32; q++) acc[q] = __bfloat162float(P[kB2 + j0 + q]);
-    for (int k = 0; k < kHid; k++) {
-      const float hk = __bfloat162float(h[k][me]);
-#pragma unroll
-      for (int q = 0; q < 32; q++) acc[q] += hk * __bfloat162float(P[kW2 + (long)k * kHid + j0 + q]);
-    }
-#pragma unroll
-    for (int q = 0; q < 32; q++) {
-      const float hq = __bfloat162float(__float2bfloat16(acc[q] > 0.f ? acc[q] : 0.f));
-      o0 += hq * __bfloat162float(P[kW3 + (long)(j0 + q) * kOut]);
-      o1 += hq * __bfloat162float(P[kW3 + (long)(j0 + q) * kOut + 1]);
-    }
+  for (int b = 0; b < 4; b++) {
+    const float bias = (float)P[kB2 + u0 + b * 16 + li];
+    acc[0][b] = acc[1][b] = f4{bias, bias, bias, bias};
   }
-  if (live) {
-    O[2 * s] = o0;
-    O[2 * s + 1] = o1;
+#pragma unroll
+  for (int ks = 0; ks < kHid / 32; ks++) {
+    const int ku = ks * 4 + lk;
+    b8 ha[2], wb[4];
+#pragma unroll
+    for (int a = 0; a < 2; a++) ha[a] = h[(a * 16 + li) * kUnits + (ku ^ li)];
+#pragma unroll
+    for (int b = 0; b < 4; b++) wb[b] = w2[(u0 + b * 16 + li) * kUnits + (ku ^ li)];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int b = 0; b < 4; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ha[a], wb[b], acc[a][b], 0, 0, 0);
+  }
+  // output layer: each lane's four units, then the 16 lanes of a row group, then the wavefronts
+  float w30[4], w31[4];
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    w30[b] = (float)P[kW3 + (u0 + b * 16 + li) * kOut];
+    w31[b] = (float)P[kW3 + (u0 + b * 16 + li) * kOut + 1];
+  }
+#pragma unroll
+  for (int a = 0; a < 2; a++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      float o0 = 0.f, o1 = 0.f;
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        const float v = acc[a][b][q];
+        const float hq = (float)(__bf16)(v > 0.f ? v : 0.f);
+        o0 += hq * w30[b];
+        o1 += hq * w31[b];
+      }
+#pragma unroll
+      for (int off = 8; off > 0; off >>= 1) {
+        o0 += __shfl_xor(o0, off, kWave);
+        o1 += __shfl_xor(o1, off, kWave);
+      }
+      if (li == 0) {
+        red[wave][a * 16 + 4 * lk + q][0] = o0;
+        red[wave][a * 16 + 4 * lk + q][1] = o1;
+      }
+    }
+  __syncthreads();
+  if (tid < 2 * kInferRows) {
+    const int s = tid >> 1, c = tid & 1;
+    if (s0 + s < B)
+      O[2 * (s0 + s) + c] = (float)P[kB3 + c] + (red[0][s][c] + red[1][s][c]) + (red[2][s][c] + red[3][s][c]);
   }
 }
 
@@ -429,13 +612,10 @@ int exc_mlp_forward(long B, const float* d_x, const float* d_p, float* d_acts, f
   o.work_bytes = work_bytes;
   int rc = exc_sgemm_opts(0, 0, B, kHid, kIn, 1.0, d_x, kIn, d_p + kW1, kHid, 0.0, Z1, kHid, o, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_bias_relu, dim3(grid_for(B * kHid)), dim3(256), 0, s, B, kHid, Z1, d_p + kB1, H1);
+  hipLaunchKernelGGL(k_bias_relu, dim3(grid_for(B * (kHid / 4))), dim3(256), 0, s, B, Z1, d_p + kB1, H1);
   rc = exc_sgemm_opts(0, 0, B, kHid, kHid, 1.0, H1, kHid, d_p + kW2, kHid, 0.0, Z2, kHid, o, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_bias_relu, dim3(grid_for(B * kHid)), dim3(256), 0, s, B, kHid, Z2, d_p + kB2, H2);
-  rc = exc_sgemm_opts(0, 0, B, kOut, kHid, 1.0, H2, kHid, d_p + kW3, kOut, 0.0, d_out, kOut, o, s);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_bias, dim3(grid_for(B * kOut)), dim3(256), 0, s, B, kOut, d_out, d_p + kB3);
+  hipLaunchKernelGGL(k_bias_relu_head, dim3(grid_for(B, 4 * kHeadRows)), dim3(256), 0, s, B, Z2, d_p, H2, d_out);
   EXC_CHECK_HIP(hipGetLastError());
   return EXC_OK;
 }
@@ -454,31 +634,30 @@ int exc_mlp_backward(long B, const float* d_x, const float* d_y, const float* d_
   float* H1 = Z1 + B * kHid;
   float* Z2 = H1 + B * kHid;
   float* H2 = Z2 + B * kHid;
-  float* dO = d_scratch;
-  float* dH = dO + B * kOut;
+  // The gradient of a layer's sums: dZ2 in the scratch, dZ1 in Z1's slot (H says where Z was
+  // positive). The slabs' partial sums go to Z2's slot (two slabs are over 16 rows, enough for them).
+  float* dZ2 = d_scratch;
+  float* part = Z2;
+  const long rows = std::max<long>(kSlab, (B + 511) / 512);  // of a slab, at most 512 slabs
+  const unsigned slabs = grid_for(B, (int)rows);
   ExcGemmOpts o;
   o.work = d_work;
   o.work_bytes = work_bytes;
-  EXC_CHECK_HIP(hipMemsetAsync(d_loss, 0, sizeof(float), s));
-  hipLaunchKernelGGL(k_head_loss, dim3(grid_for(B)), dim3(256), 0, s, B, d_out, d_y, dO, d_loss);
-  // layer 3: dW3 = H2^T dO, db3 = colsum dO, dH2 = dO W3^T
-  int rc = exc_sgemm_opts(1, 0, kHid, kOut, B, 1.0, H2, kHid, dO, kOut, 0.0, d_grad + kW3, kOut, o, s);
+  hipLaunchKernelGGL(k_head_back, dim3(slabs), dim3(256), 0, s, B, rows, d_out, d_y, H2, d_p, dZ2, part, d_grad,
+                     d_loss);
+  if (slabs > 1) hipLaunchKernelGGL(k_sum_parts, dim3(grid_for(kHeadPart, 16)), dim3(256), 0, s, (int)slabs, kHeadPart, part,
+                     (float*)nullptr, d_grad, d_loss);
+  // layer 2: dW2 = H1^T dZ2, dH1 = dZ2 W2^T
+  int rc = exc_sgemm_opts(1, 0, kHid, kHid, B, 1.0, H1, kHid, dZ2, kHid, 0.0, d_grad + kW2, kHid, o, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_colsum, dim3(1), dim3(256), 0, s, B, kOut, dO, d_grad + kB3);
-  rc = exc_sgemm_opts(0, 1, B, kHid, kOut, 1.0, dO, kOut, d_p + kW3, kOut, 0.0, dH, kHid, o, s);
+  rc = exc_sgemm_opts(0, 1, B, kHid, kHid, 1.0, dZ2, kHid, d_p + kW2, kHid, 0.0, Z1, kHid, o, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_relu_back, dim3(grid_for(B * kHid)), dim3(256), 0, s, B * kHid, dH, Z2);
-  // layer 2: dW2 = H1^T dZ2, db2, dH1 = dZ2 W2^T (into H1's slot: H1 is not needed afterwards)
-  rc = exc_sgemm_opts(1, 0, kHid, kHid, B, 1.0, H1, kHid, dH, kHid, 0.0, d_grad + kW2, kHid, o, s);
+  hipLaunchKernelGGL(k_relu_back, dim3(slabs), dim3(256), 0, s, B, rows, Z1, H1, slabs > 1 ? part : d_grad + kB1);
+  if (slabs > 1) hipLaunchKernelGGL(k_sum_parts, dim3(grid_for(kHid, 16)), dim3(256), 0, s, (int)slabs, kHid, part, d_grad + kB1,
+                     (float*)nullptr, (float*)nullptr);
+  // layer 1: dW1 = X^T dZ1
+  rc = exc_sgemm_opts(1, 0, kIn, kHid, B, 1.0, d_x, kIn, Z1, kHid, 0.0, d_grad + kW1, kHid, o, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_colsum, dim3(1), dim3(256), 0, s, B, kHid, dH, d_grad + kB2);
-  rc = exc_sgemm_opts(0, 1, B, kHid, kHid, 1.0, dH, kHid, d_p + kW2, kHid, 0.0, H1, kHid, o, s);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_relu_back, dim3(grid_for(B * kHid)), dim3(256), 0, s, B * kHid, H1, Z1);
-  // layer 1: dW1 = X^T dZ1, db1
-  rc = exc_sgemm_opts(1, 0, kIn, kHid, B, 1.0, d_x, kIn, H1, kHid, 0.0, d_grad + kW1, kHid, o, s);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_colsum, dim3(1), dim3(256), 0, s, B, kHid, H1, d_grad + kB1);
   EXC_CHECK_HIP(hipGetLastError());
   return EXC_OK;
 }
@@ -503,8 +682,8 @@ int exc_mlp_to_bf16(const float* d_p, void* d_pbf16, exc_stream_t stream) {
 
 int exc_mlp_infer_bf16(long B, const float* d_x, const void* d_pbf16, float* d_out, exc_stream_t stream) {
   EXC_REQUIRE(B >= 1 && d_x && d_pbf16 && d_out, EXC_ERR_ARG, "exc_mlp_infer_bf16: bad arguments");
-  hipLaunchKernelGGL(k_mlp_infer_bf16, dim3(grid_for(B, 128)), dim3(128), 0, exc_detail::stream(stream), B, d_x,
-                     (const __hip_bfloat16*)d_pbf16, d_out);
+  hipLaunchKernelGGL(k_mlp_infer_bf16, dim3(grid_for(B, kInferRows)), dim3(256), 0, exc_detail::stream(stream), B, d_x,
+                     (const __bf16*)d_pbf16, d_out);
   EXC_CHECK_HIP(hipGetLastError());
   return EXC_OK;
 }

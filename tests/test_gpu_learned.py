@@ -54,6 +54,31 @@ def test_bf16_inference_matches_fp64_forward(L):
     assert np.max(np.abs(got - want)) <= 3e-2 * scale
 
 
+@pytest.mark.parametrize("B", [1, 15, 17, 33, 64, 8209])
+def test_network_batch_edges(L, B):
+    """Batches around the rows a workgroup takes (16 in the backward pass, 32 in inference; 8,209
+    needs longer slabs): the gradient per block and the inference, to the bounds used above."""
+    from oracle import mlp
+    banner(f"batch {B}")
+    rng = np.random.default_rng(B)
+    p = mlp.init(rng)
+    X = rng.uniform(0, 1, (B, mlp.D_IN)).astype(np.float32)
+    y = rng.uniform(-1.5, 0, B).astype(np.float32)
+    net = L.BracketNet()
+    net.set_params(p.astype(np.float32))
+    loss, g = net.grad(X, y)
+    p64 = p.astype(np.float32).astype(np.float64)
+    lo, go = mlp.grad(p64, X.astype(np.float64), y.astype(np.float64))
+    assert abs(loss - lo) <= 1e-4 * max(abs(lo), 1.0)
+    o = 0
+    for name, shape in mlp.SHAPES:
+        k = int(np.prod(shape))
+        assert np.linalg.norm(g[o:o + k] - go[o:o + k]) <= 5e-3 * max(np.linalg.norm(go[o:o + k]), 1e-6), name
+        o += k
+    want, _ = mlp.forward(p64, X.astype(np.float64))
+    assert np.max(np.abs(net.infer(X) - want)) <= 3e-2 * np.abs(want).max()
+
+
 def gk_restated(sig, start, steps):
     """The first steps of Golub-Kahan on diag(sig) in numpy (alpha_j u_j = D v_j - beta_{j-1}
     u_{j-1}, beta_j v_{j+1} = D u_j - alpha_j v_j)."""
