@@ -577,6 +577,7 @@ __global__ __launch_bounds__(256) void k_grouped_reduce(const GroupProb* __restr
     if (gi >= pr.M || gj >= pr.N) continue;
     if (pr.lower_only && gj > gi) continue;  // the upper part of a diagonal tile comes by mirroring
     T s = T(0);
+#pragma unroll 4
     for (int q = 0; q < r.nslots; q++) s += part[(size_t)(r.first_slot + q) * kGroupBM * kGroupBN + e];
     T out = (T)alpha * s;
     if (beta != 0.0) out += (T)beta * C[gi * pr.ldc + gj];
@@ -595,6 +596,7 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs g, int splits) {
   if (g.lower_only && (j / g.bn) > (i / g.bm)) return;
   const T* P = (const T*)g.part;
   T s = T(0);
+#pragma unroll 8
   for (int z = 0; z < splits; z++) s += P[(size_t)z * total + idx];
   T* C = (T*)g.C;
   T out = (T)g.alpha * s;
