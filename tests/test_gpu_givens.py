@@ -79,3 +79,19 @@ def test_virtual_matrix_mask_bit_exact(hip, oracle, m, n, is_left):
     back = hip.block_shift_mask(got, 32, False, is_left, 4242)
     assert np.array_equal(back, oracle.block_shift_mask(want, 32, False, is_left, 4242))
     assert np.max(np.abs(back - x)) <= 1e-12
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("is_left", [True, False])
+@pytest.mark.parametrize("K,lines", [(2, 1), (127, 771), (128, 385), (130, 1540), (1025, 3), (1026, 387), (2048, 5),
+                                     (2051, 2), (4096, 3), (4099, 2), (9001, 2)])
+def test_givens_shape_edges(hip, K, lines, is_left, f32):
+    """Line counts around the strips of 1, 2, 4 and 8 lines and pair counts around the threads of one
+    wavefront, one pair per thread, two, and more than the registers hold; bit for bit."""
+    banner(f"givens K={K} lines={lines} left={is_left} f32={f32}")
+    dt = np.float32 if f32 else np.float64
+    x = np.random.default_rng(K + lines).standard_normal((K, lines) if is_left else (lines, K)).astype(dt)
+    for mask in (True, False):
+        pairs, cs = hip.givens_plan(K, 3, mask, 17)
+        got = hip.givens_apply(x, pairs, cs, mask, is_left, f32=f32)
+        assert np.array_equal(got, givens_numpy(x, pairs, cs, mask, is_left, dt)), mask
