@@ -8,6 +8,7 @@
 #include "exc_common.hpp"
 #include "sturm.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 #pragma clang fp contract(off)
@@ -33,28 +34,29 @@ __global__ __launch_bounds__(256) void k_sturm_count(int n, const double* __rest
 
 // ||alpha||^2 + ||beta||^2 with the sequential sum of squares of the reference's nrm2 restated
 // (sqrt, then squared, as bbtsvd.cpp:936 writes pow(dnrm2(.), 2)). One workgroup stages chunks
-// in LDS; thread 0 accumulates in index order.
+// in LDS; one thread per vector accumulates in index order, both at the same time.
 __global__ __launch_bounds__(256) void k_frob_bound(int n, const double* __restrict__ a,
                                                     const double* __restrict__ b, BisectHdr* hdr) {
-  __shared__ double buf[2048];
-  double sums[2] = {0.0, 0.0};
-  for (int which = 0; which < 2; which++) {
-    const double* x = which == 0 ? a : b;
-    const int len = which == 0 ? n : n - 1;
-    double s = 0.0;
-    for (int base = 0; base < len; base += 2048) {
-      const int cnt = min(2048, len - base);
-      for (int i = threadIdx.x; i < cnt; i += blockDim.x) buf[i] = x[base + i];
-      __syncthreads();
-      if (threadIdx.x == 0)
-        for (int i = 0; i < cnt; i++) {
-          const double v = buf[i];
-          s = s + v * v;
-        }
-      __syncthreads();
-    }
-    sums[which] = s;
+  __shared__ double buf[2][1024];
+  __shared__ double sums[2];
+  const int which = threadIdx.x >> 7, tid = threadIdx.x & 127;  // two wavefronts per vector
+  const double* x = which == 0 ? a : b;
+  const int len = which == 0 ? n : n - 1;
+  double s = 0.0;
+  for (int base = 0; base < n; base += 1024) {
+    const int cnt = min(1024, len - base);
+    for (int i = tid; i < cnt; i += 128) buf[which][i] = x[base + i];
+    __syncthreads();
+    if (tid == 0)
+#pragma unroll 8
+      for (int i = 0; i < cnt; i++) {
+        const double v = buf[which][i];
+        s = s + v * v;
+      }
+    __syncthreads();
   }
+  if (tid == 0) sums[which] = s;
+  __syncthreads();
   if (threadIdx.x == 0) {
     const double na = sqrt(sums[0]), nb = sqrt(sums[1]);
     hdr->lo = 0.0;
@@ -101,6 +103,118 @@ __global__ void k_bisect_init(int n, const double* __restrict__ a, const double*
   }
 }
 
+// ---- levels that many values share
+//
+// Near the root many values lie in one node (the root [0, ||a||^2 + ||b||^2] is the square of the
+// largest value's scale: for order 1000 about 14 levels hold them all), and a group of lanes per
+// value would count the same nodes over and over. So the first steps give all lanes to the distinct
+// nodes: k_bisect_share evaluates the whole subtree of depth D below each of the N nodes, D =
+// log2(kShareLanes / N), and k_bisect_descend takes every value down it and lists the nodes they
+// reach. Two such steps cover about 29 levels of order 1000 (two steps with 64 lanes per value: 12).
+// kShareLanes is one wavefront per SIMD: a step is bound by the issue of its FP64 instructions, about
+// 65 ns per row and wavefront, so more lanes would only queue.
+constexpr int kShareLanes = 65536;
+constexpr int kShareMinN = 256;       // below this a step is shorter than its two launches
+constexpr int kShareMaxTargets = 16384;
+__device__ __forceinline__ int share_depth(int nodes) { return nodes > 0 ? 31 - __clz(kShareLanes / nodes) : 0; }
+
+struct ShareWs {
+  double *node_lo, *node_hi;  // distinct nodes
+  double *lo, *hi;            // per value: its node, the counts at its ends, its index in the list
+  int *clo, *chi, *node;
+  int* nodes;                 // their number
+  int* table;                 // kShareLanes counts
+};
+
+// first: the node is the root; the last workgroup counts its ends and fills the header.
+__global__ __launch_bounds__(256) void k_bisect_share(int n, const double* __restrict__ a,
+                                                      const double* __restrict__ b, BisectHdr* hdr, double tol,
+                                                      int first, ShareWs w) {
+  if (first && blockIdx.x == gridDim.x - 1) {
+    const double lo = hdr->lo, hi = hdr->hi;
+    if (threadIdx.x < 2) {
+      const int c = sturm_count(n, a, b, threadIdx.x == 0 ? lo : hi);
+      if (threadIdx.x == 0) hdr->nclo = c;
+      else hdr->nchi = c;
+    }
+    if (threadIdx.x == 2) {
+      const double mid = (lo + hi) / 2;
+      hdr->root_mid = mid;
+      hdr->root_leaf = ((hi - lo) <= tol || mid == lo || mid == hi) ? 1 : 0;
+      hdr->status = 0;
+      hdr->flags = 0;
+    }
+    return;
+  }
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  const int nodes = first ? 1 : *w.nodes;
+  const int D = share_depth(nodes);
+  const int node = g >> D, h = (g & ((1 << D) - 1)) + 1;
+  if (node >= nodes || h == (1 << D)) return;
+  double l = first ? hdr->lo : w.node_lo[node], r = first ? hdr->hi : w.node_hi[node];
+  for (int bit = 30 - __clz(h); bit >= 0; --bit) {
+    const double mm = (l + r) / 2;
+    if ((h >> bit) & 1) l = mm;
+    else r = mm;
+  }
+  w.table[g] = sturm_count(n, a, b, (l + r) / 2);
+}
+
+// Every value down the counted subtree of its node, by the rules of k_bisect_targets, then the list
+// of distinct nodes reached (values are in descending order, so equal nodes are neighbours).
+__global__ __launch_bounds__(1024) void k_bisect_descend(BisectHdr* hdr, double tol, int cap, int first, ShareWs w) {
+  __shared__ int part[1024];
+  const int tid = threadIdx.x;
+  const int nclo = hdr->nclo, nchi = hdr->nchi;
+  int T = (nclo <= nchi) ? min(cap, nchi - nclo) : 0;
+  if (hdr->root_leaf) T = 0;
+  const int D = share_depth(first ? 1 : *w.nodes);
+  for (int q = tid; q < T; q += 1024) {
+    const int t = nchi - 1 - q, node = first ? 0 : w.node[q];
+    double lo = first ? hdr->lo : w.lo[q], hi = first ? hdr->hi : w.hi[q];
+    int clo = first ? nclo : w.clo[q], chi = first ? nchi : w.chi[q];
+    bool monotone = true;
+    int hc = 1;
+    for (int lev = 0; lev < D; ++lev) {
+      const double md = (lo + hi) / 2;
+      if ((hi - lo) <= tol || md == lo || md == hi) break;
+      const int cnt = w.table[(node << D) + hc - 1];
+      monotone = monotone && clo <= cnt && cnt <= chi;
+      if (t < cnt) { hi = md; chi = cnt; hc = 2 * hc; }
+      else { lo = md; clo = cnt; hc = 2 * hc + 1; }
+    }
+    w.lo[q] = lo;
+    w.hi[q] = hi;
+    w.clo[q] = clo;
+    w.chi[q] = chi;
+    if (!monotone) atomicOr(&hdr->flags, 2);
+  }
+  __syncthreads();
+  const int per = (T + 1023) / 1024;
+  const int s0 = min(T, tid * per), s1 = min(T, s0 + per);
+  auto starts = [&](int q) { return q == 0 || w.lo[q] != w.lo[q - 1] || w.hi[q] != w.hi[q - 1]; };
+  int local = 0;
+  for (int q = s0; q < s1; q++) local += starts(q) ? 1 : 0;
+  part[tid] = local;
+  __syncthreads();
+  for (int off = 1; off < 1024; off <<= 1) {
+    const int v = tid >= off ? part[tid - off] : 0;
+    __syncthreads();
+    part[tid] += v;
+    __syncthreads();
+  }
+  int pos = part[tid] - local;
+  for (int q = s0; q < s1; q++) {
+    if (starts(q)) {
+      w.node_lo[pos] = w.lo[q];
+      w.node_hi[pos] = w.hi[q];
+      pos++;
+    }
+    w.node[q] = pos - 1;
+  }
+  if (tid == 1023) *w.nodes = part[1023];
+}
+
 // One group of W lanes per singular value (target). Target q (descending order) is the
 // ascending index t = nchi - 1 - q. Per round the W-1 lanes evaluate the Sturm counts of the
 // W-1 interior nodes of the depth-log2(W) subtree below the current node (node intervals
@@ -108,13 +222,21 @@ __global__ void k_bisect_init(int n, const double* __restrict__ a, const double*
 // to log2(W) levels: left when t < count(mid) (the reference pushes that child, because it
 // holds singular values nc_low..nc_mid-1), right otherwise, stopping at the first leaf
 // ((hi-lo) <= tol, or mid equal to an end). These are exactly the nodes the reference's
-// depth-first search visits on the way to t, so the leaf is the same node.
+// depth-first search visits on the way to t, so the leaf is the same node. The search starts from
+// the shared levels' nodes when there are any. The last workgroup runs the LDL factorization that
+// the twisted factorization needs later, when l is given.
 template <int W>
 __global__ __launch_bounds__(256) void k_bisect_targets(int n, const double* __restrict__ a,
                                                         const double* __restrict__ b,
                                                         const BisectHdr* __restrict__ hdr, double tol, int cap,
                                                         double* __restrict__ llo, double* __restrict__ lhi,
-                                                        double* __restrict__ lmid, int* __restrict__ flags) {
+                                                        double* __restrict__ lmid, int* __restrict__ flags,
+                                                        ShareWs w, double* __restrict__ l_out,
+                                                        double* __restrict__ d_out) {
+  if (l_out && blockIdx.x == gridDim.x - 1) {
+    if (threadIdx.x == 0) ldl_seq(n, a, b, l_out, d_out);
+    return;
+  }
   constexpr int D = (W == 1) ? 1 : (W == 2 ? 1 : W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6);
   const int lane = threadIdx.x;
   const int gid = (blockIdx.x * blockDim.x + lane) / W;
@@ -124,8 +246,8 @@ __global__ __launch_bounds__(256) void k_bisect_targets(int n, const double* __r
   if (hdr->root_leaf) T = 0;
   if (gid >= T) return;  // uniform within the group
   const int t = nchi - 1 - gid;
-  double lo = hdr->lo, hi = hdr->hi;
-  int clo = nclo, chi = nchi;
+  double lo = w.lo ? w.lo[gid] : hdr->lo, hi = w.lo ? w.hi[gid] : hdr->hi;
+  int clo = w.lo ? w.clo[gid] : nclo, chi = w.lo ? w.chi[gid] : nchi;
   bool monotone = true;
   const int h = j + 1;
   const int lvl = 31 - __clz(h);
@@ -229,170 +351,287 @@ __global__ void k_ldl(int n, const double* __restrict__ a, const double* __restr
   ldl_seq(n, a, b, l, d);
 }
 
-// One lane per singular value: dstqds, dpqds, twist, inverse iteration for v, coupling, twist
-// and inverse iteration for u (bbtsvd.cpp:65-135). The per-value sequences s, p, d+, r+ live in
-// HBM interleaved by value (element i of value j at i*k + j), so a wavefront's accesses are
-// contiguous. l+ and u+ are recomputed from them with the reference's expressions instead of
-// being stored. v is written interleaved (vs) and transposed afterwards; u is written in place
-// (column j of the n x k row-major u is interleaved by construction).
-__global__ __launch_bounds__(256) void k_twisted(int n, int k, const double* __restrict__ a,
-                                                 const double* __restrict__ b, const double* __restrict__ l,
-                                                 const double* __restrict__ d, const double* __restrict__ omega,
-                                                 double* __restrict__ u, double* __restrict__ vs,
-                                                 double* __restrict__ S, double* __restrict__ Pp,
-                                                 double* __restrict__ DP, double* __restrict__ RP,
-                                                 int* __restrict__ twists) {
-  // four wavefronts per 64 values: wavefront 0 runs the recurrences; then wavefronts 0 and 1
-  // find the two twist indices, the four inverse-iteration sweeps (v and u, each backward and
-  // forward from its twist) run one per wavefront, and wavefronts 0 and 1 normalize v and u
-  const int wave = threadIdx.x >> 6;
-  const int j = blockIdx.x * 64 + (threadIdx.x & 63);
-  const bool active = j < k;
-  const size_t K = (size_t)k;
-  auto at = [&](int i) -> size_t { return (size_t)i * K + j; };
-  const double w = active ? omega[j] : 0.0;  // lanes past k read nothing (they only join the barriers)
-  const double w2 = w * w;
+// ---- twisted factorization (bbtsvd.cpp:65-135)
+//
+// Per value: dstqds, dpqds, twist, inverse iteration for v, coupling, twist and inverse iteration for
+// u. The sequences s, p, d+, r+ of all values live in HBM interleaved by value (element i of value
+// j at i*k + j), so a wavefront of 64 values accesses contiguous memory. Only three parts are chains
+// that must run in index order: the two recurrences (k_qds), the products of the inverse iteration
+// and the sums of squares (k_twist_chain); each is one wavefront per 64 values. Everything else, the
+// searches for the twists, the multipliers with their divisions, the scaling, is independent
+// per element and runs in chunks of kRows rows over the whole chip. One launch that did it all had
+// k / 64 workgroups on 256 CUs and waited on memory in each: n = k = 2000 took 2.41 ms, 0.65 now;
+// n = k = 1000 1.01 ms, 0.34 now. l+ and u+ are recomputed from the sequences with the reference's
+// expressions instead of being stored; every value is evaluated by the reference's expressions in
+// the reference's order.
+constexpr int kRows = 32;
 
-  // dstqds (bbtsvd.cpp:73-81, forward) and dpqds (bbtsvd.cpp:83-91, backward) are independent
-  // recurrences: one loop runs both, so the two chains of dependent divisions overlap. Each
-  // chain evaluates the reference's expressions in the reference's order.
-  if (wave == 0 && active) {
-  double sc = -w2;
-  S[at(0)] = sc;
-  double pc = d[n - 1] - w2;
-  Pp[at(n - 1)] = pc;
-  #pragma unroll 2
-  for (int t = 0; t < n - 1; t++) {
-    const int i = t;          // dstqds step
-    const int q = n - 2 - t;  // dpqds step
-    const double dp = d[i] + sc;
-    const double rp = d[q] * (l[q] * l[q]) + pc;
-    const double lp = d[i] * l[i] / dp;
-    const double pq = pc * d[q] / rp;
-    DP[at(i)] = dp;
-    RP[at(q + 1)] = rp;
-    sc = lp * l[i] * sc - w2;
-    pc = pq - w2;
-    S[at(i + 1)] = sc;
-    Pp[at(q)] = pc;
-  }
-  DP[at(n - 1)] = d[n - 1] + sc;
-  RP[at(0)] = pc;
-  }
-  __syncthreads();  // the sequences are visible to every wavefront of the workgroup
-  const int lane = threadIdx.x & 63;
-  __shared__ int twist_at[2][64];  // k0 (v side) and k1 (u side) of each value
-  // coupling (bbtsvd.cpp:113-124): s[n] = -omega^2, p[n] = 1, r+[n] = 1
-  auto Sv = [&](int i) -> double { return i == n ? -w2 : S[at(i)]; };
-  auto Pv = [&](int i) -> double { return i == n ? 1.0 : Pp[at(i)]; };
-  auto Rv = [&](int i) -> double { return i == n ? 1.0 : RP[at(i)]; };
-  if (active && wave == 0) {
-    // twist: first index of min |s + p + omega^2|
-    int k0 = 0;
-    double best = 0.0;
-    #pragma unroll 16
-    for (int i = 0; i < n; i++) {
-      const double g = S[at(i)] + Pp[at(i)] + w2;
-      const double ag = fabs(g);
-      if (i == 0 || ag < best) { best = ag; k0 = i; }
+struct Twist {
+  int n, k;
+  const double *a, *b, *l, *d, *omega;
+  double *u, *vs;             // u in place (column j of the n x k row-major u), v interleaved
+  double *S, *P, *DP, *RP;
+  double* best;               // [2][chunks][k]: least |gamma| of a chunk (v, u), then largest |v|
+  int* at;                    // [2][chunks][k]: its index
+  int* twist;                 // [2][k]
+  double* inv;                // [2][k]: 1 / norm
+  int chunks;
+};
+
+// dstqds (bbtsvd.cpp:73-81, forward) on wavefront 0 and dpqds (bbtsvd.cpp:83-91, backward) on
+// wavefront 1, independent chains with a division per step. The uniform d and l of the next eight
+// steps are loaded while these eight run.
+__global__ __launch_bounds__(128) void k_qds(Twist T) {
+  const int n = T.n, jj = blockIdx.x * 64 + (threadIdx.x & 63);
+  const bool active = jj < T.k;
+  const int j = min(jj, T.k - 1);
+  const size_t K = (size_t)T.k;
+  const double* __restrict__ d = T.d;
+  const double* __restrict__ l = T.l;
+  const double w = T.omega[j], w2 = w * w;
+  constexpr int U = 8;
+  double dc[U], lc[U], dn[U], ln[U];
+  const int steps = n - 1;
+  const bool fwd = threadIdx.x < 64;
+  auto load = [&](int t0, double* dd, double* ll) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+      const int t = min(t0 + q, max(steps - 1, 0));
+      const int i = fwd ? t : steps - 1 - t;
+      dd[q] = steps > 0 ? d[i] : 0.0;
+      ll[q] = steps > 0 ? l[i] : 0.0;
     }
-    twist_at[0][lane] = k0;
-    vs[at(k0)] = 1.0;
-    if (twists) twists[2 * j] = k0;
-  }
-  if (active && wave == 1) {
-    int k1 = 0;
-    double best = 0.0;
-    #pragma unroll 16
-    for (int i = 0; i < n; i++) {
-      const double si = Sv(i), pi = Pv(i);
-      const double g = si + pi + w2;
-      const double gn = -w2 * g * Rv(i + 1) / (si * Pv(i + 1));
-      const double ag = fabs(gn);
-      if (i == 0 || ag < best) { best = ag; k1 = i; }
+  };
+  if (fwd) {
+    double sc = -w2;
+    if (active) T.S[j] = sc;
+    load(0, dc, lc);
+    for (int t0 = 0; t0 < steps; t0 += U) {
+      load(t0 + U, dn, ln);
+#pragma unroll
+      for (int q = 0; q < U; q++) {
+        const int i = t0 + q;
+        if (i < steps) {
+          const double dp = dc[q] + sc;
+          const double lp = dc[q] * lc[q] / dp;
+          sc = lp * lc[q] * sc - w2;
+          if (active) {
+            T.DP[i * K + j] = dp;
+            T.S[(i + 1) * K + j] = sc;
+          }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < U; q++) { dc[q] = dn[q]; lc[q] = ln[q]; }
     }
-    twist_at[1][lane] = k1;
-    u[at(k1)] = 1.0;
-    if (twists) twists[2 * j + 1] = k1;
+    if (active) T.DP[(n - 1) * K + j] = d[n - 1] + sc;
+  } else {
+    double pc = d[n - 1] - w2;
+    if (active) T.P[(n - 1) * K + j] = pc;
+    load(0, dc, lc);
+    for (int t0 = 0; t0 < steps; t0 += U) {
+      load(t0 + U, dn, ln);
+#pragma unroll
+      for (int q = 0; q < U; q++) {
+        const int i = n - 2 - (t0 + q);
+        if (i >= 0) {
+          const double rp = dc[q] * (lc[q] * lc[q]) + pc;
+          const double pq = pc * dc[q] / rp;
+          pc = pq - w2;
+          if (active) {
+            T.RP[(i + 1) * K + j] = rp;
+            T.P[i * K + j] = pc;
+          }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < U; q++) { dc[q] = dn[q]; lc[q] = ln[q]; }
+    }
+    if (active) T.RP[j] = pc;
   }
-  __syncthreads();
-  // the four inverse-iteration sweeps, one per wavefront: v (bbtsvd.cpp:65-71) with
-  // l+ = d l / d+, u+ = l d / r+; u with l+_i = a_{i+1} / d+'_i b_i, u+_i = a_{i+1} / r+'_{i+1} b_i,
-  // d+'_i = s_{i+1} / s_i d+_i, r+'_i = p_i / p_{i+1} r+_{i+1}
+}
+
+// Least |gamma| of each chunk of rows and its first index: v side on wavefront 0 (|s + p +
+// omega^2|), u side on wavefront 1 (the coupling, bbtsvd.cpp:113-124, with s[n] = -omega^2, p[n] =
+// 1, r+[n] = 1). The search takes row 0 whatever it holds and then only strictly smaller values, so
+// later chunks start from +inf.
+__global__ __launch_bounds__(128) void k_twist_min(Twist T) {
+  const int n = T.n, side = threadIdx.x >> 6, jj = blockIdx.x * 64 + (threadIdx.x & 63);
+  const bool active = jj < T.k;
+  const int j = min(jj, T.k - 1), i0 = blockIdx.y * kRows;
+  const size_t K = (size_t)T.k;
+  const double w = T.omega[j], w2 = w * w;
+  double best = __longlong_as_double(0x7ff0000000000000LL);
+  int at = -1;
+  // rows past the end are read again and not used: no branch stands between the loads
+#pragma unroll 8
+  for (int q = 0; q < kRows; q++) {
+    const int i = min(i0 + q, n - 1), h = min(i + 1, n - 1);
+    const double si = T.S[i * K + j], pi = T.P[i * K + j];
+    double g = si + pi + w2;
+    if (side == 1) {
+      const double rh = T.RP[h * K + j], ph = T.P[h * K + j];
+      const double r1 = i + 1 == n ? 1.0 : rh, p1 = i + 1 == n ? 1.0 : ph;
+      g = -w2 * g * r1 / (si * p1);
+    }
+    const double ag = fabs(g);
+    const bool take = i0 + q < n && (i == 0 || ag < best);
+    best = take ? ag : best;
+    at = take ? i : at;
+  }
   if (active) {
-    double z = 1.0;
-    if (wave == 0) {
-      const int k0 = twist_at[0][lane];
-      #pragma unroll 16
-      for (int i = k0 - 1; i >= 0; i--) {
-        const double lp = d[i] * l[i] / DP[at(i)];
-        z = -lp * z;
-        vs[at(i)] = z;
-      }
-    } else if (wave == 1) {
-      const int k0 = twist_at[0][lane];
-      #pragma unroll 16
-      for (int i = k0 + 1; i < n; i++) {
-        const double up = l[i - 1] * d[i - 1] / RP[at(i)];
-        z = -up * z;
-        vs[at(i)] = z;
-      }
-    } else if (wave == 2) {
-      const int k1 = twist_at[1][lane];
-      #pragma unroll 16
-      for (int i = k1 - 1; i >= 0; i--) {
-        const double dpn = Sv(i + 1) / Sv(i) * DP[at(i)];
-        const double lpn = a[i + 1] / dpn * b[i];
-        z = -lpn * z;
-        u[at(i)] = z;
-      }
+    const size_t e = ((size_t)side * T.chunks + blockIdx.y) * K + j;
+    T.best[e] = best;
+    T.at[e] = at;
+  }
+}
+
+// The twists: the chunks' minima combined in order.
+__global__ __launch_bounds__(256) void k_twist_pick(Twist T, int* __restrict__ twists) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= 2 * T.k) return;
+  const int side = e / T.k, j = e - side * T.k;
+  const size_t base = (size_t)side * T.chunks * T.k + j;
+  double best = T.best[base];
+  int at = T.at[base];
+#pragma unroll 8
+  for (int c = 1; c < T.chunks; c++) {
+    const double g = T.best[base + (size_t)c * T.k];
+    const int i = T.at[base + (size_t)c * T.k];
+    if (g < best) { best = g; at = i; }
+  }
+  T.twist[e] = at;
+  if (twists) twists[2 * j + side] = at;
+}
+
+// Multipliers of the inverse iteration (bbtsvd.cpp:65-71) into the vectors' own places, one at the
+// twist: v with -l+ = -(d l / d+) before it and -u+ = -(l d / r+) after it; u with the coupled l+_i
+// = a_{i+1} / d+'_i b_i, u+_i = a_{i+1} / r+'_{i+1} b_i, d+'_i = s_{i+1} / s_i d+_i, r+'_i = p_i /
+// p_{i+1} r+_{i+1}. Two wavefronts per side, half a chunk each.
+__global__ __launch_bounds__(256) void k_twist_mult(Twist T) {
+  const int n = T.n, wave = threadIdx.x >> 6, side = wave >> 1, jj = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int j = min(jj, T.k - 1), i0 = blockIdx.y * kRows + (wave & 1) * (kRows / 2);
+  if (jj >= T.k) return;
+  const size_t K = (size_t)T.k;
+  const int k0 = T.twist[side * T.k + j];
+#pragma unroll 8
+  for (int q = 0; q < kRows / 2; q++) {
+    const int i = min(i0 + q, n - 1), g = min(i + 1, n - 1);
+    const size_t e = i * K + j, f = g * K + j;
+    const bool low = i < k0, last = i + 1 == n, in = i0 + q < n;
+    if (side == 0) {
+      const int h = min(max(low ? i : i - 1, 0), max(n - 2, 0));
+      const double num = n > 1 ? T.d[h] * T.l[h] : 0.0;
+      const double dp = T.DP[e], rp = T.RP[e];
+      const double m = -(num / (low ? dp : rp));
+      if (in) T.vs[e] = i == k0 ? 1.0 : m;
     } else {
-      const int k1 = twist_at[1][lane];
-      #pragma unroll 16
-      for (int i = k1 + 1; i < n; i++) {
-        const int q = i - 1;
-        const double rpn = Pv(q + 1) / Pv(q + 2) * Rv(q + 2);
-        const double upn = a[q + 1] / rpn * b[q];
-        z = -upn * z;
-        u[at(i)] = z;
-      }
+      const double s0 = T.S[e], s1 = T.S[f], p0 = T.P[e], pf = T.P[f], dp = T.DP[e], rf = T.RP[f];
+      const double p1 = last ? 1.0 : pf, r1 = last ? 1.0 : rf;
+      const double x = (low ? s1 : p0) / (low ? s0 : p1) * (low ? dp : r1);
+      const int hb = min(max(low ? i : i - 1, 0), max(n - 2, 0));
+      const double m = -(T.a[low ? g : i] / x * (n > 1 ? T.b[hb] : 0.0));
+      if (in) T.u[e] = i == k0 ? 1.0 : m;
     }
   }
-  __syncthreads();
-  // normalization: the sum of squares in index order, then the scaling (wave 0: v, wave 1: u)
-  if (active && wave < 2) {
-    double* vec = wave == 0 ? vs : u;
-    double ss = 0.0;
-    #pragma unroll 16
-    for (int i = 0; i < n; i++) {
-      const double v = vec[at(i)];
-      ss = ss + v * v;
+}
+
+// The chains of 64 values: the products outward from the twist (v and u, backward and forward, a
+// wavefront each; rows in step for all values, so that accesses stay contiguous although the twists
+// differ), then the sums of squares in index order. Blocks of kDeep rows are read one block ahead.
+constexpr int kDeep = 32;
+__global__ __launch_bounds__(256, 1) void k_twist_chain(Twist T) {
+  const int n = T.n, wave = threadIdx.x >> 6, side = wave >> 1, jj = blockIdx.x * 64 + (threadIdx.x & 63);
+  const bool active = jj < T.k;
+  const int j = min(jj, T.k - 1);
+  const size_t K = (size_t)T.k;
+  double* vec = (side == 0 ? T.vs : T.u) + j;
+  const int k0 = T.twist[side * T.k + j];
+  const bool back = (wave & 1) == 0;
+  double cur[kDeep], nxt[kDeep];
+  // row of step t: downward from n - 1 for the backward sweep
+  auto load = [&](int t0, double* x, bool down) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < kDeep; q++) {
+      const int t = min(t0 + q, n - 1);
+      x[q] = vec[(down ? n - 1 - t : t) * K];
     }
-    const double inv = 1.0 / sqrt(ss);
-    #pragma unroll 16
-    for (int i = 0; i < n; i++) vec[at(i)] = inv * vec[at(i)];
+  };
+  double z = 1.0;
+  load(0, cur, back);
+  for (int t0 = 0; t0 < n; t0 += kDeep) {
+    load(t0 + kDeep, nxt, back);
+#pragma unroll
+    for (int q = 0; q < kDeep; q++) {
+      const int t = t0 + q, i = back ? n - 1 - t : t;
+      const bool on = t < n && (back ? i < k0 : i > k0);
+      z = on ? cur[q] * z : z;
+      if (on && active) vec[i * K] = z;
+    }
+#pragma unroll
+    for (int q = 0; q < kDeep; q++) cur[q] = nxt[q];
+  }
+  __syncthreads();  // both sweeps of a vector are visible to the wavefront that sums it
+  if (!back) return;
+  double ss = 0.0;
+  load(0, cur, false);
+  for (int t0 = 0; t0 < n; t0 += kDeep) {
+    load(t0 + kDeep, nxt, false);
+#pragma unroll
+    for (int q = 0; q < kDeep; q++) ss = t0 + q < n ? ss + cur[q] * cur[q] : ss;
+#pragma unroll
+    for (int q = 0; q < kDeep; q++) cur[q] = nxt[q];
+  }
+  if (active) T.inv[side * T.k + j] = 1.0 / sqrt(ss);
+}
+
+// Scaling to unit length, v on wavefront 0 (with each chunk's largest |v_i| and its first index, for
+// the sign rule), u on wavefront 1.
+__global__ __launch_bounds__(128) void k_twist_scale(Twist T) {
+  const int n = T.n, side = threadIdx.x >> 6, j = blockIdx.x * 64 + (threadIdx.x & 63), i0 = blockIdx.y * kRows;
+  if (j >= T.k) return;
+  const size_t K = (size_t)T.k;
+  double* vec = (side == 0 ? T.vs : T.u) + j;
+  const double inv = T.inv[side * T.k + j];
+  double best = -1.0, row[kRows];
+  int at = 0;
+#pragma unroll
+  for (int q = 0; q < kRows; q++) {
+    const int i = min(i0 + q, n - 1);
+    row[q] = vec[i * K];
+  }
+#pragma unroll
+  for (int q = 0; q < kRows; q++) {
+    const int i = i0 + q;
+    const double x = inv * row[q];
+    if (i < n) vec[i * K] = x;
+    const bool take = i < n && fabs(x) > best;
+    best = take ? fabs(x) : best;
+    at = take ? i : at;
+  }
+  if (side == 0) {
+    T.best[(size_t)blockIdx.y * K + j] = best;
+    T.at[(size_t)blockIdx.y * K + j] = at;
   }
 }
 
 // Sign of v (bbtsvd.cpp:943-955): p = first index of max |v_j|, signer = (B^T u_j)_p / sigma_j.
-__global__ __launch_bounds__(256) void k_vsign(int n, int k, const double* __restrict__ a,
-                                               const double* __restrict__ b, const double* __restrict__ sigma,
-                                               const double* __restrict__ u, const double* __restrict__ vs,
-                                               double* __restrict__ sgn) {
+__global__ __launch_bounds__(64) void k_vsign(Twist T, const double* __restrict__ sigma, double* __restrict__ sgn) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= k) return;
-  const size_t K = (size_t)k;
-  int p = 0;
+  if (j >= T.k) return;
+  const size_t K = (size_t)T.k;
   double best = -1.0;
+  int p = 0;
 #pragma unroll 8
-  for (int i = 0; i < n; i++) {
-    const double av = fabs(vs[(size_t)i * K + j]);
-    if (av > best) { best = av; p = i; }
+  for (int c = 0; c < T.chunks; c++) {
+    const double x = T.best[c * K + j];
+    const int i = T.at[c * K + j];
+    if (x > best) { best = x; p = i; }
   }
   double signer;
-  if (p == 0) signer = u[(size_t)p * K + j] * a[p] / sigma[j];
-  else signer = (u[(size_t)(p - 1) * K + j] * b[p - 1] + u[(size_t)p * K + j] * a[p]) / sigma[j];
-  sgn[j] = ((signer * vs[(size_t)p * K + j]) < 0) ? -1.0 : 1.0;
+  if (p == 0) signer = T.u[(size_t)p * K + j] * T.a[p] / sigma[j];
+  else signer = (T.u[(size_t)(p - 1) * K + j] * T.b[p - 1] + T.u[(size_t)p * K + j] * T.a[p]) / sigma[j];
+  sgn[j] = ((signer * T.vs[(size_t)p * K + j]) < 0) ? -1.0 : 1.0;
 }
 
 // v (k x n) = sign_j * vs^T, through a 64 x 64 LDS tile.
@@ -443,22 +682,26 @@ struct Bump {
   bool ok() const { return used <= cap; }
 };
 
+// Lanes per value: the most that leave every SIMD one wavefront (a wider group's rounds are fewer
+// but queue: 2000 values at n = 2000 took 2.54 ms with 64 lanes each, with 32 after the two shared
+// steps 1.19, and 0.34 in those).
 int pick_w(int targets) {
-  long lanes = 262144;  // about four wavefronts per SIMD across the chip
   int w = 64;
-  while (w > 1 && (long)targets * w > lanes) w >>= 1;
+  while (w > 1 && (long)targets * w > kShareLanes) w >>= 1;
   return w;
 }
 
 int launch_targets(int n, const double* a, const double* b, const BisectHdr* hdr, double tol, int cap, double* llo,
-                   double* lhi, double* lmid, int* flags, hipStream_t s) {
-  if (cap <= 0) return EXC_OK;
-  const int W = pick_w(cap);
-  const unsigned grid = exc_detail::ceil_div((long)cap * W, 256);
+                   double* lhi, double* lmid, int* flags, const ShareWs& share, double* ldl_l, double* ldl_d,
+                   hipStream_t s) {
+  const int W = pick_w(std::max(cap, 0));
+  cap = std::max(cap, 0);
+  const unsigned grid = exc_detail::ceil_div((long)cap * W, 256) + (ldl_l ? 1 : 0);
+  if (grid == 0) return EXC_OK;
 #define EXC_TGT(WW)                                                                                  \
   case WW:                                                                                           \
     hipLaunchKernelGGL(k_bisect_targets<WW>, dim3(grid), dim3(256), 0, s, n, a, b, hdr, tol, cap,   \
-                       llo, lhi, lmid, flags);                                                       \
+                       llo, lhi, lmid, flags, share, ldl_l, ldl_d);                                  \
     break;
   switch (W) {
     EXC_TGT(1) EXC_TGT(2) EXC_TGT(4) EXC_TGT(8) EXC_TGT(16) EXC_TGT(32) EXC_TGT(64)
@@ -477,6 +720,7 @@ struct BisectWs {
   int *f_clo[2], *f_chi[2];
   int* ctr;  // [0] frontier size (next), [1] leaf count, [2] overflow
   double *L_lo, *L_hi;
+  ShareWs share;  // in the replay's frontiers, which are not in use at the same time
 };
 
 size_t bisect_ws_bytes(int n, void* base, BisectWs* ws, Bump* bump) {
@@ -496,6 +740,8 @@ size_t bisect_ws_bytes(int n, void* base, BisectWs* ws, Bump* bump) {
   w.ctr = B.take<int>(4);
   w.L_lo = B.take<double>(w.cap);
   w.L_hi = B.take<double>(w.cap);
+  w.share = ShareWs{w.f_lo[0], w.f_hi[0], w.f_lo[1], w.f_hi[1], w.f_clo[1], w.f_chi[1], w.f_clo[0], w.ctr,
+                    B.take<int>(kShareLanes)};
   if (ws) *ws = w;
   (void)base;
   return B.used;
@@ -602,12 +848,30 @@ int run_bfs(int n, const double* a, const double* b, double tol, int top_k, doub
 int run_bisection(int n, const double* a, const double* b, double tol, int top_k, double* sigma, int* count,
                   double* olo, double* ohi, const BisectWs& w, hipStream_t s, double* ldl_l = nullptr,
                   double* ldl_d = nullptr) {
-  hipLaunchKernelGGL(k_bisect_init, dim3(1), dim3(128), 0, s, n, a, b, tol, w.hdr, ldl_l, ldl_d);
-  EXC_CHECK_HIP(hipGetLastError());
   int cap = min(n, top_k + 64);
+  const bool small = n < kShareMinN;
+  if (small) {
+    hipLaunchKernelGGL(k_bisect_init, dim3(1), dim3(128), 0, s, n, a, b, tol, w.hdr, ldl_l, ldl_d);
+    EXC_CHECK_HIP(hipGetLastError());
+    ldl_l = ldl_d = nullptr;  // done there
+  }
   for (int attempt = 0; attempt < 2; attempt++) {
-    int rc = launch_targets(n, a, b, w.hdr, tol, cap, w.llo, w.lhi, w.lmid, &w.hdr->flags, s);
+    ShareWs share = w.share;
+    if (!small) {
+      const int steps = cap <= kShareMaxTargets ? 2 : 1;
+      for (int step = 0; step < steps; step++) {
+        const int first = step == 0;
+        hipLaunchKernelGGL(k_bisect_share, dim3(kShareLanes / 256 + first), dim3(256), 0, s, n, a, b, w.hdr, tol,
+                           first, share);
+        hipLaunchKernelGGL(k_bisect_descend, dim3(1), dim3(1024), 0, s, w.hdr, tol, cap, first, share);
+      }
+      EXC_CHECK_HIP(hipGetLastError());
+    } else {
+      share.lo = nullptr;
+    }
+    int rc = launch_targets(n, a, b, w.hdr, tol, cap, w.llo, w.lhi, w.lmid, &w.hdr->flags, share, ldl_l, ldl_d, s);
     if (rc) return rc;
+    ldl_l = ldl_d = nullptr;  // once
     hipLaunchKernelGGL(k_bisect_compact, dim3(1), dim3(1024), 0, s, w.hdr, top_k, cap, w.llo, w.lhi, w.lmid,
                        sigma, count, olo, ohi);
     EXC_CHECK_HIP(hipGetLastError());
@@ -671,7 +935,8 @@ int exc_ldl(int n, const double* d_alpha, const double* d_beta, double* d_l, dou
 
 namespace {
 struct TwistWs {
-  double *l, *d, *S, *P, *DP, *RP, *vs, *sgn;
+  double *l, *d, *S, *P, *DP, *RP, *vs, *sgn, *best, *inv;
+  int *at, *twist;
 };
 void twist_ws(int n, int k, Bump& B, TwistWs* w) {
   w->l = B.take<double>(n);
@@ -682,6 +947,11 @@ void twist_ws(int n, int k, Bump& B, TwistWs* w) {
   w->RP = B.take<double>((size_t)(n + 1) * k);
   w->vs = B.take<double>((size_t)n * k);
   w->sgn = B.take<double>(k);
+  const size_t chunks = ((size_t)n + kRows - 1) / kRows;
+  w->best = B.take<double>(2 * chunks * k);
+  w->at = B.take<int>(2 * chunks * k);
+  w->twist = B.take<int>(2 * (size_t)k);
+  w->inv = B.take<double>(2 * (size_t)k);
 }
 
 int run_twisted(int n, int k, const double* omega, const double* a, const double* b, double* u, double* v,
@@ -691,12 +961,18 @@ int run_twisted(int n, int k, const double* omega, const double* a, const double
     hipLaunchKernelGGL(k_ldl, dim3(1), dim3(64), 0, s, n, a, b, w.l, w.d);
     EXC_CHECK_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL(k_twisted, dim3(exc_detail::ceil_div(k, 64)), dim3(256), 0, s, n, k, a, b, w.l, w.d, omega, u,
-                     w.vs, w.S, w.P, w.DP, w.RP, twists);
+  const int chunks = (n + kRows - 1) / kRows;
+  const Twist T{n, k, a, b, w.l, w.d, omega, u, w.vs, w.S, w.P, w.DP, w.RP, w.best, w.at, w.twist, w.inv, chunks};
+  const unsigned groups = exc_detail::ceil_div(k, 64);
+  hipLaunchKernelGGL(k_qds, dim3(groups), dim3(128), 0, s, T);
+  hipLaunchKernelGGL(k_twist_min, dim3(groups, chunks), dim3(128), 0, s, T);
+  hipLaunchKernelGGL(k_twist_pick, dim3(exc_detail::ceil_div(2L * k, 256)), dim3(256), 0, s, T, twists);
+  hipLaunchKernelGGL(k_twist_mult, dim3(groups, chunks), dim3(256), 0, s, T);
+  hipLaunchKernelGGL(k_twist_chain, dim3(groups), dim3(256), 0, s, T);
+  hipLaunchKernelGGL(k_twist_scale, dim3(groups, chunks), dim3(128), 0, s, T);
   EXC_CHECK_HIP(hipGetLastError());
   if (apply_vsign) {
-    hipLaunchKernelGGL(k_vsign, dim3(exc_detail::ceil_div(k, 64)), dim3(64), 0, s, n, k, a, b, sigma_for_sign, u,
-                       w.vs, w.sgn);
+    hipLaunchKernelGGL(k_vsign, dim3(groups), dim3(64), 0, s, T, sigma_for_sign, w.sgn);
     EXC_CHECK_HIP(hipGetLastError());
   }
   hipLaunchKernelGGL(k_transpose_sign, dim3(exc_detail::ceil_div(k, 64), exc_detail::ceil_div(n, 64)), dim3(256), 0, s,

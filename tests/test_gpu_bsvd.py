@@ -129,3 +129,21 @@ def test_bisection_nonmonotone_counts_bit_exact(hip, oracle, n):
     so, loo, hio = oracle.bisection(a, b, 0.0, ub, 1e-20, n)
     assert np.array_equal(sg, so)
     assert np.array_equal(lo, loo) and np.array_equal(hi, hio)
+
+
+@pytest.mark.parametrize("kind", ["gauss", "graded", "clustered"])
+@pytest.mark.parametrize("n,top_k", [(31, 31), (32, 7), (33, 33), (97, 65), (255, 255), (256, 256), (257, 3),
+                                     (1026, 1026), (1300, 129)])
+def test_bidiag_svd_edges(hip, oracle, kind, n, top_k):
+    """Orders around the chunks of 32 rows, the order from which the first levels are shared and the
+    values that halve the lanes per value; value counts around the wavefront. Bit for bit."""
+    banner(f"bidiag_svd edges n={n} top_k={top_k} kind={kind}")
+    a, b = random_bidiagonal(np.random.default_rng(n + top_k), n, kind)
+    so, uo, vo, two, rco = oracle.bidiag_svd(a, b, top_k)
+    sg, ug, vg, twg, rcg = hip.bidiag_svd(a, b, top_k)
+    if rco < 0:
+        assert rcg == -5
+        return
+    assert rcg == 0
+    assert np.array_equal(sg, so) and np.array_equal(twg, two)
+    assert np.array_equal(ug, uo) and np.array_equal(vg, vo)
