@@ -231,36 +231,70 @@ __device__ __forceinline__ int potf2_loop(double* S, double* xc, int kb) {
   return bad;
 }
 
-// LU without pivoting of S - diag(s) (sign rule of the Householder reconstruction), lane i = row
-// i; row j is published through LDS at step j. sgn receives s for the kb valid pivots.
-__device__ __forceinline__ void getf2_reg(double* S, double* xr, int kb, double* sgn, bool last_plus) {
+// LU without pivoting of S - diag(s) (sign rule of the Householder reconstruction), lane i = row i.
+// sgn receives s for the kb valid pivots. As in potf2_loop only a panel of PW columns is unrolled:
+// inside it row j reaches the other lanes by v_readlane; then the panel's PW rows of U are finished
+// for the later columns and every lane takes the panel's rank-PW update of its row, blocks of 8
+// columns at a time in a loop, with U read from LDS. Every element receives the same fused
+// multiply-adds in the same order as a column-by-column right-looking factorization. (Fully unrolled
+// the routine was bound by instruction fetch, as potf2_loop's comment says.)
+__device__ __forceinline__ void getf2_loop(double* S, int kb, double* sgn, bool last_plus) {
   const int lane = threadIdx.x;
-  __asm__ volatile("" ::: "memory");  // keep this routine's loads inside its branch
-  double x[TB];
+  __asm__ volatile("" ::: "memory");
+#pragma unroll 1
+  for (int j0 = 0; j0 < TB; j0 += PW) {
+    double x[PW], l[PW];
 #pragma unroll
-  for (int k = 0; k < TB; k++) x[k] = S[lane * LD + k];
+    for (int jj = 0; jj < PW; jj++) x[jj] = S[lane * LD + j0 + jj];
 #pragma unroll
-  for (int j = 0; j < TB; j++) {
-    double* r = xr + (j & 1) * (TB + 1);  // row j (r[k], k > j) and the pivot (r[TB])
-    if (lane == j) {
-      const double w = x[j];
+    for (int jj = 0; jj < PW; jj++) {
+      const int j = j0 + jj;
+      const double w = readlane_f64(x[jj], j);
       double sj = signbit(w) ? 1.0 : -1.0;
       if (last_plus && j == kb - 1) sj = -sj;
-      x[j] = w - sj;
-      r[TB] = x[j];
-      if (j < kb) sgn[j] = sj;
+      const double piv = w - sj;
+      if (lane == 0 && j < kb) sgn[j] = sj;
+      const double rp = 1.0 / piv;
+      l[jj] = lane > j ? x[jj] * rp : 0.0;
+      x[jj] = lane == j ? piv : (lane > j ? l[jj] : x[jj]);
 #pragma unroll
-      for (int k = j + 1; k < TB; k++) r[k] = x[k];
+      for (int kk = jj + 1; kk < PW; kk++) x[kk] = fma(-l[jj], readlane_f64(x[kk], j), x[kk]);
+    }
+#pragma unroll
+    for (int jj = 0; jj < PW; jj++) S[lane * LD + j0 + jj] = x[jj];
+    wave_sync();
+    // the later columns: lane = column c first finishes the panel's rows of U there ...
+    const int c = lane;
+    if (c >= j0 + PW) {
+      double u[PW];
+#pragma unroll
+      for (int jj = 0; jj < PW; jj++) u[jj] = S[(j0 + jj) * LD + c];
+#pragma unroll
+      for (int jj = 0; jj < PW; jj++)
+#pragma unroll
+        for (int kk = jj + 1; kk < PW; kk++) u[kk] = fma(-S[(j0 + kk) * LD + j0 + jj], u[jj], u[kk]);
+#pragma unroll
+      for (int jj = 0; jj < PW; jj++) S[(j0 + jj) * LD + c] = u[jj];
     }
     wave_sync();
-    const double rp = 1.0 / r[TB];
-    const double l = lane > j ? x[j] * rp : 0.0;
-    if (lane > j) x[j] = l;
+    // ... then lane = row updates its row
+    const bool below = lane >= j0 + PW;
+#pragma unroll 1
+    for (int k0 = j0 + PW; k0 < TB; k0 += 8) {
+      double a[8];
 #pragma unroll
-    for (int k = j + 1; k < TB; k++) x[k] = fma(-l, r[k], x[k]);
+      for (int kk = 0; kk < 8; kk++) a[kk] = S[lane * LD + k0 + kk];
+#pragma unroll
+      for (int jj = 0; jj < PW; jj++)
+#pragma unroll
+        for (int kk = 0; kk < 8; kk++) a[kk] = fma(-l[jj], S[(j0 + jj) * LD + k0 + kk], a[kk]);
+      if (below) {
+#pragma unroll
+        for (int kk = 0; kk < 8; kk++) S[lane * LD + k0 + kk] = a[kk];
+      }
+    }
+    wave_sync();
   }
-#pragma unroll
-  for (int k = 0; k < TB; k++) S[lane * LD + k] = x[k];
 }
 
 // Off-diagonal tile solves against the final diagonal tile, read from HBM with wave-uniform
@@ -270,15 +304,10 @@ __device__ __forceinline__ void getf2_reg(double* S, double* xr, int kb, double*
 // staged in T (triangular inverse).
 template <int MODE>  // 0: rows, L^T; 1: rows, U; 2: columns, unit L; 3: columns, L
 __device__ __forceinline__ void tile_solve(double* S, double* T, const double* Dg, long lda, int kd) {
-  // The diagonal tile was finished by another workgroup. The LU modes copy it into LDS (T) with
-  // one batched coherent copy and substitute from there; the Cholesky mode, whose substitution
-  // walks rows of L^T, is faster reading it through the caches after one acquire fence.
-  if (MODE == 1 || MODE == 2) {
-    tile_to_lds(T, Dg, lda, 0, 0, kd, kd);
-    __syncthreads();
-  } else if (MODE == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  }  // MODE 3: the caller staged the diagonal tile in T
+  // The diagonal tile was finished by another workgroup. Except in the Cholesky mode the caller
+  // staged it in T; that mode's substitution walks rows of L^T and is faster reading it through
+  // the caches after one acquire fence.
+  if (MODE == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   __asm__ volatile("" ::: "memory");
   const int lane = threadIdx.x;
   double x[TB];
@@ -534,9 +563,25 @@ __host__ __device__ inline int lu_index(int i, int j, int nb) {
   return before + 2 * off - ((i < j) ? 1 : 0);
 }
 
-__global__ __launch_bounds__(TNT) void k_lu_tiles(int n, double* __restrict__ A, long lda, int nb,
-                                                  double* __restrict__ sgn, int square_last,
-                                                  int* __restrict__ done, int* __restrict__ error) {
+// acc -= X Y for this wavefront's row block (X, Y 64 x 64 in LDS)
+__device__ __forceinline__ void acc_update4_nn(d4 (&acc)[4], const Quad4& q, const double* X, const double* Y) {
+#pragma unroll 2
+  for (int kk = 0; kk < TB; kk += 4) {
+    const double xa = -X[(16 * q.w + q.li) * LD + kk + q.lk];
+    double yb[4];
+#pragma unroll
+    for (int b = 0; b < 4; b++) yb[b] = Y[(kk + q.lk) * LD + 16 * b + q.li];
+#pragma unroll
+    for (int b = 0; b < 4; b++) acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa, yb[b], acc[b], 0, 0, 0);
+  }
+}
+
+// Four wavefronts per tile, as in the Cholesky: updates, staging and stores split four ways, the
+// factorization and the solve on wavefront 0. Order 1000: 1.52 ms with one wavefront and the
+// unrolled factorization, 0.97 ms now.
+__global__ __launch_bounds__(TNT4) void k_lu_tiles(int n, double* __restrict__ A, long lda, int nb,
+                                                   double* __restrict__ sgn, int square_last,
+                                                   int* __restrict__ done, int* __restrict__ error) {
   extern __shared__ double smem[];  // S, X, Y: three 64 x 65 tiles
   double* S = smem;
   double* X = smem + TB * LD;
@@ -547,35 +592,39 @@ __global__ __launch_bounds__(TNT) void k_lu_tiles(int n, double* __restrict__ A,
   const long r0 = (long)ti * TB, c0 = (long)tj * TB;
   const int nr = min(TB, n - (int)r0), nc = min(TB, n - (int)c0);
   const int d = min(ti, tj);
-  const Quad q;
-  d4 acc[4][4];
-  acc_load(acc, q, A, lda, r0, c0, nr, nc);
+  const Quad4 q;
+  d4 acc[4];
+  acc_load4(acc, q, A, lda, r0, c0, nr, nc);
   for (int k = 0; k < d; k++) {
     if (!wait_flag(&done[lu_index(ti, k, nb)], error, sh)) return;
     if (!wait_flag(&done[lu_index(k, tj, nb)], error, sh)) return;
     const int kc = min(TB, n - k * TB);
-    tile_to_lds(X, A, lda, r0, (long)k * TB, nr, kc);  // L(i, k)
-    tile_to_lds(Y, A, lda, (long)k * TB, c0, kc, nc);  // U(k, j)
+    tile_to_lds4(X, A, lda, r0, (long)k * TB, nr, kc);  // L(i, k)
+    tile_to_lds4(Y, A, lda, (long)k * TB, c0, kc, nc);  // U(k, j)
     __syncthreads();
-    acc_update<false>(acc, q, X, Y);
+    acc_update4_nn(acc, q, X, Y);
     __syncthreads();
   }
-  acc_to_lds(acc, q, S);
+  acc_to_lds4(acc, q, S);
   __syncthreads();
   if (ti == tj) {
-    pad_identity(S, nr);
+    pad_identity4(S, nr);
     __syncthreads();
-    getf2_reg(S, X, nr, sgn + r0, square_last && ti == nb - 1);
+    if (threadIdx.x < TB) getf2_loop(S, nr, sgn + r0, square_last && ti == nb - 1);
     __syncthreads();
-    lds_to_tile(S, A, lda, r0, c0, nr, nc, false);
+    lds_to_tile4(S, A, lda, r0, c0, nr, nc, false);
   } else {
     if (!wait_flag(&done[lu_index(d, d, nb)], error, sh)) return;
     const long dd = (long)d * TB;
     const int kd = min(TB, n - (int)dd);
-    if (ti > tj) tile_solve<1>(S, X, A + dd * lda + dd, lda, kd);  // L(i, j) = A(i, j) U(j, j)^-1
-    else tile_solve<2>(S, X, A + dd * lda + dd, lda, kd);          // U(i, j) = L(i, i)^-1 A(i, j)
+    tile_to_lds4(X, A + dd * lda + dd, lda, 0, 0, kd, kd);  // the diagonal tile
     __syncthreads();
-    lds_to_tile(S, A, lda, r0, c0, nr, nc, false);
+    if (threadIdx.x < TB) {
+      if (ti > tj) tile_solve<1>(S, X, nullptr, 0, kd);  // L(i, j) = A(i, j) U(j, j)^-1
+      else tile_solve<2>(S, X, nullptr, 0, kd);          // U(i, j) = L(i, i)^-1 A(i, j)
+    }
+    __syncthreads();
+    lds_to_tile4(S, A, lda, r0, c0, nr, nc, false);
   }
   signal_flag(&done[blockIdx.x]);
 }
@@ -723,7 +772,7 @@ int lu_tiles(int n, double* A, long lda, double* sgn, int square_last, void* wor
     attr = true;
   }
   hipLaunchKernelGGL(k_zero_ints, dim3(exc_detail::ceil_div(nb * nb + 8, 256)), dim3(256), 0, s, done, nb * nb + 8);
-  hipLaunchKernelGGL(k_lu_tiles, dim3(T), dim3(TNT), kTileLds, s, n, A, lda, nb, sgn, square_last, done, err);
+  hipLaunchKernelGGL(k_lu_tiles, dim3(T), dim3(TNT4), kTileLds, s, n, A, lda, nb, sgn, square_last, done, err);
   EXC_CHECK_HIP(hipGetLastError());
   int herr = 0;
   EXC_CHECK_HIP(hipMemcpyAsync(&herr, err, sizeof herr, hipMemcpyDeviceToHost, s));
