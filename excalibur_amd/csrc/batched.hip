@@ -172,6 +172,7 @@ size_t exc_batched_local_qr_workspace(int nb, int m, const long* h_cols) {
     probs[b].N = h_cols[b];
     probs[b].K = m;
     probs[b].lower_only = probs[b].mirror = 0;
+    probs[b].tri = EXC_TRI_A_LOWER;
   }
   g = std::max(g, exc_gemm_grouped_workspace(8, nb, probs.data(), -1));
   a.take<char>(g);

@@ -15,6 +15,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "exc_common.hpp"
@@ -528,16 +529,19 @@ struct GroupRed {
   int p, tile_m, tile_n, first_slot, nslots, pad;
 };
 
-template <typename T>
-using GroupShape = typename Shapes<T>::Big;
-constexpr int kGroupBM = 128, kGroupBN = 128;
+// 64 x 64 tiles where an operand is triangular (they skip more of its zeros, and the large tile's
+// registers do not hold the triangle's code: 32 products L^-1 X of order 512 took 7.1 ms with it,
+// 6.9 with the small one), 128 x 128 elsewhere.
+template <typename T, bool TRI>
+using GroupShape = std::conditional_t<TRI, typename Shapes<T>::Small, typename Shapes<T>::Big>;
 
 template <typename T, int TA, int TB, bool TRI>
-__global__ __launch_bounds__(GroupShape<T>::kThreads, GroupShape<T>::kPerCu * GroupShape<T>::kThreads / 256) void k_gemm_grouped(
+__global__ __launch_bounds__((GroupShape<T, TRI>::kThreads), (GroupShape<T, TRI>::kPerCu * GroupShape<T, TRI>::kThreads / 256)) void k_gemm_grouped(
     const GroupProb* __restrict__ probs, const GroupItem* __restrict__ items, long nitems, T* __restrict__ part,
     double alpha, double beta) {
-  constexpr int BM = kGroupBM, BN = kGroupBN;
-  __shared__ Tiles<GroupShape<T>> lds;
+  using S = GroupShape<T, TRI>;
+  constexpr int BM = S::BM, BN = S::BN;
+  __shared__ Tiles<S> lds;
   // each die takes a contiguous range of the items, as in tile_of
   const long L = blockIdx.x, q = nitems / kXcds, r = nitems % kXcds;
   const GroupItem w = items[(L % kXcds) * q + min(L % kXcds, r) + L / kXcds];
@@ -556,8 +560,8 @@ __global__ __launch_bounds__(GroupShape<T>::kThreads, GroupShape<T>::kPerCu * Gr
       k0 = max(k0, w.k0);
       k1 = min(k1, w.k1);
     }
-    gemm_tile<T, TA, TB, TRI, GroupShape<T>>(g, i0, j0, k0, k1, Cb, direct ? pr.ldc : BN, direct ? 0 : i0,
-                                             direct ? 0 : j0, direct, lds);
+    gemm_tile<T, TA, TB, TRI, S>(g, i0, j0, k0, k1, Cb, direct ? pr.ldc : BN, direct ? 0 : i0, direct ? 0 : j0,
+                                 direct, lds);
     if (!TRI || w.other_m < 0 || tile_m == w.other_m) break;
     tile_m = w.other_m;
     lds_barrier();  // the next tile restages the slabs
@@ -567,18 +571,18 @@ __global__ __launch_bounds__(GroupShape<T>::kThreads, GroupShape<T>::kPerCu * Gr
 template <typename T>
 __global__ __launch_bounds__(256) void k_grouped_reduce(const GroupProb* __restrict__ probs,
                                                         const GroupRed* __restrict__ reds, const T* __restrict__ part,
-                                                        double alpha, double beta) {
+                                                        int tile, double alpha, double beta) {
   const GroupRed r = reds[blockIdx.x];
   const GroupProb pr = probs[r.p];
   T* C = (T*)pr.C;
-  for (int e = threadIdx.x; e < kGroupBM * kGroupBN; e += blockDim.x) {
-    const int li = e / kGroupBN, lj = e - li * kGroupBN;
-    const long gi = (long)r.tile_m * kGroupBM + li, gj = (long)r.tile_n * kGroupBN + lj;
+  for (int e = threadIdx.x; e < tile * tile; e += blockDim.x) {
+    const int li = e / tile, lj = e - li * tile;
+    const long gi = (long)r.tile_m * tile + li, gj = (long)r.tile_n * tile + lj;
     if (gi >= pr.M || gj >= pr.N) continue;
     if (pr.lower_only && gj > gi) continue;  // the upper part of a diagonal tile comes by mirroring
     T s = T(0);
 #pragma unroll 4
-    for (int q = 0; q < r.nslots; q++) s += part[(size_t)(r.first_slot + q) * kGroupBM * kGroupBN + e];
+    for (int q = 0; q < r.nslots; q++) s += part[(size_t)(r.first_slot + q) * tile * tile + e];
     T out = (T)alpha * s;
     if (beta != 0.0) out += (T)beta * C[gi * pr.ldc + gj];
     C[gi * pr.ldc + gj] = out;
@@ -741,13 +745,18 @@ struct GroupPlan {
   std::vector<GroupItem> items;
   std::vector<GroupRed> reds;
   long slots = 0;
+  int tile = 128;
+  bool tri = false;  // any triangular problem: the kernel for both, with its tile
   double flops = 0.0;
 };
 
 GroupPlan group_plan(int nprob, const ExcGemmProblem* P, long kchunk) {
-  constexpr int BM = kGroupBM, BN = kGroupBN, BK = Shapes<double>::Big::BK;
+  constexpr int BK = Shapes<double>::Big::BK;
   static_assert(BK == Shapes<float>::Big::BK, "one chunk length for both types");
   GroupPlan g;
+  g.tri = std::any_of(P, P + nprob, [](const ExcGemmProblem& q) { return q.tri != EXC_TRI_NONE; });
+  g.tile = g.tri ? GroupShape<double, true>::BM : GroupShape<double, false>::BM;
+  const int BM = g.tile, BN = g.tile;
   if (kchunk > 0) kchunk = ((kchunk + BK - 1) / BK) * BK;
   for (int p = 0; p < nprob; p++) {
     const ExcGemmProblem& q = P[p];
@@ -783,7 +792,7 @@ GroupPlan group_plan(int nprob, const ExcGemmProblem* P, long kchunk) {
 size_t group_bytes(const GroupPlan& g, size_t tsize) {
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   return up(g.probs.size() * sizeof(GroupProb)) + up(g.items.size() * sizeof(GroupItem)) +
-         up(std::max<size_t>(1, g.reds.size()) * sizeof(GroupRed)) + (size_t)g.slots * kGroupBM * kGroupBN * tsize;
+         up(std::max<size_t>(1, g.reds.size()) * sizeof(GroupRed)) + (size_t)g.slots * g.tile * g.tile * tsize;
 }
 
 template <typename T>
@@ -808,19 +817,18 @@ int group_run(int ta, int tb, const GroupPlan& g, double alpha, double beta, voi
   EXC_CHECK_HIP(hipStreamSynchronize(s));
   const long nitems = (long)g.items.size();
   EXC_REQUIRE(nitems < (1L << 31), EXC_ERR_ARG, "exc_gemm_grouped: too many tiles");
-  const dim3 grid((unsigned)nitems), block(GroupShape<T>::kThreads);
+  const dim3 grid((unsigned)nitems), block(g.tri ? GroupShape<T, true>::kThreads : GroupShape<T, false>::kThreads);
   hipEvent_t e0 = exc_prof::mark(s);
-  // one transposition pattern per call; a set with any triangular problem takes the kernel for both
   auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, dp, di, nitems, part, alpha, beta); };
-  const bool tri = std::any_of(g.probs.begin(), g.probs.end(), [](const GroupProb& p) { return p.tri != EXC_TRI_NONE; });
+  const bool tri = g.tri;
   if (!ta && !tb) tri ? launch(k_gemm_grouped<T, 0, 0, true>) : launch(k_gemm_grouped<T, 0, 0, false>);
   else if (!ta && tb) tri ? launch(k_gemm_grouped<T, 0, 1, true>) : launch(k_gemm_grouped<T, 0, 1, false>);
   else if (ta && !tb) tri ? launch(k_gemm_grouped<T, 1, 0, true>) : launch(k_gemm_grouped<T, 1, 0, false>);
   else tri ? launch(k_gemm_grouped<T, 1, 1, true>) : launch(k_gemm_grouped<T, 1, 1, false>);
   EXC_CHECK_HIP(hipGetLastError());
   if (!g.reds.empty()) {
-    hipLaunchKernelGGL(k_grouped_reduce<T>, dim3((unsigned)g.reds.size()), dim3(256), 0, s, dp, dr, part, alpha,
-                       beta);
+    hipLaunchKernelGGL(k_grouped_reduce<T>, dim3((unsigned)g.reds.size()), dim3(256), 0, s, dp, dr, part, g.tile,
+                       alpha, beta);
     EXC_CHECK_HIP(hipGetLastError());
   }
   if (e0) exc_prof::book(sizeof(T) == 8 ? "gemm_grouped_f64" : "gemm_grouped_f32", e0, exc_prof::mark(s), g.flops, 0.0);
