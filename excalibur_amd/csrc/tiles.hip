@@ -177,110 +177,119 @@ __device__ inline void wave_sync() {
 // The routine runs once per diagonal tile on one wavefront, so every instruction is fetched cold:
 // a fully unrolled form (tens of KB of straight-line code) was bound by instruction fetch, not
 // arithmetic. So only a panel of PW columns is unrolled (inside it the pivot and the multipliers
-// L[k][j] reach the other lanes by v_readlane, no LDS, no barrier); the panel loop is not, and the
-// panel's rank-PW update of the later columns runs as a loop over blocks of 8 columns with eight
-// independent chains, the panel's multipliers read back from LDS (xc).
+// L[k][j] reach the other lanes by v_readlane, no LDS, no barrier); the panel loop is not. The
+// panels run on wavefront 0; the panel's rank-PW update of the later columns runs as a loop over
+// blocks of 8 columns with eight independent chains, the blocks dealt to the four wavefronts and the
+// panel's multipliers read back from LDS (xc). All 256 threads call it.
 constexpr int PW = 8;
 __device__ __forceinline__ int potf2_loop(double* S, double* xc, int kb) {
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __asm__ volatile("" ::: "memory");
   int bad = 0;
 #pragma unroll 1
   for (int j0 = 0; j0 < TB; j0 += PW) {
-    double x[PW], lown[PW];
+    if (wave == 0) {
+      double x[PW];
 #pragma unroll
-    for (int jj = 0; jj < PW; jj++) x[jj] = S[lane * LD + j0 + jj];
+      for (int jj = 0; jj < PW; jj++) x[jj] = S[lane * LD + j0 + jj];
 #pragma unroll
-    for (int jj = 0; jj < PW; jj++) {
-      const int j = j0 + jj;
-      double d = readlane_f64(x[jj], j);
-      if (!(d > 0.0)) {
-        if (!bad && j < kb) bad = j + 1;
-        d = 1.0;
+      for (int jj = 0; jj < PW; jj++) {
+        const int j = j0 + jj;
+        double d = readlane_f64(x[jj], j);
+        if (!(d > 0.0)) {
+          if (!bad && j < kb) bad = j + 1;
+          d = 1.0;
+        }
+        double rp, piv;
+        rsqrt_pair(d, &rp, &piv);
+        const double l = lane > j ? x[jj] * rp : 0.0;
+        x[jj] = lane == j ? piv : (lane > j ? l : x[jj]);
+        xc[lane * (PW + 1) + jj] = l;
+#pragma unroll
+        for (int kk = jj + 1; kk < PW; kk++) x[kk] = fma(-l, readlane_f64(l, j0 + kk), x[kk]);
       }
-      double rp, piv;
-      rsqrt_pair(d, &rp, &piv);
-      const double l = lane > j ? x[jj] * rp : 0.0;
-      x[jj] = lane == j ? piv : (lane > j ? l : x[jj]);
-      lown[jj] = l;
 #pragma unroll
-      for (int kk = jj + 1; kk < PW; kk++) x[kk] = fma(-l, readlane_f64(l, j0 + kk), x[kk]);
+      for (int jj = 0; jj < PW; jj++) S[lane * LD + j0 + jj] = x[jj];
     }
+    lds_barrier();
+    double l[PW];
 #pragma unroll
-    for (int jj = 0; jj < PW; jj++) {
-      S[lane * LD + j0 + jj] = x[jj];
-      xc[lane * (PW + 1) + jj] = lown[jj];
-    }
-    wave_sync();
+    for (int jj = 0; jj < PW; jj++) l[jj] = xc[lane * (PW + 1) + jj];
 #pragma unroll 1
-    for (int k0 = j0 + PW; k0 < TB; k0 += 8) {
+    for (int k0 = j0 + PW + 8 * wave; k0 < TB; k0 += 32) {
       double a[8];
 #pragma unroll
       for (int kk = 0; kk < 8; kk++) a[kk] = S[lane * LD + k0 + kk];
 #pragma unroll
       for (int jj = 0; jj < PW; jj++)
 #pragma unroll
-        for (int kk = 0; kk < 8; kk++) a[kk] = fma(-lown[jj], xc[(k0 + kk) * (PW + 1) + jj], a[kk]);
+        for (int kk = 0; kk < 8; kk++) a[kk] = fma(-l[jj], xc[(k0 + kk) * (PW + 1) + jj], a[kk]);
 #pragma unroll
       for (int kk = 0; kk < 8; kk++) S[lane * LD + k0 + kk] = a[kk];
     }
-    wave_sync();
+    lds_barrier();
   }
 #pragma unroll 1
-  for (int k = lane + 1; k < TB; k++) S[lane * LD + k] = 0.0;
+  for (int k = lane + 1 + wave; k < TB; k += 4) S[lane * LD + k] = 0.0;
   return bad;
 }
 
 // LU without pivoting of S - diag(s) (sign rule of the Householder reconstruction), lane i = row i.
 // sgn receives s for the kb valid pivots. As in potf2_loop only a panel of PW columns is unrolled:
 // inside it row j reaches the other lanes by v_readlane; then the panel's PW rows of U are finished
-// for the later columns and every lane takes the panel's rank-PW update of its row, blocks of 8
-// columns at a time in a loop, with U read from LDS. Every element receives the same fused
-// multiply-adds in the same order as a column-by-column right-looking factorization. (Fully unrolled
-// the routine was bound by instruction fetch, as potf2_loop's comment says.)
+// for the later columns (both on wavefront 0) and every lane takes the panel's rank-PW update of its
+// row, blocks of 8 columns dealt to the four wavefronts, with U read from LDS. Every element receives
+// the same fused multiply-adds in the same order as a column-by-column right-looking
+// factorization. (Fully unrolled the routine was bound by instruction fetch, as potf2_loop's comment
+// says.) All 256 threads call it.
 __device__ __forceinline__ void getf2_loop(double* S, int kb, double* sgn, bool last_plus) {
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __asm__ volatile("" ::: "memory");
 #pragma unroll 1
   for (int j0 = 0; j0 < TB; j0 += PW) {
-    double x[PW], l[PW];
+    if (wave == 0) {
+      double x[PW];
 #pragma unroll
-    for (int jj = 0; jj < PW; jj++) x[jj] = S[lane * LD + j0 + jj];
+      for (int jj = 0; jj < PW; jj++) x[jj] = S[lane * LD + j0 + jj];
 #pragma unroll
-    for (int jj = 0; jj < PW; jj++) {
-      const int j = j0 + jj;
-      const double w = readlane_f64(x[jj], j);
-      double sj = signbit(w) ? 1.0 : -1.0;
-      if (last_plus && j == kb - 1) sj = -sj;
-      const double piv = w - sj;
-      if (lane == 0 && j < kb) sgn[j] = sj;
-      const double rp = 1.0 / piv;
-      l[jj] = lane > j ? x[jj] * rp : 0.0;
-      x[jj] = lane == j ? piv : (lane > j ? l[jj] : x[jj]);
+      for (int jj = 0; jj < PW; jj++) {
+        const int j = j0 + jj;
+        const double w = readlane_f64(x[jj], j);
+        double sj = signbit(w) ? 1.0 : -1.0;
+        if (last_plus && j == kb - 1) sj = -sj;
+        const double piv = w - sj;
+        if (lane == 0 && j < kb) sgn[j] = sj;
+        const double rp = 1.0 / piv;
+        const double l = lane > j ? x[jj] * rp : 0.0;
+        x[jj] = lane == j ? piv : (lane > j ? l : x[jj]);
 #pragma unroll
-      for (int kk = jj + 1; kk < PW; kk++) x[kk] = fma(-l[jj], readlane_f64(x[kk], j), x[kk]);
+        for (int kk = jj + 1; kk < PW; kk++) x[kk] = fma(-l, readlane_f64(x[kk], j), x[kk]);
+      }
+#pragma unroll
+      for (int jj = 0; jj < PW; jj++) S[lane * LD + j0 + jj] = x[jj];
+      wave_sync();
+      // the later columns' rows of U: lane = column
+      const int c = lane;
+      if (c >= j0 + PW) {
+        double u[PW];
+#pragma unroll
+        for (int jj = 0; jj < PW; jj++) u[jj] = S[(j0 + jj) * LD + c];
+#pragma unroll
+        for (int jj = 0; jj < PW; jj++)
+#pragma unroll
+          for (int kk = jj + 1; kk < PW; kk++) u[kk] = fma(-S[(j0 + kk) * LD + j0 + jj], u[jj], u[kk]);
+#pragma unroll
+        for (int jj = 0; jj < PW; jj++) S[(j0 + jj) * LD + c] = u[jj];
+      }
     }
-#pragma unroll
-    for (int jj = 0; jj < PW; jj++) S[lane * LD + j0 + jj] = x[jj];
-    wave_sync();
-    // the later columns: lane = column c first finishes the panel's rows of U there ...
-    const int c = lane;
-    if (c >= j0 + PW) {
-      double u[PW];
-#pragma unroll
-      for (int jj = 0; jj < PW; jj++) u[jj] = S[(j0 + jj) * LD + c];
-#pragma unroll
-      for (int jj = 0; jj < PW; jj++)
-#pragma unroll
-        for (int kk = jj + 1; kk < PW; kk++) u[kk] = fma(-S[(j0 + kk) * LD + j0 + jj], u[jj], u[kk]);
-#pragma unroll
-      for (int jj = 0; jj < PW; jj++) S[(j0 + jj) * LD + c] = u[jj];
-    }
-    wave_sync();
-    // ... then lane = row updates its row
+    lds_barrier();
+    // the later rows: lane = row
     const bool below = lane >= j0 + PW;
+    double l[PW];
+#pragma unroll
+    for (int jj = 0; jj < PW; jj++) l[jj] = S[lane * LD + j0 + jj];
 #pragma unroll 1
-    for (int k0 = j0 + PW; k0 < TB; k0 += 8) {
+    for (int k0 = j0 + PW + 8 * wave; k0 < TB; k0 += 32) {
       double a[8];
 #pragma unroll
       for (int kk = 0; kk < 8; kk++) a[kk] = S[lane * LD + k0 + kk];
@@ -293,7 +302,7 @@ __device__ __forceinline__ void getf2_loop(double* S, int kb, double* sgn, bool 
         for (int kk = 0; kk < 8; kk++) S[lane * LD + k0 + kk] = a[kk];
       }
     }
-    wave_sync();
+    lds_barrier();
   }
 }
 
@@ -467,10 +476,8 @@ __device__ __forceinline__ void potrf_tile_run(int n, double* __restrict__ A, lo
   if (ti == tj) {
     pad_identity4(S, nr);
     __syncthreads();
-    if (threadIdx.x < TB) {
-      const int bad = potf2_loop(S, X, nr);
-      if (threadIdx.x == 0 && bad) atomicCAS(&error[1], 0, (int)r0 + bad);
-    }
+    const int bad = potf2_loop(S, X, nr);
+    if (threadIdx.x == 0 && bad) atomicCAS(&error[1], 0, (int)r0 + bad);
     __syncthreads();
     lds_to_tile4(S, A, lda, r0, c0, nr, nc, true);
   } else {
@@ -578,7 +585,7 @@ __device__ __forceinline__ void acc_update4_nn(d4 (&acc)[4], const Quad4& q, con
 
 // Four wavefronts per tile, as in the Cholesky: updates, staging and stores split four ways, the
 // factorization and the solve on wavefront 0. Order 1000: 1.52 ms with one wavefront and the
-// unrolled factorization, 0.97 ms now.
+// unrolled factorization, 0.87 ms now.
 __global__ __launch_bounds__(TNT4) void k_lu_tiles(int n, double* __restrict__ A, long lda, int nb,
                                                    double* __restrict__ sgn, int square_last,
                                                    int* __restrict__ done, int* __restrict__ error) {
@@ -610,7 +617,7 @@ __global__ __launch_bounds__(TNT4) void k_lu_tiles(int n, double* __restrict__ A
   if (ti == tj) {
     pad_identity4(S, nr);
     __syncthreads();
-    if (threadIdx.x < TB) getf2_loop(S, nr, sgn + r0, square_last && ti == nb - 1);
+    getf2_loop(S, nr, sgn + r0, square_last && ti == nb - 1);
     __syncthreads();
     lds_to_tile4(S, A, lda, r0, c0, nr, nc, false);
   } else {
