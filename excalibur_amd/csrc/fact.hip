@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void k_trsm_left_blk(int kb, const double* __r
 // coefficient, the solved unknowns broadcast from LDS), then solve the second block. Each wave
 // keeps its 128 x C right-hand sides in LDS for the whole launch.
 template <bool UPPER, bool UNIT, int C>
-__global__ __launch_bounds__(256) void k_trsm_left_blk2(int kb, const double* __restrict__ L, long ldl,
+__global__ __launch_bounds__(256, 2) void k_trsm_left_blk2(int kb, const double* __restrict__ L, long ldl,
                                                         double* __restrict__ X, long ldx, long nrhs) {
   constexpr int SL = NB + 2, S = C + 2, RPI = 64 / C;
   __shared__ __attribute__((aligned(16))) double Ls[NB * SL];
@@ -201,17 +201,32 @@ __global__ __launch_bounds__(256) void k_trsm_left_blk2(int kb, const double* __
   // rows [b0, b0 + bn) of the first and second blocks
   const int f0 = UPPER ? NB : 0, fn = UPPER ? kb - NB : NB;
   const int s0 = UPPER ? 0 : NB, sn = UPPER ? NB : kb - NB;
-  // Ls <- the bn x bn diagonal triangle at (b0, b0); lanes read their scaled row into lr
-  auto stage = [&](int r0, int rn, int q0, int qn) {
+  // A rn x qn block of L at (r0, q0), through registers into Ls. The loads are unconditional (clamped):
+  // behind a condition each waited for itself, and the three blocks of a narrow launch took most of
+  // its 27 us (20 now). AHEAD: they are issued while the block before is in use; with 8 columns per
+  // wavefront their registers would cost the second workgroup of a CU (50,000 right-hand sides: 205
+  // us with it, 130 without).
+  constexpr bool AHEAD = C <= 4;
+  double blk[NB / 4];
+  auto fetch = [&](int r0, int rn, int q0, int qn) __attribute__((always_inline)) {
     const int lc = lane < qn ? lane : qn - 1;
 #pragma unroll
-    for (int r = wave; r < NB; r += 4)
-      Ls[r * SL + lane] = (r < rn && lane < qn) ? L[(long)(r0 + (r < rn ? r : rn - 1)) * ldl + q0 + lc] : 0.0;
+    for (int z = 0; z < NB / 4; z++) {
+      const int r = wave + 4 * z;
+      blk[z] = L[(long)(r0 + (r < rn ? r : rn - 1)) * ldl + q0 + lc];
+    }
   };
-  auto solve = [&](int b0, int bn, double (&y)[C]) {
+  auto put = [&](int rn, int qn) __attribute__((always_inline)) {
     __syncthreads();  // earlier readers of Ls are done
-    stage(b0, bn, b0, bn);
+#pragma unroll
+    for (int z = 0; z < NB / 4; z++) {
+      const int r = wave + 4 * z;
+      Ls[r * SL + lane] = (r < rn && lane < qn) ? blk[z] : 0.0;
+    }
     __syncthreads();
+  };
+  // the diagonal triangle at (b0, b0) is in Ls; lanes read their scaled row into lr
+  auto solve = [&](int b0, int bn, double (&y)[C]) {
     const bool live = lane < bn;
     const int row = live ? lane : bn - 1;
     const double rinv = UNIT ? 1.0 : 1.0 / Ls[row * SL + row];
@@ -233,15 +248,17 @@ __global__ __launch_bounds__(256) void k_trsm_left_blk2(int kb, const double* __
 #pragma unroll
     for (int c = 0; c < C; c++) Xs[(b0 + lane) * S + c] = y[c];
   };
-  __syncthreads();
+  fetch(f0, fn, f0, fn);
+  put(fn, fn);
+  if (AHEAD) fetch(s0, sn, f0, fn);
   double y[C];
 #pragma unroll
   for (int c = 0; c < C; c++) y[c] = Xs[(f0 + lane) * S + c];
   solve(f0, fn, y);
   // second block: y -= O x_first, O = rows [s0, s0 + sn) x columns [f0, f0 + fn) of the triangle
-  __syncthreads();
-  stage(s0, sn, f0, fn);
-  __syncthreads();
+  if (!AHEAD) fetch(s0, sn, f0, fn);
+  put(sn, fn);
+  if (AHEAD) fetch(s0, sn, s0, sn);
   {
     double o[NB];
 #pragma unroll
@@ -254,6 +271,8 @@ __global__ __launch_bounds__(256) void k_trsm_left_blk2(int kb, const double* __
       for (int c = 0; c < C; c++) y[c] = fma(-o[k], Xs[(f0 + k) * S + c], y[c]);
     }
   }
+  if (!AHEAD) fetch(s0, sn, s0, sn);
+  put(sn, sn);
   solve(s0, sn, y);
   __syncthreads();
 #pragma unroll
