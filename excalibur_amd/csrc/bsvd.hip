@@ -374,7 +374,7 @@ struct Twist {
   double* best;               // [2][chunks][k]: least |gamma| of a chunk (v, u), then largest |v|
   int* at;                    // [2][chunks][k]: its index
   int* twist;                 // [2][k]
-  double* inv;                // [2][k]: 1 / norm
+  double* inv[2];             // [k]: 1 / norm (v, u)
   int chunks;
 };
 
@@ -582,7 +582,7 @@ __global__ __launch_bounds__(256, 1) void k_twist_chain(Twist T) {
 #pragma unroll
     for (int q = 0; q < kDeep; q++) cur[q] = nxt[q];
   }
-  if (active) T.inv[side * T.k + j] = 1.0 / sqrt(ss);
+  if (active) T.inv[side][j] = 1.0 / sqrt(ss);
 }
 
 // Scaling to unit length, v on wavefront 0 (with each chunk's largest |v_i| and its first index, for
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(128) void k_twist_scale(Twist T) {
   if (j >= T.k) return;
   const size_t K = (size_t)T.k;
   double* vec = (side == 0 ? T.vs : T.u) + j;
-  const double inv = T.inv[side * T.k + j];
+  const double inv = T.inv[side][j];
   double best = -1.0, row[kRows];
   int at = 0;
 #pragma unroll
@@ -723,7 +723,7 @@ struct BisectWs {
   ShareWs share;  // in the replay's frontiers, which are not in use at the same time
 };
 
-size_t bisect_ws_bytes(int n, void* base, BisectWs* ws, Bump* bump) {
+size_t bisect_ws_bytes(int n, void* base, BisectWs* ws, Bump* bump, bool own_table = true) {
   Bump& B = *bump;
   BisectWs w;
   w.hdr = B.take<BisectHdr>(1);
@@ -741,7 +741,7 @@ size_t bisect_ws_bytes(int n, void* base, BisectWs* ws, Bump* bump) {
   w.L_lo = B.take<double>(w.cap);
   w.L_hi = B.take<double>(w.cap);
   w.share = ShareWs{w.f_lo[0], w.f_hi[0], w.f_lo[1], w.f_hi[1], w.f_clo[1], w.f_chi[1], w.f_clo[0], w.ctr,
-                    B.take<int>(kShareLanes)};
+                    own_table ? B.take<int>(kShareLanes) : nullptr};
   if (ws) *ws = w;
   (void)base;
   return B.used;
@@ -935,9 +935,12 @@ int exc_ldl(int n, const double* d_alpha, const double* d_beta, double* d_l, dou
 
 namespace {
 struct TwistWs {
-  double *l, *d, *S, *P, *DP, *RP, *vs, *sgn, *best, *inv;
-  int *at, *twist;
+  double *l, *d, *S, *P, *DP, *RP, *vs, *sgn, *best;
 };
+// Chunk results of the search for the twists: 2 x chunks x k doubles and as many ints.
+size_t twist_best_doubles(int n, int k) { return 3 * (((size_t)n + kRows - 1) / kRows) * k; }
+// The shared levels' table fits in the sequences, which are not in use before the bisection ends.
+bool table_in_sequences(int n, int k) { return 4 * ((size_t)n + 1) * k * sizeof(double) >= kShareLanes * sizeof(int); }
 void twist_ws(int n, int k, Bump& B, TwistWs* w) {
   w->l = B.take<double>(n);
   w->d = B.take<double>(n);
@@ -947,11 +950,8 @@ void twist_ws(int n, int k, Bump& B, TwistWs* w) {
   w->RP = B.take<double>((size_t)(n + 1) * k);
   w->vs = B.take<double>((size_t)n * k);
   w->sgn = B.take<double>(k);
-  const size_t chunks = ((size_t)n + kRows - 1) / kRows;
-  w->best = B.take<double>(2 * chunks * k);
-  w->at = B.take<int>(2 * chunks * k);
-  w->twist = B.take<int>(2 * (size_t)k);
-  w->inv = B.take<double>(2 * (size_t)k);
+  // the chunk results live in v's place until the multipliers are written there (n >= 3 has room)
+  w->best = (size_t)n * k >= twist_best_doubles(n, k) ? w->vs : B.take<double>(twist_best_doubles(n, k));
 }
 
 int run_twisted(int n, int k, const double* omega, const double* a, const double* b, double* u, double* v,
@@ -962,13 +962,19 @@ int run_twisted(int n, int k, const double* omega, const double* a, const double
     EXC_CHECK_HIP(hipGetLastError());
   }
   const int chunks = (n + kRows - 1) / kRows;
-  const Twist T{n, k, a, b, w.l, w.d, omega, u, w.vs, w.S, w.P, w.DP, w.RP, w.best, w.at, w.twist, w.inv, chunks};
+  // row n of each sequence is not stored: the twists and the norms go there
+  const size_t end = (size_t)n * k;
+  Twist T{n, k, a, b, w.l, w.d, omega, u, w.vs, w.S, w.P, w.DP, w.RP, w.best, (int*)(w.best + 2 * (size_t)chunks * k),
+          (int*)(w.S + end), {w.P + end, w.DP + end}, chunks};
   const unsigned groups = exc_detail::ceil_div(k, 64);
   hipLaunchKernelGGL(k_qds, dim3(groups), dim3(128), 0, s, T);
   hipLaunchKernelGGL(k_twist_min, dim3(groups, chunks), dim3(128), 0, s, T);
   hipLaunchKernelGGL(k_twist_pick, dim3(exc_detail::ceil_div(2L * k, 256)), dim3(256), 0, s, T, twists);
   hipLaunchKernelGGL(k_twist_mult, dim3(groups, chunks), dim3(256), 0, s, T);
   hipLaunchKernelGGL(k_twist_chain, dim3(groups), dim3(256), 0, s, T);
+  // the sequences are done with: the scaling's chunk results go over s
+  T.best = w.S;
+  T.at = (int*)(w.S + (size_t)chunks * k);
   hipLaunchKernelGGL(k_twist_scale, dim3(groups, chunks), dim3(128), 0, s, T);
   EXC_CHECK_HIP(hipGetLastError());
   if (apply_vsign) {
@@ -1005,7 +1011,7 @@ int exc_twisted_vectors(int n, int k, const double* d_omega, const double* d_alp
 
 size_t exc_bidiag_svd_workspace(int k, int top_k) {
   Bump B(nullptr, 0);
-  bisect_ws_bytes(k, nullptr, nullptr, &B);
+  bisect_ws_bytes(k, nullptr, nullptr, &B, !table_in_sequences(k, top_k));
   B.take<int>(1);
   TwistWs w;
   twist_ws(k, top_k, B, &w);
@@ -1019,10 +1025,11 @@ int exc_bidiag_svd(int k, const double* d_alpha, const double* d_beta, double* d
               EXC_ERR_ARG, "exc_bidiag_svd: bad arguments");
   Bump B(d_work, work_bytes);
   BisectWs bw;
-  bisect_ws_bytes(k, d_work, &bw, &B);
+  bisect_ws_bytes(k, d_work, &bw, &B, !table_in_sequences(k, top_k));
   int* dcount = B.take<int>(1);
   TwistWs tw;
   twist_ws(k, top_k, B, &tw);
+  if (!bw.share.table) bw.share.table = (int*)tw.S;
   EXC_REQUIRE(B.ok(), EXC_ERR_SPACE, "exc_bidiag_svd: workspace too small");
   hipStream_t s = exc_detail::stream(stream);
   hipLaunchKernelGGL(k_frob_bound, dim3(1), dim3(256), 0, s, k, d_alpha, d_beta, bw.hdr);
