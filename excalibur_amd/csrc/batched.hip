@@ -4,7 +4,7 @@
 // Every block X_b (m x r_b row-major, r_b > 5 m so that the reference reduces it by a local QR)
 // gets R_b^T (m x m, lower) from a CholeskyQR whose bulk pass runs in FP32 on the MFMA:
 //   pass 1 (FP32): G_b = X_b X_b^T for all blocks in one grouped launch (the autotuner picks the K
-//     chunk and the persistent grid), L1_b = chol(G_b + s_b I) with s_b = u32 trace(G_b), doubled
+//     chunk), L1_b = chol(G_b + s_b I) with s_b = u32 trace(G_b), doubled
 //     until the factor exists;
 //   pass 2 (FP64): Z_b = L1_b^-1 X_b (one grouped launch, the inverses from one batched launch),
 //     G3_b = Z_b Z_b^T (one grouped launch), L3_b = chol(G3_b); a pass repeats for blocks whose

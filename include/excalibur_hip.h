@@ -371,8 +371,7 @@ int exc_givens_apply_batched(int nb, double* const* d_xs, long m, long n, const 
  * block X_b (m x cols[b] row-major FP64, cols[b] >= m; host array of device pointers h_x) R_b^T
  * (m x m lower, positive diagonal) into h_rt[b] and, when h_qt is given, Q_b^T (m x cols[b]) into
  * h_qt[b]. A shifted CholeskyQR whose first pass runs in FP32 on the MFMA (all blocks' Gram
- * matrices in one grouped persistent launch, its K chunk and grid chosen by the library's
- * autotuner), refined by FP64 passes (grouped launches); the m x m factorizations run one
+ * matrices in one grouped launch, its K chunk chosen by the library's autotuner), refined by FP64 passes (grouped launches); the m x m factorizations run one
  * workgroup per block in one launch. h_stats (nullable, 3 nb doubles): per block the FP32 shift,
  * max |Z Z^T - I| before the last FP64 pass and the number of FP64 passes. Synchronizes. No
  * counterpart in the reference, which runs one peer per process. */
