@@ -781,8 +781,11 @@ GroupPlan group_plan(int nprob, const ExcGemmProblem* P, long kchunk) {
           continue;
         }
         const long first = g.slots;
-        for (long k0 = 0; k0 < q.K || k0 == 0; k0 += chunk)
+        long k0 = 0;
+        do {  // an empty K too takes one item: its sum is zero
           g.items.push_back(GroupItem{p, (int)a, (int)b, (int)(g.slots++), -1, 0, k0, std::min(q.K, k0 + chunk)});
+          k0 += chunk;
+        } while (k0 < q.K);
         g.reds.push_back(GroupRed{p, (int)a, (int)b, (int)first, (int)(g.slots - first), 0});
       }
   }

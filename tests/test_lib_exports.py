@@ -153,3 +153,26 @@ def test_givens_restatement_matches_oracle(oracle, shape, is_left, mask):
     pairs, cs = hip.givens_plan(K, 32, mask, 99)
     want = oracle.givens_mask(x, 32, mask, is_left, 99)
     assert np.array_equal(givens_numpy(x, pairs, cs, mask, is_left, np.float64), want)
+
+
+def test_batched_workspace_of_an_empty_block(tmp_path):
+    """The workspace query of the batched local QR returns for blocks without columns too, and the call
+    itself refuses such a block before it touches the device. In a process of its own with a bound on
+    its memory: a query that never ends would take all of it."""
+    import subprocess
+    import sys
+    code = """
+import ctypes, resource
+resource.setrlimit(resource.RLIMIT_DATA, (6 << 30, 6 << 30))
+from excalibur_amd import hip
+for cols in ((600, 0), (0,), (0, 0, 700)):
+    n = len(cols)
+    c = (ctypes.c_long * n)(*cols)
+    p = (ctypes.c_void_p * n)(*([64] * n))
+    need = hip.lib.exc_batched_local_qr_workspace(n, 100, c)
+    rc = hip.lib.exc_batched_local_qr(n, 100, c, p, p, None, None, 64, 1 << 40, None)
+    print(cols, need, rc)
+    assert need > 0 and rc == -1
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, (r.stdout, r.stderr[-2000:])
