@@ -109,22 +109,24 @@ __global__ void k_bisect_init(int n, const double* __restrict__ a, const double*
 // largest value's scale: for order 1000 about 14 levels hold them all), and a group of lanes per
 // value would count the same nodes over and over. So the first steps give all lanes to the distinct
 // nodes: k_bisect_share evaluates the whole subtree of depth D below each of the N nodes, D =
-// log2(kShareLanes / N), and k_bisect_descend takes every value down it and lists the nodes they
+// log2(lanes / N), and k_bisect_descend takes every value down it and lists the nodes they
 // reach. Two such steps cover about 29 levels of order 1000 (two steps with 64 lanes per value: 12).
-// kShareLanes is one wavefront per SIMD: a step is bound by the issue of its FP64 instructions, about
-// 65 ns per row and wavefront, so more lanes would only queue.
+// kShareLanes, the most lanes, is one wavefront per SIMD: a step is bound by the issue of its FP64
+// instructions, about 65 ns per row and wavefront, so more would only queue. A step needs a word per
+// lane for its counts. They lie in scratch that is idle at the time, and where that holds fewer (in
+// the replay's 16,384 from order 256, 32,768 from 312, all from 934) a step takes fewer lanes.
 constexpr int kShareLanes = 65536;
 constexpr int kShareMinN = 256;       // below this a step is shorter than its two launches
 constexpr int kShareMaxTargets = 16384;
-__device__ __forceinline__ int share_depth(int nodes) { return nodes > 0 ? 31 - __clz(kShareLanes / nodes) : 0; }
-
 struct ShareWs {
   double *node_lo, *node_hi;  // distinct nodes
   double *lo, *hi;            // per value: its node, the counts at its ends, its index in the list
   int *clo, *chi, *node;
   int* nodes;                 // their number
-  int* table;                 // kShareLanes counts
+  int* table;                 // the counts, one per lane
+  int lanes;                  // a power of two, at least as many as there are values
 };
+__device__ __forceinline__ int share_depth(int lanes, int nodes) { return nodes > 0 ? 31 - __clz(lanes / nodes) : 0; }
 
 // first: the node is the root; the last workgroup counts its ends and fills the header.
 __global__ __launch_bounds__(256) void k_bisect_share(int n, const double* __restrict__ a,
@@ -148,7 +150,7 @@ __global__ __launch_bounds__(256) void k_bisect_share(int n, const double* __res
   }
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   const int nodes = first ? 1 : *w.nodes;
-  const int D = share_depth(nodes);
+  const int D = share_depth(w.lanes, nodes);
   const int node = g >> D, h = (g & ((1 << D) - 1)) + 1;
   if (node >= nodes || h == (1 << D)) return;
   double l = first ? hdr->lo : w.node_lo[node], r = first ? hdr->hi : w.node_hi[node];
@@ -168,7 +170,7 @@ __global__ __launch_bounds__(1024) void k_bisect_descend(BisectHdr* hdr, double 
   const int nclo = hdr->nclo, nchi = hdr->nchi;
   int T = (nclo <= nchi) ? min(cap, nchi - nclo) : 0;
   if (hdr->root_leaf) T = 0;
-  const int D = share_depth(first ? 1 : *w.nodes);
+  const int D = share_depth(w.lanes, first ? 1 : *w.nodes);
   for (int q = tid; q < T; q += 1024) {
     const int t = nchi - 1 - q, node = first ? 0 : w.node[q];
     double lo = first ? hdr->lo : w.lo[q], hi = first ? hdr->hi : w.hi[q];
@@ -371,8 +373,8 @@ struct Twist {
   const double *a, *b, *l, *d, *omega;
   double *u, *vs;             // u in place (column j of the n x k row-major u), v interleaved
   double *S, *P, *DP, *RP;
-  double* best;               // [2][chunks][k]: least |gamma| of a chunk (v, u), then largest |v|
-  int* at;                    // [2][chunks][k]: its index
+  double* best[2];            // [chunks][k]: least |gamma| of a chunk (v, u), then largest |v|
+  int* at[2];                 // [chunks][k]: its index
   int* twist;                 // [2][k]
   double* inv[2];             // [k]: 1 / norm (v, u)
   int chunks;
@@ -480,9 +482,9 @@ __global__ __launch_bounds__(128) void k_twist_min(Twist T) {
     at = take ? i : at;
   }
   if (active) {
-    const size_t e = ((size_t)side * T.chunks + blockIdx.y) * K + j;
-    T.best[e] = best;
-    T.at[e] = at;
+    const size_t e = blockIdx.y * K + j;
+    T.best[side][e] = best;
+    T.at[side][e] = at;
   }
 }
 
@@ -491,13 +493,14 @@ __global__ __launch_bounds__(256) void k_twist_pick(Twist T, int* __restrict__ t
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= 2 * T.k) return;
   const int side = e / T.k, j = e - side * T.k;
-  const size_t base = (size_t)side * T.chunks * T.k + j;
-  double best = T.best[base];
-  int at = T.at[base];
+  const double* __restrict__ bests = T.best[side];
+  const int* __restrict__ ats = T.at[side];
+  double best = bests[j];
+  int at = ats[j];
 #pragma unroll 8
   for (int c = 1; c < T.chunks; c++) {
-    const double g = T.best[base + (size_t)c * T.k];
-    const int i = T.at[base + (size_t)c * T.k];
+    const double g = bests[(size_t)c * T.k + j];
+    const int i = ats[(size_t)c * T.k + j];
     if (g < best) { best = g; at = i; }
   }
   T.twist[e] = at;
@@ -610,8 +613,8 @@ __global__ __launch_bounds__(128) void k_twist_scale(Twist T) {
     at = take ? i : at;
   }
   if (side == 0) {
-    T.best[(size_t)blockIdx.y * K + j] = best;
-    T.at[(size_t)blockIdx.y * K + j] = at;
+    T.best[0][blockIdx.y * K + j] = best;
+    T.at[0][blockIdx.y * K + j] = at;
   }
 }
 
@@ -624,8 +627,8 @@ __global__ __launch_bounds__(64) void k_vsign(Twist T, const double* __restrict_
   int p = 0;
 #pragma unroll 8
   for (int c = 0; c < T.chunks; c++) {
-    const double x = T.best[c * K + j];
-    const int i = T.at[c * K + j];
+    const double x = T.best[0][c * K + j];
+    const int i = T.at[0][c * K + j];
     if (x > best) { best = x; p = i; }
   }
   double signer;
@@ -720,10 +723,17 @@ struct BisectWs {
   int *f_clo[2], *f_chi[2];
   int* ctr;  // [0] frontier size (next), [1] leaf count, [2] overflow
   double *L_lo, *L_hi;
-  ShareWs share;  // in the replay's frontiers, which are not in use at the same time
+  ShareWs share;  // in the replay's scratch, which is not in use at the same time
 };
 
-size_t bisect_ws_bytes(int n, void* base, BisectWs* ws, Bump* bump, bool own_table = true) {
+// The most lanes whose counts fit in so many bytes.
+int share_lanes(size_t bytes) {
+  int lanes = kShareLanes;
+  while (lanes > 1 && lanes * sizeof(int) > bytes) lanes >>= 1;
+  return lanes;
+}
+
+size_t bisect_ws_bytes(int n, void* base, BisectWs* ws, Bump* bump) {
   Bump& B = *bump;
   BisectWs w;
   w.hdr = B.take<BisectHdr>(1);
@@ -740,8 +750,17 @@ size_t bisect_ws_bytes(int n, void* base, BisectWs* ws, Bump* bump, bool own_tab
   w.ctr = B.take<int>(4);
   w.L_lo = B.take<double>(w.cap);
   w.L_hi = B.take<double>(w.cap);
-  w.share = ShareWs{w.f_lo[0], w.f_hi[0], w.f_lo[1], w.f_hi[1], w.f_clo[1], w.f_chi[1], w.f_clo[0], w.ctr,
-                    own_table ? B.take<int>(kShareLanes) : nullptr};
+  Bump R(w.f_lo[0], (size_t)64 * w.cap);  // two frontiers and the leaves: 24 + 24 + 16 bytes a node
+  w.share.node_lo = R.take<double>(n);
+  w.share.node_hi = R.take<double>(n);
+  w.share.lo = R.take<double>(n);
+  w.share.hi = R.take<double>(n);
+  w.share.clo = R.take<int>(n);
+  w.share.chi = R.take<int>(n);
+  w.share.node = R.take<int>(n);
+  w.share.nodes = R.take<int>(1);
+  w.share.table = R.take<int>(0);
+  w.share.lanes = share_lanes(R.cap - R.used);
   if (ws) *ws = w;
   (void)base;
   return B.used;
@@ -861,7 +880,7 @@ int run_bisection(int n, const double* a, const double* b, double tol, int top_k
       const int steps = cap <= kShareMaxTargets ? 2 : 1;
       for (int step = 0; step < steps; step++) {
         const int first = step == 0;
-        hipLaunchKernelGGL(k_bisect_share, dim3(kShareLanes / 256 + first), dim3(256), 0, s, n, a, b, w.hdr, tol,
+        hipLaunchKernelGGL(k_bisect_share, dim3(share.lanes / 256 + first), dim3(256), 0, s, n, a, b, w.hdr, tol,
                            first, share);
         hipLaunchKernelGGL(k_bisect_descend, dim3(1), dim3(1024), 0, s, w.hdr, tol, cap, first, share);
       }
@@ -935,12 +954,8 @@ int exc_ldl(int n, const double* d_alpha, const double* d_beta, double* d_l, dou
 
 namespace {
 struct TwistWs {
-  double *l, *d, *S, *P, *DP, *RP, *vs, *sgn, *best;
+  double *l, *d, *S, *P, *DP, *RP, *vs, *sgn;
 };
-// Chunk results of the search for the twists: 2 x chunks x k doubles and as many ints.
-size_t twist_best_doubles(int n, int k) { return 3 * (((size_t)n + kRows - 1) / kRows) * k; }
-// The shared levels' table fits in the sequences, which are not in use before the bisection ends.
-bool table_in_sequences(int n, int k) { return 4 * ((size_t)n + 1) * k * sizeof(double) >= kShareLanes * sizeof(int); }
 void twist_ws(int n, int k, Bump& B, TwistWs* w) {
   w->l = B.take<double>(n);
   w->d = B.take<double>(n);
@@ -950,8 +965,6 @@ void twist_ws(int n, int k, Bump& B, TwistWs* w) {
   w->RP = B.take<double>((size_t)(n + 1) * k);
   w->vs = B.take<double>((size_t)n * k);
   w->sgn = B.take<double>(k);
-  // the chunk results live in v's place until the multipliers are written there (n >= 3 has room)
-  w->best = (size_t)n * k >= twist_best_doubles(n, k) ? w->vs : B.take<double>(twist_best_doubles(n, k));
 }
 
 int run_twisted(int n, int k, const double* omega, const double* a, const double* b, double* u, double* v,
@@ -962,9 +975,14 @@ int run_twisted(int n, int k, const double* omega, const double* a, const double
     EXC_CHECK_HIP(hipGetLastError());
   }
   const int chunks = (n + kRows - 1) / kRows;
-  // row n of each sequence is not stored: the twists and the norms go there
-  const size_t end = (size_t)n * k;
-  Twist T{n, k, a, b, w.l, w.d, omega, u, w.vs, w.S, w.P, w.DP, w.RP, w.best, (int*)(w.best + 2 * (size_t)chunks * k),
+  // Row n of each sequence is not stored: the twists and the norms go there, and before the norms a
+  // single chunk's results. Those of several chunks live in v's place until the multipliers are
+  // written there (two chunks are over 32 rows, and 6 are needed).
+  const size_t end = (size_t)n * k, per = (size_t)chunks * k;
+  double* best = chunks == 1 ? w.P + end : w.vs;
+  double* best_u = chunks == 1 ? w.DP + end : w.vs + per;
+  int* at = (int*)(chunks == 1 ? w.RP + end : w.vs + 2 * per);
+  Twist T{n, k, a, b, w.l, w.d, omega, u, w.vs, w.S, w.P, w.DP, w.RP, {best, best_u}, {at, at + per},
           (int*)(w.S + end), {w.P + end, w.DP + end}, chunks};
   const unsigned groups = exc_detail::ceil_div(k, 64);
   hipLaunchKernelGGL(k_qds, dim3(groups), dim3(128), 0, s, T);
@@ -973,8 +991,8 @@ int run_twisted(int n, int k, const double* omega, const double* a, const double
   hipLaunchKernelGGL(k_twist_mult, dim3(groups, chunks), dim3(256), 0, s, T);
   hipLaunchKernelGGL(k_twist_chain, dim3(groups), dim3(256), 0, s, T);
   // the sequences are done with: the scaling's chunk results go over s
-  T.best = w.S;
-  T.at = (int*)(w.S + (size_t)chunks * k);
+  T.best[0] = w.S;
+  T.at[0] = (int*)(w.S + per);
   hipLaunchKernelGGL(k_twist_scale, dim3(groups, chunks), dim3(128), 0, s, T);
   EXC_CHECK_HIP(hipGetLastError());
   if (apply_vsign) {
@@ -1011,7 +1029,7 @@ int exc_twisted_vectors(int n, int k, const double* d_omega, const double* d_alp
 
 size_t exc_bidiag_svd_workspace(int k, int top_k) {
   Bump B(nullptr, 0);
-  bisect_ws_bytes(k, nullptr, nullptr, &B, !table_in_sequences(k, top_k));
+  bisect_ws_bytes(k, nullptr, nullptr, &B);
   B.take<int>(1);
   TwistWs w;
   twist_ws(k, top_k, B, &w);
@@ -1025,11 +1043,16 @@ int exc_bidiag_svd(int k, const double* d_alpha, const double* d_beta, double* d
               EXC_ERR_ARG, "exc_bidiag_svd: bad arguments");
   Bump B(d_work, work_bytes);
   BisectWs bw;
-  bisect_ws_bytes(k, d_work, &bw, &B, !table_in_sequences(k, top_k));
+  bisect_ws_bytes(k, d_work, &bw, &B);
   int* dcount = B.take<int>(1);
   TwistWs tw;
   twist_ws(k, top_k, B, &tw);
-  if (!bw.share.table) bw.share.table = (int*)tw.S;
+  // the sequences, which are not in use before the bisection ends, may hold more lanes' counts
+  const int lanes = share_lanes(4 * ((size_t)k + 1) * top_k * sizeof(double));
+  if (lanes > bw.share.lanes) {
+    bw.share.table = (int*)tw.S;
+    bw.share.lanes = lanes;
+  }
   EXC_REQUIRE(B.ok(), EXC_ERR_SPACE, "exc_bidiag_svd: workspace too small");
   hipStream_t s = exc_detail::stream(stream);
   hipLaunchKernelGGL(k_frob_bound, dim3(1), dim3(256), 0, s, k, d_alpha, d_beta, bw.hdr);

@@ -147,3 +147,27 @@ def test_bidiag_svd_edges(hip, oracle, kind, n, top_k):
     assert rcg == 0
     assert np.array_equal(sg, so) and np.array_equal(twg, two)
     assert np.array_equal(ug, uo) and np.array_equal(vg, vo)
+
+
+@pytest.mark.parametrize("n,top_k", [(1, 1), (2, 1), (2, 2), (3, 2), (32, 32), (100, 60), (256, 3), (300, 5), (300, 20),
+                                     (311, 4), (312, 4), (933, 7), (934, 7)])
+def test_bidiag_svd_fewer_values_in_the_workspace_of_all(hip, oracle, n, top_k):
+    """A workspace of the size for all values serves a call for fewer, where the shared levels' counts
+    lie in the search's scratch (few values) or in the sequences, and the bisection alone. Bit for bit."""
+    banner(f"bidiag_svd n={n} top_k={top_k} in the workspace of {n}")
+    a, b = random_bidiagonal(np.random.default_rng(7 * n + top_k), n, "gauss")
+    so, uo, vo, two, rco = oracle.bidiag_svd(a, b, top_k)
+    assert rco >= 0
+    da = hip.DeviceArray.from_host(a)
+    db = hip.DeviceArray.from_host(np.append(b, 0.0))
+    du, dv, ds = hip.DeviceArray((n, top_k)), hip.DeviceArray((top_k, n)), hip.DeviceArray((top_k,))
+    dt = hip.DeviceArray((2 * top_k,), np.int32)
+    ws = hip.workspace(hip.lib.exc_bidiag_svd_workspace(n, n))
+    hip.call("exc_bidiag_svd", n, da.ptr, db.ptr, du.ptr, dv.ptr, ds.ptr, top_k, dt.ptr, ws.ptr, ws.nbytes, None)
+    hip.sync()
+    assert np.array_equal(ds.to_host(), so) and np.array_equal(dt.to_host().reshape(two.shape), two)
+    assert np.array_equal(du.to_host(), uo) and np.array_equal(dv.to_host(), vo)
+    ub = float(np.sum(a * a) + np.sum(b * b))
+    sg, lo, hi = hip.bisection(a, b, 0.0, ub, 1e-20, top_k)
+    so, loo, hio = oracle.bisection(a, b, 0.0, ub, 1e-20, top_k)
+    assert np.array_equal(sg, so) and np.array_equal(lo, loo) and np.array_equal(hi, hio)

@@ -176,3 +176,23 @@ for cols in ((600, 0), (0,), (0, 0, 700)):
 """
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, (r.stdout, r.stderr[-2000:])
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 33, 100, 255, 256, 300, 933, 934, 2000])
+def test_bidiag_workspaces_cover_fewer_values(n):
+    """A workspace sized for many values serves fewer: the queries do not fall with the number of values.
+    And they hold nothing beyond the header, the leaves, the search's frontiers, the factorization, the
+    sequences, v and the signs, each rounded up to 256 bytes."""
+    from excalibur_amd import hip
+    up = lambda b: (b + 255) // 256 * 256  # noqa: E731
+    cap = 4 * n + 1024
+    bisect = 256 + 3 * up(8 * (n + 1)) + 2 * (2 * up(8 * cap) + 2 * up(4 * cap)) + 256 + 2 * up(8 * cap)
+    twisted = lambda k: 2 * up(8 * n) + 4 * up(8 * (n + 1) * k) + up(8 * n * k) + up(8 * k)  # noqa: E731
+    last = 0
+    for k in sorted({0, 1, 2, 20, 27, 28, 36, 81, n // 2, n} & set(range(n + 1))):
+        need = hip.lib.exc_bidiag_svd_workspace(n, k)
+        assert need >= last
+        last = need
+        assert hip.lib.exc_bisection_workspace(n, k) <= bisect + 256
+        assert hip.lib.exc_twisted_workspace(n, k) <= twisted(k) + 256
+        assert need <= bisect + 256 + twisted(k) + 256
