@@ -635,11 +635,33 @@ struct GemmPlan {
   int splits;  // of K
 };
 
+// The least splits of K: they bound the length of a running sum, and with it the rounding error of
+// the result. They are those that let 128 x 128 tiles on `slots` resident workgroups end soonest: rounds
+// of the chip times steps of about 3 us, and the sum of the partials at 3 TB/s. The faster kernels of
+// today would take fewer (1000 x 1000 x 2000 in FP64: 2 instead of 8), but then the sums are longer (1008
+// terms instead of 256) and the error of their rounding was 1.7 to 2.9 times as large.
+template <typename T>
+long least_splits(long M, long N, long K, long tiles, long slots, long room) {
+  constexpr int BK = Shapes<T>::Big::BK;
+  if (tiles >= slots) return 1;
+  long best = 1;
+  double best_us = -1.0;
+  for (long sp = 1; sp <= std::min({K / BK, 4 * ((slots + tiles - 1) / tiles), room}); sp++) {
+    const long rounds = (tiles * sp + slots - 1) / slots, depth = ((K + sp - 1) / sp + BK - 1) / BK;
+    const double us = 3.0 * (double)(rounds * depth) + (sp > 1 ? 5.0 + (double)sp * M * N * sizeof(T) / 3.0e6 : 0.0);
+    if (best_us < 0.0 || us < best_us) {
+      best_us = us;
+      best = sp;
+    }
+  }
+  return best;
+}
+
 // Tile and split of one product: the pair with the least estimated time. A CU with w workgroups
 // takes max(w kStep, kAlone) per step; a split adds the write and the fixed-order sum of its partials
-// (about 5 TB/s, they stay in the caches) and 5 us for its launch. Splits need a workspace and keep
-// at least two steps each (a lone step is all latency); near ties go to the larger tile and fewer
-// splits.
+// (about 5 TB/s, they stay in the caches) and 5 us for its launch. Splits need a workspace, and those
+// beyond the least keep two steps each (a lone step is all latency); near ties go to the larger tile and
+// fewer splits.
 template <typename T>
 GemmPlan gemm_plan(long M, long N, long K, const ExcGemmOpts& o) {
   constexpr int BK = Shapes<T>::Big::BK;
@@ -647,6 +669,11 @@ GemmPlan gemm_plan(long M, long N, long K, const ExcGemmOpts& o) {
   const long cus = compute_units();
   GemmPlan best{128, 1};
   double best_us = -1.0;
+  const long fit = o.work && K > 4 * BK ? (long)std::min<size_t>(K, o.work_bytes / ((size_t)M * N * sizeof(T))) : 1;
+  const long room = std::min(fit, K / (2 * BK));
+  const long tm128 = (M + 127) / 128, tn128 = (N + 127) / 128;
+  const long floor = least_splits<T>(M, N, K, o.lower_only ? tm128 * (tm128 + 1) / 2 : tm128 * tn128,
+                                     cus * Shapes<T>::Big::kPerCu, fit);
   for (int c = 0; c < 2; c++) {
     const long tile = c == 0 ? 128 : 64;
     const long tm = (M + tile - 1) / tile, tn = (N + tile - 1) / tile;
@@ -655,11 +682,10 @@ GemmPlan gemm_plan(long M, long N, long K, const ExcGemmOpts& o) {
     const double share = o.tri != EXC_TRI_NONE ? 0.5 + 0.5 / (double)(o.tri <= EXC_TRI_A_UPPER ? tm : tn) : 1.0;
     const long slots = cus * (c == 0 ? Shapes<T>::Big::kPerCu : Shapes<T>::Small::kPerCu);
     const double out = (double)sizeof(T) * M * N * (o.lower_only ? 0.5 : 1.0);
-    const long room = o.work && K > 4 * BK ? (long)std::min<size_t>(K / (2 * BK), o.work_bytes / ((size_t)M * N * sizeof(T))) : 1;
     const long most = std::max(1L, std::min(room, 2 * ((slots + tiles - 1) / tiles)));
     long least = std::min(room, (K + kMaxSum - 1) / kMaxSum);
     if (Shapes<T>::kMaxSumFills) least = std::min(least, 2 * cus / tiles);
-    least = std::max(1L, least);
+    least = std::max(least, floor);
     for (long sp = least; sp <= std::max(least, most); sp++) {
       const long depth = ((K + sp - 1) / sp + BK - 1) / BK;
       const long per_cu = (tiles * sp + cus - 1) / cus;

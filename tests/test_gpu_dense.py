@@ -161,3 +161,27 @@ def test_gemm_edges(hip, f32, ta, tb):
             got = got[1:].reshape(M, ldc)
             assert np.isnan(got[:, N:]).all()
             assert (np.abs(got[:, :N] - want) <= bound).all(), (M, N, K, work)
+
+
+@pytest.mark.parametrize("f32,M,N,K,longest", [
+    (False, 500, 1000, 496, 64), (False, 1000, 1000, 992, 128), (False, 1000, 1000, 2000, 256),
+    (False, 200, 600, 96, 16), (False, 843, 1365, 320, 80), (False, 364, 1027, 8000, 1008),
+    (True, 584, 584, 5200, 336), (True, 996, 996, 14384, 1200), (True, 1202, 1202, 8000, 1152),
+    (True, 2000, 2000, 20000, 2000), (True, 234, 234, 128, 16)])
+def test_gemm_sum_length(hip, f32, M, N, K, longest):
+    """The rounding error of a product grows with the terms of a running sum, so with a workspace K is split
+    at least this far. All factors are one except the first of every row, 2^27 (2^56 in FP64): a running
+    sum that starts there loses each later term (up to 7 at a time are less than half a unit of the last
+    place), the others are whole numbers and exact, so the result shows the first sum's length."""
+    dt, first = (np.float32, 2.0 ** 27) if f32 else (np.float64, 2.0 ** 56)
+    banner(f"gemm sum length {M}x{N}x{K} f32={f32}")
+    A = np.ones((M, K), dt)
+    A[:, 0] = first
+    dA, dB = hip.DeviceArray.from_host(A), hip.DeviceArray.from_host(np.ones((N, K), dt))
+    dC = hip.DeviceArray((M, N), dt)
+    ws = hip.workspace(hip.lib.exc_gemm_workspace(M, N, K))
+    hip.call("exc_sgemm" if f32 else "exc_dgemm", 0, 1, M, N, K, 1.0, dA.ptr, K, dB.ptr, K, 0.0, dC.ptr, N, ws.ptr,
+             ws.nbytes, None)
+    hip.sync()
+    # K and the lengths are multiples of the unit of the last place, 16
+    assert np.max(K - (dC.to_host().astype(np.float64) - first)) <= longest
