@@ -276,7 +276,7 @@ int exc_batched_local_qr(int nb, int m, const long* h_cols, const double* const*
     q.K = h_cols[b];
     q.lower_only = q.mirror = 1;
   }
-  int rc = exc_gemm_grouped_opts(4, 0, 1, nb, P.data(), 1.0, 0.0, -1, gwork, gws, s);
+  int rc = exc_gemm_grouped_opts(4, 1, nb, P.data(), 1.0, 0.0, -1, gwork, gws, s);
   if (rc) return rc;
   hipLaunchKernelGGL(k_f32_to_f64_batched, dim3((unsigned)std::min<size_t>(1024, (mm + 255) / 256), nb), dim3(256), 0, s,
                      (long)mm, tg32, tG);
@@ -323,7 +323,7 @@ int exc_batched_local_qr(int nb, int m, const long* h_cols, const double* const*
     q.K = m;
     q.tri = EXC_TRI_A_LOWER;
   }
-  rc = exc_gemm_grouped_opts(8, 0, 0, nb, P.data(), 1.0, 0.0, -1, gwork, gws, s);
+  rc = exc_gemm_grouped_opts(8, 0, nb, P.data(), 1.0, 0.0, -1, gwork, gws, s);
   if (rc) return rc;
   std::vector<int> passes(nb, 1);
   std::vector<double> dev(nb, 0.0);
@@ -342,7 +342,7 @@ int exc_batched_local_qr(int nb, int m, const long* h_cols, const double* const*
       q.K = h_cols[b];
       q.lower_only = q.mirror = 1;
     }
-    rc = exc_gemm_grouped_opts(8, 0, 1, nb, P.data(), 1.0, 0.0, -1, gwork, gws, s);
+    rc = exc_gemm_grouped_opts(8, 1, nb, P.data(), 1.0, 0.0, -1, gwork, gws, s);
     if (rc) return rc;
     hipLaunchKernelGGL(k_stats_batched, dim3(nb), dim3(256), 0, s, m, (const double* const*)tG, (long)m, stats);
     EXC_CHECK_HIP(hipMemcpyAsync(L3, G, mm * nb * sizeof(double), hipMemcpyDeviceToDevice, s));
@@ -378,7 +378,7 @@ int exc_batched_local_qr(int nb, int m, const long* h_cols, const double* const*
     // the product may not overwrite its own input: d_qt serves as its FP64 scratch
     EXC_REQUIRE(h_qt != nullptr, EXC_ERR_NUMERIC,
                 "exc_batched_local_qr: an ill-conditioned block needs a second FP64 pass; pass d_qt for its scratch");
-    rc = exc_gemm_grouped_opts(8, 0, 0, nb, P.data(), 1.0, 0.0, -1, gwork, gws, s);
+    rc = exc_gemm_grouped_opts(8, 0, nb, P.data(), 1.0, 0.0, -1, gwork, gws, s);
     if (rc) return rc;
     for (int b = 0; b < nb; b++)
       EXC_CHECK_HIP(hipMemcpyAsync(Z + xoff[b], h_qt[b], (size_t)m * h_cols[b] * sizeof(double),
@@ -395,7 +395,7 @@ int exc_batched_local_qr(int nb, int m, const long* h_cols, const double* const*
       q.M = q.N = q.K = m;
       q.tri = EXC_TRI_A_LOWER;
     }
-    rc = exc_gemm_grouped_opts(8, 0, 0, nb, P.data(), 1.0, 0.0, 0, gwork, gws, s);
+    rc = exc_gemm_grouped_opts(8, 0, nb, P.data(), 1.0, 0.0, 0, gwork, gws, s);
     if (rc) return rc;
     EXC_CHECK_HIP(hipMemcpyAsync(L1, S, mm * nb * sizeof(double), hipMemcpyDeviceToDevice, s));
     for (int b = 0; b < nb; b++) passes[b]++;
@@ -413,7 +413,7 @@ int exc_batched_local_qr(int nb, int m, const long* h_cols, const double* const*
     q.M = q.N = q.K = m;
     q.tri = EXC_TRI_A_LOWER;
   }
-  rc = exc_gemm_grouped_opts(8, 0, 0, nb, P.data(), 1.0, 0.0, 0, gwork, gws, s);
+  rc = exc_gemm_grouped_opts(8, 0, nb, P.data(), 1.0, 0.0, 0, gwork, gws, s);
   if (rc) return rc;
   if (h_qt) {  // Q^T = L3^-1 Z
     rc = trinv(tL3, tS);
@@ -432,7 +432,7 @@ int exc_batched_local_qr(int nb, int m, const long* h_cols, const double* const*
       q.K = m;
       q.tri = EXC_TRI_A_LOWER;
     }
-    rc = exc_gemm_grouped_opts(8, 0, 0, nb, P.data(), 1.0, 0.0, -1, gwork, gws, s);
+    rc = exc_gemm_grouped_opts(8, 0, nb, P.data(), 1.0, 0.0, -1, gwork, gws, s);
     if (rc) return rc;
   }
   if (h_stats)

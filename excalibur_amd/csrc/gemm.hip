@@ -49,7 +49,6 @@ struct Mfma<float> {
 
 
 struct GemmArgs {
-  int ta, tb;
   long M, N, K;
   const void* A;
   long lda;
@@ -99,17 +98,10 @@ __device__ inline void tile_of(const GemmArgs& g, long& tile_m, long& tile_n, lo
   }
 }
 
-// K range [k0, k1) that can contribute to output rows [i0, i0+bm) / columns [j0, j0+bn).
-__device__ inline void k_range(const GemmArgs& g, long i0, long j0, int bm, int bn, long& k0, long& k1) {
-  k0 = 0;
-  k1 = g.K;
-  switch (g.tri) {
-    case EXC_TRI_A_LOWER: k1 = min(k1, i0 + bm); break;  // op(A)[i][k] = 0 for k > i
-    case EXC_TRI_A_UPPER: k0 = max(k0, i0); break;       // op(A)[i][k] = 0 for k < i
-    case EXC_TRI_B_LOWER: k0 = max(k0, j0); break;       // op(B)[k][j] = 0 for k < j
-    case EXC_TRI_B_UPPER: k1 = min(k1, j0 + bn); break;  // op(B)[k][j] = 0 for k > j
-    default: break;
-  }
+// K range [k0, k1) that can contribute to output rows [i0, i0+bm).
+__device__ inline void k_range(const GemmArgs& g, long i0, int bm, long& k0, long& k1) {
+  k0 = g.tri == EXC_TRI_A_UPPER ? i0 : 0;                   // op(A)[i][k] = 0 for k < i
+  k1 = g.tri == EXC_TRI_A_LOWER ? min(g.K, i0 + bm) : g.K;  // op(A)[i][k] = 0 for k > i
 }
 
 // 16 bytes of one operand, in registers and in LDS; in global memory only the elements' own
@@ -379,13 +371,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, long i0, long j0, l
       if (tail || ragged_b) sb.fix(kb, k1);
     }
     if (TRI) {
-      switch (g.tri) {
-        case EXC_TRI_A_LOWER: if (kb + BK > i0 + 1) sa.mask(kb, true); break;
-        case EXC_TRI_A_UPPER: if (kb < i0 + S::BM - 1) sa.mask(kb, false); break;
-        case EXC_TRI_B_LOWER: if (kb < j0 + S::BN - 1) sb.mask(kb, false); break;
-        case EXC_TRI_B_UPPER: if (kb + BK > j0 + 1) sb.mask(kb, true); break;
-        default: break;
-      }
+      const bool lower = g.tri == EXC_TRI_A_LOWER;
+      if (lower ? kb + BK > i0 + 1 : g.tri == EXC_TRI_A_UPPER && kb < i0 + S::BM - 1) sa.mask(kb, lower);
     }
     sa.store(lds.a[buf]);
     sb.store(lds.b[buf]);
@@ -477,7 +464,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, long i0, long j0, l
       }
 }
 
-// TRI: one operand is triangular. The general products are a kernel of their own: the triangle's
+// TRI: op(A) is triangular. The general products are a kernel of their own: the triangle's
 // code in their loop costs registers, and with them 5 % of their rate.
 template <typename T, int TA, int TB, bool TRI, class S>
 __global__ __launch_bounds__(S::kThreads, S::kPerCu * S::kThreads / 256) void k_gemm(GemmArgs g) {
@@ -494,7 +481,7 @@ __global__ __launch_bounds__(S::kThreads, S::kPerCu * S::kThreads / 256) void k_
   }
   for (;;) {
     long k0, k1;
-    k_range(g, tile_m * S::BM, j0, S::BM, S::BN, k0, k1);
+    k_range(g, tile_m * S::BM, S::BM, k0, k1);
     k0 = max(k0, ks);
     k1 = min(k1, ke);
     gemm_tile<T, TA, TB, true, S>(g, tile_m * S::BM, j0, k0, k1, Cb, ldc, 0, 0, g.kchunk == 0, lds);
@@ -529,13 +516,13 @@ struct GroupRed {
   int p, tile_m, tile_n, first_slot, nslots, pad;
 };
 
-// 64 x 64 tiles where an operand is triangular (they skip more of its zeros, and the large tile's
+// 64 x 64 tiles where op(A) is triangular (they skip more of its zeros, and the large tile's
 // registers do not hold the triangle's code: 32 products L^-1 X of order 512 took 7.1 ms with it,
 // 6.9 with the small one), 128 x 128 elsewhere.
 template <typename T, bool TRI>
 using GroupShape = std::conditional_t<TRI, typename Shapes<T>::Small, typename Shapes<T>::Big>;
 
-template <typename T, int TA, int TB, bool TRI>
+template <typename T, int TB, bool TRI>
 __global__ __launch_bounds__((GroupShape<T, TRI>::kThreads), (GroupShape<T, TRI>::kPerCu * GroupShape<T, TRI>::kThreads / 256)) void k_gemm_grouped(
     const GroupProb* __restrict__ probs, const GroupItem* __restrict__ items, long nitems, T* __restrict__ part,
     double alpha, double beta) {
@@ -556,11 +543,11 @@ __global__ __launch_bounds__((GroupShape<T, TRI>::kThreads), (GroupShape<T, TRI>
     const long i0 = (long)tile_m * BM;
     long k0 = w.k0, k1 = w.k1;
     if (TRI) {
-      k_range(g, i0, j0, BM, BN, k0, k1);
+      k_range(g, i0, BM, k0, k1);
       k0 = max(k0, w.k0);
       k1 = min(k1, w.k1);
     }
-    gemm_tile<T, TA, TB, TRI, S>(g, i0, j0, k0, k1, Cb, direct ? pr.ldc : BN, direct ? 0 : i0, direct ? 0 : j0,
+    gemm_tile<T, 0, TB, TRI, S>(g, i0, j0, k0, k1, Cb, direct ? pr.ldc : BN, direct ? 0 : i0, direct ? 0 : j0,
                                  direct, lds);
     if (!TRI || w.other_m < 0 || tile_m == w.other_m) break;
     tile_m = w.other_m;
@@ -678,8 +665,8 @@ GemmPlan gemm_plan(long M, long N, long K, const ExcGemmOpts& o) {
     const long tile = c == 0 ? 128 : 64;
     const long tm = (M + tile - 1) / tile, tn = (N + tile - 1) / tile;
     const long tiles = o.lower_only ? tm * (tm + 1) / 2 : tm * tn;
-    // a triangular operand leaves the tiles about half of K on average
-    const double share = o.tri != EXC_TRI_NONE ? 0.5 + 0.5 / (double)(o.tri <= EXC_TRI_A_UPPER ? tm : tn) : 1.0;
+    // a triangular op(A) leaves the tiles about half of K on average
+    const double share = o.tri != EXC_TRI_NONE ? 0.5 + 0.5 / (double)tm : 1.0;
     const long slots = cus * (c == 0 ? Shapes<T>::Big::kPerCu : Shapes<T>::Small::kPerCu);
     const double out = (double)sizeof(T) * M * N * (o.lower_only ? 0.5 : 1.0);
     const long most = std::max(1L, std::min(room, 2 * ((slots + tiles - 1) / tiles)));
@@ -704,10 +691,14 @@ GemmPlan gemm_plan(long M, long N, long K, const ExcGemmOpts& o) {
 template <typename T, bool TRI, class S>
 void gemm_launch(int ta, int tb, const GemmArgs& g, hipStream_t s) {
   const dim3 grid((unsigned)g.total), block(S::kThreads);
-  if (!ta && !tb) hipLaunchKernelGGL((k_gemm<T, 0, 0, TRI, S>), grid, block, 0, s, g);
-  else if (!ta && tb) hipLaunchKernelGGL((k_gemm<T, 0, 1, TRI, S>), grid, block, 0, s, g);
-  else if (ta && !tb) hipLaunchKernelGGL((k_gemm<T, 1, 0, TRI, S>), grid, block, 0, s, g);
-  else hipLaunchKernelGGL((k_gemm<T, 1, 1, TRI, S>), grid, block, 0, s, g);
+  if constexpr (!TRI)
+    if (tb) {
+      if (ta) hipLaunchKernelGGL((k_gemm<T, 1, 1, TRI, S>), grid, block, 0, s, g);
+      else hipLaunchKernelGGL((k_gemm<T, 0, 1, TRI, S>), grid, block, 0, s, g);
+      return;
+    }
+  if (ta) hipLaunchKernelGGL((k_gemm<T, 1, 0, TRI, S>), grid, block, 0, s, g);
+  else hipLaunchKernelGGL((k_gemm<T, 0, 0, TRI, S>), grid, block, 0, s, g);
 }
 
 template <typename T>
@@ -715,8 +706,9 @@ int gemm_impl(int ta, int tb, long M, long N, long K, double alpha, const T* A, 
               double beta, T* C, long ldc, const ExcGemmOpts& o, hipStream_t s) {
   EXC_REQUIRE(M >= 0 && N >= 0 && K >= 0 && C, EXC_ERR_ARG, "exc_gemm: bad shape");
   if (M == 0 || N == 0) return EXC_OK;
+  EXC_REQUIRE(o.tri == EXC_TRI_NONE || !tb, EXC_ERR_ARG, "exc_gemm: a triangular op(A) takes op(B) = B");
   GemmArgs g{};
-  g.ta = ta; g.tb = tb; g.M = M; g.N = N; g.K = K;
+  g.M = M; g.N = N; g.K = K;
   g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc;
   g.alpha = alpha; g.beta = beta; g.tri = o.tri; g.lower_only = o.lower_only;
   constexpr int BK = Shapes<T>::Big::BK;
@@ -724,7 +716,7 @@ int gemm_impl(int ta, int tb, long M, long N, long K, double alpha, const T* A, 
   g.bm = g.bn = p.tile;
   g.tm = (M + p.tile - 1) / p.tile;
   const long tn = (N + p.tile - 1) / p.tile;
-  g.pair = !o.lower_only && (o.tri == EXC_TRI_A_LOWER || o.tri == EXC_TRI_A_UPPER) ;
+  g.pair = !o.lower_only && o.tri != EXC_TRI_NONE;
   g.ntile = o.lower_only ? g.tm * (g.tm + 1) / 2 : (g.pair ? (g.tm + 1) / 2 : g.tm) * tn;
   int splits = p.splits;
   if (splits > 1) {
@@ -772,7 +764,7 @@ struct GroupPlan {
   std::vector<GroupRed> reds;
   long slots = 0;
   int tile = 128;
-  bool tri = false;  // any triangular problem: the kernel for both, with its tile
+  bool tri = false;  // any triangular problem: the kernel for all, with its tile
   double flops = 0.0;
 };
 
@@ -797,7 +789,7 @@ GroupPlan group_plan(int nprob, const ExcGemmProblem* P, long kchunk) {
     // chunks of about kchunk, of equal length within a problem
     const long splits = (kchunk > 0 && q.K > kchunk) ? (q.K + kchunk - 1) / kchunk : 1;
     const long chunk = splits == 1 ? q.K : ((q.K + splits - 1) / splits + BK - 1) / BK * BK;
-    const bool pair = splits == 1 && !q.lower_only && (q.tri == EXC_TRI_A_LOWER || q.tri == EXC_TRI_A_UPPER);
+    const bool pair = splits == 1 && !q.lower_only && q.tri != EXC_TRI_NONE;
     for (long b = 0; b < tn; b++)
       for (long a = 0; a < (pair ? (tm + 1) / 2 : tm); a++) {
         if (q.lower_only && a < b) continue;
@@ -825,10 +817,11 @@ size_t group_bytes(const GroupPlan& g, size_t tsize) {
 }
 
 template <typename T>
-int group_run(int ta, int tb, const GroupPlan& g, double alpha, double beta, void* work, size_t wb,
+int group_run(int tb, const GroupPlan& g, double alpha, double beta, void* work, size_t wb,
               hipStream_t s) {
   EXC_REQUIRE(group_bytes(g, sizeof(T)) <= wb, EXC_ERR_SPACE, "exc_gemm_grouped: workspace too small");
   if (g.items.empty()) return EXC_OK;
+  EXC_REQUIRE(tb ? !g.tri : g.tri && sizeof(T) == 8, EXC_ERR_ARG, "exc_gemm_grouped: no kernel for this form");
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   char* w = (char*)work;
   GroupProb* dp = (GroupProb*)w;
@@ -849,11 +842,8 @@ int group_run(int ta, int tb, const GroupPlan& g, double alpha, double beta, voi
   const dim3 grid((unsigned)nitems), block(g.tri ? GroupShape<T, true>::kThreads : GroupShape<T, false>::kThreads);
   hipEvent_t e0 = exc_prof::mark(s);
   auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, dp, di, nitems, part, alpha, beta); };
-  const bool tri = g.tri;
-  if (!ta && !tb) tri ? launch(k_gemm_grouped<T, 0, 0, true>) : launch(k_gemm_grouped<T, 0, 0, false>);
-  else if (!ta && tb) tri ? launch(k_gemm_grouped<T, 0, 1, true>) : launch(k_gemm_grouped<T, 0, 1, false>);
-  else if (ta && !tb) tri ? launch(k_gemm_grouped<T, 1, 0, true>) : launch(k_gemm_grouped<T, 1, 0, false>);
-  else tri ? launch(k_gemm_grouped<T, 1, 1, true>) : launch(k_gemm_grouped<T, 1, 1, false>);
+  if (tb) launch(k_gemm_grouped<T, 1, false>);
+  else if constexpr (sizeof(T) == 8) launch(k_gemm_grouped<T, 0, true>);
   EXC_CHECK_HIP(hipGetLastError());
   if (!g.reds.empty()) {
     hipLaunchKernelGGL(k_grouped_reduce<T>, dim3((unsigned)g.reds.size()), dim3(256), 0, s, dp, dr, part, g.tile,
@@ -875,13 +865,13 @@ std::vector<TuneEntry> g_tune;
 std::mutex g_tune_mu;
 
 template <typename T>
-int grouped_impl(int ta, int tb, int nprob, const ExcGemmProblem* P, double alpha, double beta, long kchunk,
+int grouped_impl(int tb, int nprob, const ExcGemmProblem* P, double alpha, double beta, long kchunk,
                  void* work, size_t wb, hipStream_t s) {
   EXC_REQUIRE(nprob >= 0 && (nprob == 0 || P), EXC_ERR_ARG, "exc_gemm_grouped: bad arguments");
-  if (kchunk >= 0) return group_run<T>(ta, tb, group_plan(nprob, P, kchunk), alpha, beta, work, wb, s);
+  if (kchunk >= 0) return group_run<T>(tb, group_plan(nprob, P, kchunk), alpha, beta, work, wb, s);
   // autotune: one timed run per candidate on the caller's data (each run overwrites the outputs
   // completely, so the last one leaves the result), the fastest kept per problem-set key
-  long key[8] = {(long)sizeof(T), ta, tb, nprob, 0, 0, 0, 0};
+  long key[8] = {(long)sizeof(T), 0, tb, nprob, 0, 0, 0, 0};
   for (int p = 0; p < nprob; p++) {
     key[4] += P[p].K;
     key[5] = std::max(key[5], P[p].K);
@@ -892,7 +882,7 @@ int grouped_impl(int ta, int tb, int nprob, const ExcGemmProblem* P, double alph
     std::lock_guard<std::mutex> lock(g_tune_mu);
     for (const TuneEntry& e : g_tune)
       if (std::equal(e.key, e.key + 8, key))
-        return group_run<T>(ta, tb, group_plan(nprob, P, e.kchunk), alpha, beta, work, wb, s);
+        return group_run<T>(tb, group_plan(nprob, P, e.kchunk), alpha, beta, work, wb, s);
   }
   EXC_REQUIRE(beta == 0.0, EXC_ERR_ARG, "exc_gemm_grouped: tuning runs need beta = 0 (each run overwrites C)");
   const long chunks[] = {0, 16384, 8192, 4096, 2048};
@@ -904,10 +894,10 @@ int grouped_impl(int ta, int tb, int nprob, const ExcGemmProblem* P, double alph
   for (long kc : chunks) {
     const GroupPlan g = group_plan(nprob, P, kc);
     if (group_bytes(g, sizeof(T)) > wb) continue;
-    int rc = group_run<T>(ta, tb, g, alpha, beta, work, wb, s);  // warm (and tables uploaded)
+    int rc = group_run<T>(tb, g, alpha, beta, work, wb, s);  // warm (and tables uploaded)
     if (rc) return rc;
     EXC_CHECK_HIP(hipEventRecord(a, s));
-    rc = group_run<T>(ta, tb, g, alpha, beta, work, wb, s);
+    rc = group_run<T>(tb, g, alpha, beta, work, wb, s);
     if (rc) return rc;
     EXC_CHECK_HIP(hipEventRecord(b, s));
     EXC_CHECK_HIP(hipEventSynchronize(b));
@@ -927,16 +917,16 @@ int grouped_impl(int ta, int tb, int nprob, const ExcGemmProblem* P, double alph
     std::lock_guard<std::mutex> lock(g_tune_mu);
     g_tune.push_back(best);
   }
-  return group_run<T>(ta, tb, group_plan(nprob, P, best.kchunk), alpha, beta, work, wb, s);
+  return group_run<T>(tb, group_plan(nprob, P, best.kchunk), alpha, beta, work, wb, s);
 }
 
 }  // namespace
 
-int exc_gemm_grouped_opts(int dtype, int ta, int tb, int nprob, const ExcGemmProblem* probs, double alpha, double beta,
+int exc_gemm_grouped_opts(int dtype, int tb, int nprob, const ExcGemmProblem* probs, double alpha, double beta,
                           long kchunk, void* work, size_t work_bytes, hipStream_t s) {
   EXC_REQUIRE(dtype == 4 || dtype == 8, EXC_ERR_ARG, "exc_gemm_grouped: dtype is 4 (float) or 8 (double)");
-  if (dtype == 8) return grouped_impl<double>(ta, tb, nprob, probs, alpha, beta, kchunk, work, work_bytes, s);
-  return grouped_impl<float>(ta, tb, nprob, probs, alpha, beta, kchunk, work, work_bytes, s);
+  if (dtype == 8) return grouped_impl<double>(tb, nprob, probs, alpha, beta, kchunk, work, work_bytes, s);
+  return grouped_impl<float>(tb, nprob, probs, alpha, beta, kchunk, work, work_bytes, s);
 }
 
 size_t exc_gemm_grouped_workspace(int dtype, int nprob, const ExcGemmProblem* probs, long kchunk) {

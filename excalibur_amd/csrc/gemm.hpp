@@ -5,9 +5,9 @@
 
 #include <cstddef>
 
-// Triangular restriction of one operand (after transposition): the other triangle is treated as
-// zero and the zero K range of each output tile is skipped.
-enum { EXC_TRI_NONE = 0, EXC_TRI_A_LOWER = 1, EXC_TRI_A_UPPER = 2, EXC_TRI_B_LOWER = 3, EXC_TRI_B_UPPER = 4 };
+// Triangular restriction of op(A): the other triangle is treated as zero and the zero K range of each
+// output tile is skipped. op(B) is then B.
+enum { EXC_TRI_NONE = 0, EXC_TRI_A_LOWER = 1, EXC_TRI_A_UPPER = 2 };
 
 struct ExcGemmOpts {
   int tri = EXC_TRI_NONE;
@@ -38,11 +38,11 @@ struct ExcGemmProblem {
   int mirror = 0;
   int beta_zero_hint = 0;
 };
-// Many independent products (all FP32 when dtype = 4, all FP64 when 8; one transposition pattern)
-// in one launch plus one reduction launch. kchunk: split K into chunks of about this length (0: no
-// split); kchunk < 0 lets the autotuner choose it by timing candidates on these problems once
+// Many independent products in one launch plus one reduction launch: with tb A B^T, none of them
+// triangular (all FP32 when dtype = 4, all FP64 when 8), without it A B in FP64 with a triangular A among
+// them. kchunk: split K into chunks of about this length (0: no split); kchunk < 0 lets the autotuner choose it by timing candidates on these problems once
 // (beta must be 0), then reuse the choice for problem sets of the same shape.
-int exc_gemm_grouped_opts(int dtype, int ta, int tb, int nprob, const ExcGemmProblem* probs, double alpha, double beta,
+int exc_gemm_grouped_opts(int dtype, int tb, int nprob, const ExcGemmProblem* probs, double alpha, double beta,
                           long kchunk, void* work, size_t work_bytes, hipStream_t s);
 size_t exc_gemm_grouped_workspace(int dtype, int nprob, const ExcGemmProblem* probs, long kchunk);
 // The autotuner's choices so far as a JSON list (extern "C", declared in excalibur_hip.h).
