@@ -137,12 +137,9 @@ struct Arena {
   }
 };
 
-}  // namespace
-
-extern "C" {
-
-size_t exc_batched_local_qr_workspace(int nb, int m, const long* h_cols) {
-  if (nb < 1 || m < 1 || !h_cols) return 0;
+// Workspace with room for the triangular products' candidates of the given K chunk (-1: all of them).
+// Without room for its partial tiles the autotuner passes a candidate over.
+size_t workspace_bytes(int nb, int m, const long* h_cols, long tri_kchunk) {
   Arena a{nullptr, 0, 0};
   size_t xs = 0;
   long kmax = 0;
@@ -174,9 +171,18 @@ size_t exc_batched_local_qr_workspace(int nb, int m, const long* h_cols) {
     probs[b].lower_only = probs[b].mirror = 0;
     probs[b].tri = EXC_TRI_A_LOWER;
   }
-  g = std::max(g, exc_gemm_grouped_workspace(8, nb, probs.data(), -1));
+  g = std::max(g, exc_gemm_grouped_workspace(8, nb, probs.data(), tri_kchunk));
   a.take<char>(g);
   return a.used + 256;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t exc_batched_local_qr_workspace(int nb, int m, const long* h_cols) {
+  if (nb < 1 || m < 1 || !h_cols) return 0;
+  return workspace_bytes(nb, m, h_cols, -1);
 }
 
 // See the file comment. d_x[b]: X_b (m x cols[b], row-major, FP64, not modified); d_rt[b]: R_b^T
@@ -187,7 +193,7 @@ int exc_batched_local_qr(int nb, int m, const long* h_cols, const double* const*
   EXC_REQUIRE(nb >= 1 && m >= 1 && h_cols && h_x && h_rt && d_work, EXC_ERR_ARG, "exc_batched_local_qr: bad arguments");
   for (int b = 0; b < nb; b++)
     EXC_REQUIRE(h_cols[b] >= m && h_x[b] && h_rt[b], EXC_ERR_ARG, "exc_batched_local_qr: block narrower than m");
-  EXC_REQUIRE(work_bytes >= exc_batched_local_qr_workspace(nb, m, h_cols), EXC_ERR_SPACE,
+  EXC_REQUIRE(work_bytes >= workspace_bytes(nb, m, h_cols, 0), EXC_ERR_SPACE,
               "exc_batched_local_qr: workspace too small");
   hipStream_t s = exc_detail::stream(stream);
   const size_t mm = (size_t)m * m;

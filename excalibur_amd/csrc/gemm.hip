@@ -508,10 +508,12 @@ struct GroupProb {
   int tri, lower_only, mirror, pad;
 };
 struct GroupItem {
-  int p, tile_m, tile_n, slot;  // slot < 0: the item owns its whole tile and stores it directly
-  int other_m, pad;             // >= 0: tile row it takes as well (a triangular op(A), see k_gemm)
+  // slot < 0: the item owns its whole tile and stores it directly; kPaired: and the tile of row
+  // tm - 1 - tile_m as well (a triangular op(A), see k_gemm)
+  int p, tile_m, tile_n, slot;
   long k0, k1;
 };
+constexpr int kPaired = -2;
 struct GroupRed {
   int p, tile_m, tile_n, first_slot, nslots, pad;
 };
@@ -539,6 +541,7 @@ __global__ __launch_bounds__((GroupShape<T, TRI>::kThreads), (GroupShape<T, TRI>
   const bool direct = w.slot < 0;
   const long j0 = (long)w.tile_n * BN;
   T* Cb = direct ? (T*)pr.C : part + (size_t)w.slot * BM * BN;
+  const int other_m = (int)((pr.M + BM - 1) / BM) - 1 - w.tile_m;
   for (int tile_m = w.tile_m;;) {
     const long i0 = (long)tile_m * BM;
     long k0 = w.k0, k1 = w.k1;
@@ -549,8 +552,8 @@ __global__ __launch_bounds__((GroupShape<T, TRI>::kThreads), (GroupShape<T, TRI>
     }
     gemm_tile<T, 0, TB, TRI, S>(g, i0, j0, k0, k1, Cb, direct ? pr.ldc : BN, direct ? 0 : i0, direct ? 0 : j0,
                                  direct, lds);
-    if (!TRI || w.other_m < 0 || tile_m == w.other_m) break;
-    tile_m = w.other_m;
+    if (!TRI || w.slot != kPaired || tile_m >= other_m) break;
+    tile_m = other_m;
     lds_barrier();  // the next tile restages the slabs
   }
 }
@@ -794,14 +797,13 @@ GroupPlan group_plan(int nprob, const ExcGemmProblem* P, long kchunk) {
       for (long a = 0; a < (pair ? (tm + 1) / 2 : tm); a++) {
         if (q.lower_only && a < b) continue;
         if (splits == 1 && !q.mirror) {
-          const long other = pair && 2 * a < tm - 1 ? tm - 1 - a : -1;
-          g.items.push_back(GroupItem{p, (int)a, (int)b, -1, (int)other, 0, 0, q.K});
+          g.items.push_back(GroupItem{p, (int)a, (int)b, pair ? kPaired : -1, 0, q.K});
           continue;
         }
         const long first = g.slots;
         long k0 = 0;
         do {  // an empty K too takes one item: its sum is zero
-          g.items.push_back(GroupItem{p, (int)a, (int)b, (int)(g.slots++), -1, 0, k0, std::min(q.K, k0 + chunk)});
+          g.items.push_back(GroupItem{p, (int)a, (int)b, (int)(g.slots++), k0, std::min(q.K, k0 + chunk)});
           k0 += chunk;
         } while (k0 < q.K);
         g.reds.push_back(GroupRed{p, (int)a, (int)b, (int)first, (int)(g.slots - first), 0});

@@ -196,3 +196,13 @@ def test_bidiag_workspaces_cover_fewer_values(n):
         assert hip.lib.exc_bisection_workspace(n, k) <= bisect + 256
         assert hip.lib.exc_twisted_workspace(n, k) <= twisted(k) + 256
         assert need <= bisect + 256 + twisted(k) + 256
+
+
+@pytest.mark.parametrize("m,cols,size", [(100, (600, 700), 2544896), (300, (1800, 3001, 2000), 37353216),
+                                         (512, (3072, 60000), 448344832)])
+def test_batched_workspace_keeps_its_size(m, cols, size):
+    """The batched local QR's workspace is what it was with 128 x 128 tiles alone: smaller tiles of the
+    triangular products need longer tables, but no more room."""
+    import ctypes
+    from excalibur_amd import hip
+    assert hip.lib.exc_batched_local_qr_workspace(len(cols), m, (ctypes.c_long * len(cols))(*cols)) == size
