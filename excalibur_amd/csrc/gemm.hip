@@ -74,12 +74,23 @@ constexpr int kXcds = 8;  // dies of the device; the dispatcher deals workgroups
 // of the natural order would land on eight dies with eight separate L2s. The remap gives die x a
 // contiguous range of the tile order instead, and that order runs the row tiles of one column
 // (m fastest) back to back, so their shared B column tile is fetched from HBM once per die and
-// the row tiles read it from that die's L2. Splits of K are the slowest index.
+// the row tiles read it from that die's L2. Splits of K are the slowest index, except where op(A) is
+// triangular: its splits differ in their work, so every die takes all splits of its columns (with a
+// split or two per die the first ones had 1.75 times the average work).
+template <bool TRI>
 __device__ inline void tile_of(const GemmArgs& g, long& tile_m, long& tile_n, long& split) {
   const long L = blockIdx.x;
   const long q = g.total / kXcds, r = g.total % kXcds;
   const long x = L % kXcds, j = L / kXcds;
   const long t = x * q + min(x, r) + j;
+  if (TRI) {
+    const long rows = g.pair ? (g.tm + 1) / 2 : g.tm, column = rows * (g.total / g.ntile);
+    tile_n = t / column;
+    const long u = t - tile_n * column;
+    split = u / rows;
+    tile_m = u - split * rows;
+    return;
+  }
   split = t / g.ntile;
   long u = t - split * g.ntile;
   if (g.lower_only) {
@@ -92,9 +103,8 @@ __device__ inline void tile_of(const GemmArgs& g, long& tile_m, long& tile_n, lo
     tile_n = n;
     tile_m = n + u;
   } else {
-    const long rows = g.pair ? (g.tm + 1) / 2 : g.tm;
-    tile_n = u / rows;
-    tile_m = u - tile_n * rows;
+    tile_n = u / g.tm;
+    tile_m = u - tile_n * g.tm;
   }
 }
 
@@ -303,7 +313,9 @@ struct Slab {
 };
 
 // The 128 x 128 and 64 x 64 workgroup tiles. kStep: measured time of a step on a CU with its
-// resident workgroups (us per workgroup), kAlone: with one workgroup on the CU. The MFMAs alone take
+// resident workgroups (us per workgroup), kAlone: with one workgroup on the CU; kTriStep, kTriAlone: the
+// same with a triangular op(A), whose mask costs registers (the FP64 128 x 128 kernel of A B reloads a
+// few in its loop). The MFMAs alone take
 // 1.73 / 0.43 us in FP64 and 0.86 / 0.22 us in FP32. The FP64 tile is split over eight wavefronts
 // (65.9 TFLOP/s at order 4096, 63.7 with four of 64 x 64, whose 256 registers leave two wavefronts
 // per SIMD); in FP32 four reach 129.5 at order 8192, eight 122.4. kMaxSum: terms of one running sum
@@ -316,6 +328,7 @@ struct Shapes<double> {
   using Big = Shape<double, 4, 2, 2, 4, 2, false, 2>;
   using Small = Shape<double, 2, 2, 2, 2, 4, true, 1>;
   static constexpr double kStep[2] = {1.98, 0.54}, kAlone[2] = {2.09, 0.73};
+  static constexpr double kTriStep[2] = {2.10, 0.60}, kTriAlone[2] = {2.65, 1.0};
   static constexpr long kMaxSum = 256;
   static constexpr bool kMaxSumFills = true;
 };
@@ -324,6 +337,7 @@ struct Shapes<float> {
   using Big = Shape<float, 2, 2, 4, 4, 3, true, 4>;
   using Small = Shape<float, 2, 2, 2, 2, 4, true, 4>;
   static constexpr double kStep[2] = {1.00, 0.287}, kAlone[2] = {1.18, 0.52};
+  static constexpr double kTriStep[2] = {1.09, 0.322}, kTriAlone[2] = {1.58, 0.63};
   static constexpr long kMaxSum = 2048;
   static constexpr bool kMaxSumFills = false;
 };
@@ -470,7 +484,7 @@ template <typename T, int TA, int TB, bool TRI, class S>
 __global__ __launch_bounds__(S::kThreads, S::kPerCu * S::kThreads / 256) void k_gemm(GemmArgs g) {
   __shared__ Tiles<S> lds;
   long tile_m, tile_n, split;
-  tile_of(g, tile_m, tile_n, split);
+  tile_of<TRI>(g, tile_m, tile_n, split);
   const long j0 = tile_n * S::BN;
   T* Cb = g.kchunk > 0 ? (T*)g.part + (size_t)split * g.M * g.N : (T*)g.C;
   const long ldc = g.kchunk > 0 ? g.N : g.ldc;
@@ -484,6 +498,7 @@ __global__ __launch_bounds__(S::kThreads, S::kPerCu * S::kThreads / 256) void k_
     k_range(g, tile_m * S::BM, S::BM, k0, k1);
     k0 = max(k0, ks);
     k1 = min(k1, ke);
+    if (k0 >= k1 && g.kchunk > 0) return;  // the sum of the partials passes over this one
     gemm_tile<T, TA, TB, true, S>(g, tile_m * S::BM, j0, k0, k1, Cb, ldc, 0, 0, g.kchunk == 0, lds);
     // a triangular op(A) gives row r of the tiles a K range that grows or shrinks with r: rows r and
     // tm - 1 - r together are the same work for every workgroup
@@ -589,9 +604,16 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs g, int splits) {
   const long i = idx / g.N, j = idx - i * g.N;
   if (g.lower_only && (j / g.bn) > (i / g.bm)) return;
   const T* P = (const T*)g.part;
+  int z0 = 0, z1 = splits;
+  if (g.tri != EXC_TRI_NONE) {  // the splits outside the tile's K range have no partial
+    long k0, k1;
+    k_range(g, i / g.bm * g.bm, g.bm, k0, k1);
+    z0 = (int)(k0 / g.kchunk);
+    z1 = (int)((k1 + g.kchunk - 1) / g.kchunk);
+  }
   T s = T(0);
 #pragma unroll 8
-  for (int z = 0; z < splits; z++) s += P[(size_t)z * total + idx];
+  for (int z = z0; z < z1; z++) s += P[(size_t)z * total + idx];
   T* C = (T*)g.C;
   T out = (T)g.alpha * s;
   if (g.beta != 0.0) out += (T)g.beta * C[i * g.ldc + j];
@@ -651,7 +673,10 @@ long least_splits(long M, long N, long K, long tiles, long slots, long room) {
 // takes max(w kStep, kAlone) per step; a split adds the write and the fixed-order sum of its partials
 // (about 5 TB/s, they stay in the caches) and 5 us for its launch. Splits need a workspace, and those
 // beyond the least keep two steps each (a lone step is all latency); near ties go to the larger tile and
-// fewer splits.
+// fewer splits. A triangular product takes the large tile unsplit only: split, its uneven pieces fill the
+// chip better as small ones (FP64, order 1000 in 8 splits 52 us against 58, order 2000 in 4 222 against
+// 236). Unsplit, L X with L of order 1000 and 50,000 columns takes 1.03 ms with the small tile and 1.10
+// with the large, of order 2000 and 40,000 columns 3.08 and 2.85; in FP32 567 and 565 us, 1.67 and 1.46 ms.
 template <typename T>
 GemmPlan gemm_plan(long M, long N, long K, const ExcGemmOpts& o) {
   constexpr int BK = Shapes<T>::Big::BK;
@@ -659,6 +684,9 @@ GemmPlan gemm_plan(long M, long N, long K, const ExcGemmOpts& o) {
   const long cus = compute_units();
   GemmPlan best{128, 1};
   double best_us = -1.0;
+  const bool tri = o.tri != EXC_TRI_NONE;
+  const double* step = tri ? Shapes<T>::kTriStep : Shapes<T>::kStep;
+  const double* alone = tri ? Shapes<T>::kTriAlone : Shapes<T>::kAlone;
   const long fit = o.work && K > 4 * BK ? (long)std::min<size_t>(K, o.work_bytes / ((size_t)M * N * sizeof(T))) : 1;
   const long room = std::min(fit, K / (2 * BK));
   const long tm128 = (M + 127) / 128, tn128 = (N + 127) / 128;
@@ -668,19 +696,28 @@ GemmPlan gemm_plan(long M, long N, long K, const ExcGemmOpts& o) {
     const long tile = c == 0 ? 128 : 64;
     const long tm = (M + tile - 1) / tile, tn = (N + tile - 1) / tile;
     const long tiles = o.lower_only ? tm * (tm + 1) / 2 : tm * tn;
-    // a triangular op(A) leaves the tiles about half of K on average
-    const double share = o.tri != EXC_TRI_NONE ? 0.5 + 0.5 / (double)tm : 1.0;
     const long slots = cus * (c == 0 ? Shapes<T>::Big::kPerCu : Shapes<T>::Small::kPerCu);
     const double out = (double)sizeof(T) * M * N * (o.lower_only ? 0.5 : 1.0);
-    const long most = std::max(1L, std::min(room, 2 * ((slots + tiles - 1) / tiles)));
+    const long filled = tri ? tiles / 2 + 1 : tiles;  // about half of a split triangle's tiles are empty
+    const long most = std::max(1L, std::min(room, 2 * ((slots + filled - 1) / filled)));
     long least = std::min(room, (K + kMaxSum - 1) / kMaxSum);
     if (Shapes<T>::kMaxSumFills) least = std::min(least, 2 * cus / tiles);
     least = std::max(least, floor);
     for (long sp = least; sp <= std::max(least, most); sp++) {
-      const long depth = ((K + sp - 1) / sp + BK - 1) / BK;
-      const long per_cu = (tiles * sp + cus - 1) / cus;
-      double us = 6.0 + depth * std::max(per_cu * Shapes<T>::kStep[c] * share, Shapes<T>::kAlone[c]);
-      if (sp > 1) us += 5.0 + (2 * sp + 1) * out / 5.0e6;
+      if (tri && sp > 1 && c == 0) break;
+      double depth = (double)(((K + sp - 1) / sp + BK - 1) / BK);
+      long units = tiles * sp;
+      double sums = (double)sp;
+      if (tri && sp == 1) {  // pairs of tile rows, 1 + 1 / tm of K together
+        units = (tm + 1) / 2 * tn;
+        depth *= 1.0 + 1.0 / (double)tm;
+      } else if (tri) {  // half the tiles and partials, and those on the diagonal, are not empty
+        units = (tiles * (sp + 1) + 1) / 2;
+        sums = 0.5 * (double)(sp + 1);
+      }
+      const long per_cu = (units + cus - 1) / cus;
+      double us = 6.0 + depth * std::max(per_cu * step[c], alone[c]);
+      if (sp > 1) us += 5.0 + (2 * sums + 1) * out / 5.0e6;
       if (Shapes<T>::kMaxSumFills && K > sp * kMaxSum) us *= 1.1;
       if (best_us < 0.0 || us < 0.99 * best_us) {
         best_us = us;
@@ -709,7 +746,8 @@ int gemm_impl(int ta, int tb, long M, long N, long K, double alpha, const T* A, 
               double beta, T* C, long ldc, const ExcGemmOpts& o, hipStream_t s) {
   EXC_REQUIRE(M >= 0 && N >= 0 && K >= 0 && C, EXC_ERR_ARG, "exc_gemm: bad shape");
   if (M == 0 || N == 0) return EXC_OK;
-  EXC_REQUIRE(o.tri == EXC_TRI_NONE || !tb, EXC_ERR_ARG, "exc_gemm: a triangular op(A) takes op(B) = B");
+  EXC_REQUIRE(o.tri == EXC_TRI_NONE || (!tb && !o.lower_only), EXC_ERR_ARG,
+              "exc_gemm: a triangular op(A) takes op(B) = B and a whole C");
   GemmArgs g{};
   g.M = M; g.N = N; g.K = K;
   g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc;
@@ -719,8 +757,6 @@ int gemm_impl(int ta, int tb, long M, long N, long K, double alpha, const T* A, 
   g.bm = g.bn = p.tile;
   g.tm = (M + p.tile - 1) / p.tile;
   const long tn = (N + p.tile - 1) / p.tile;
-  g.pair = !o.lower_only && o.tri != EXC_TRI_NONE;
-  g.ntile = o.lower_only ? g.tm * (g.tm + 1) / 2 : (g.pair ? (g.tm + 1) / 2 : g.tm) * tn;
   int splits = p.splits;
   if (splits > 1) {
     long chunk = (K + splits - 1) / splits;
@@ -729,6 +765,9 @@ int gemm_impl(int ta, int tb, long M, long N, long K, double alpha, const T* A, 
     g.kchunk = chunk;
     g.part = o.work;
   }
+  // an unsplit triangular product's tile rows are paired; a split one's have finer work by themselves
+  g.pair = o.tri != EXC_TRI_NONE && splits == 1;
+  g.ntile = o.lower_only ? g.tm * (g.tm + 1) / 2 : (g.pair ? (g.tm + 1) / 2 : g.tm) * tn;
   g.total = g.ntile * splits;
   EXC_REQUIRE(g.total < (1L << 31), EXC_ERR_ARG, "exc_gemm: too many tiles");
   hipEvent_t e0 = exc_prof::mark(s);

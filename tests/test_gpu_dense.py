@@ -1,4 +1,6 @@
 """GPU checks of the MFMA GEMM and the blocked factorizations against numpy (LAPACK)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -185,3 +187,148 @@ def test_gemm_sum_length(hip, f32, M, N, K, longest):
     hip.sync()
     # K and the lengths are multiples of the unit of the last place, 16
     assert np.max(K - (dC.to_host().astype(np.float64) - first)) <= longest
+
+
+class GemmOpts(ctypes.Structure):
+    """ExcGemmOpts of csrc/gemm.hpp, the products as the factorizations call them."""
+    _fields_ = [("tri", ctypes.c_int), ("lower_only", ctypes.c_int), ("mirror", ctypes.c_int),
+                ("work", ctypes.c_void_p), ("work_bytes", ctypes.c_size_t)]
+
+
+class GemmProblem(ctypes.Structure):
+    """ExcGemmProblem of csrc/gemm.hpp."""
+    _fields_ = [("A", ctypes.c_void_p), ("lda", ctypes.c_long), ("B", ctypes.c_void_p), ("ldb", ctypes.c_long),
+                ("C", ctypes.c_void_p), ("ldc", ctypes.c_long), ("M", ctypes.c_long), ("N", ctypes.c_long),
+                ("K", ctypes.c_long), ("tri", ctypes.c_int), ("lower_only", ctypes.c_int), ("mirror", ctypes.c_int),
+                ("beta_zero_hint", ctypes.c_int)]
+
+
+LOWER, UPPER = 1, 2  # EXC_TRI_A_LOWER, EXC_TRI_A_UPPER
+
+
+def internal(hip, f32, grouped=False):
+    """The internal (C++) entry points that the factorizations use."""
+    i, l, d, p = ctypes.c_int, ctypes.c_long, ctypes.c_double, ctypes.c_void_p
+    if grouped:
+        f = getattr(hip.lib, "_Z21exc_gemm_grouped_optsiiiPK14ExcGemmProblemddlPvmP12ihipStream_t")
+        f.argtypes = [i, i, i, p, d, d, l, p, ctypes.c_size_t, p]
+    else:
+        f = getattr(hip.lib, "_Z14exc_sgemm_optsiillldPKflS0_ldPflRK11ExcGemmOptsP12ihipStream_t" if f32 else
+                    "_Z13exc_gemm_optsiillldPKdlS0_ldPdlRK11ExcGemmOptsP12ihipStream_t")
+        f.argtypes = [i, i, l, l, l, d, p, l, p, l, d, p, l, p, p]
+    f.restype = i
+    return f
+
+
+def triangle(rng, m, upper, dt):
+    """A triangular factor and the same with NaN in the triangle that is not part of it."""
+    A = np.triu(rng.standard_normal((m, m))) if upper else np.tril(rng.standard_normal((m, m)))
+    A = A.astype(dt)
+    dirty = A.copy()
+    dirty[np.tril_indices(m, -1) if upper else np.triu_indices(m, 1)] = np.nan
+    return A, dirty
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("ta,tri", [(0, LOWER), (1, LOWER), (1, UPPER)])
+@pytest.mark.parametrize("m,N", [(1, 1), (3, 5), (63, 70), (64, 1), (65, 130), (129, 67), (193, 66), (257, 1025),
+                                 (321, 321), (500, 500), (1001, 999), (2049, 130), (641, 19097), (1025, 12753)])
+def test_triangular_gemm(hip, f32, ta, tri, m, N):
+    """op(A) triangular: odd and even numbers of tile rows of both tiles (the large one from about 19,097 columns at
+    order 641 and 12,753 at 1025), split and unsplit, odd leading dimensions, NaN in the triangle that is
+    not part of A. The bound is the a-priori one of the dot products in any order, here and in numpy."""
+    dt, u = (np.float32, 2.0 ** -24) if f32 else (np.float64, 2.0 ** -53)
+    s = np.dtype(dt).itemsize
+    banner(f"triangular gemm m={m} N={N} ta={ta} tri={tri} f32={f32}")
+    rng = np.random.default_rng(m + N + ta + tri)
+    A, dirty = triangle(rng, m, tri == UPPER, dt)
+    B, C = (rng.standard_normal((m, N)).astype(dt) for _ in range(2))
+    cols = np.unique(np.r_[0:min(N, 130), max(0, N - 130):N])
+    A64, B64, C64 = A.astype(np.float64), B[:, cols].astype(np.float64), C[:, cols].astype(np.float64)
+    want = -1.0 * (A64 @ B64) + C64
+    bound = (2 * m + 4) * u * (np.abs(A64) @ np.abs(B64) + np.abs(C64) + 1.0)
+    stored = np.full((m, m + 1), np.nan, dt)
+    stored[:, :m] = dirty.T if ta else dirty
+    dA, dB = hip.DeviceArray.from_host(np.append(dt(np.nan), stored)), hip.DeviceArray.from_host(B)
+    for work in (False, True):
+        dC = hip.DeviceArray.from_host(C)
+        ws = hip.workspace(hip.lib.exc_gemm_workspace(m, N, m)) if work else None
+        o = GemmOpts(tri, 0, 0, ws.ptr if work else None, ws.nbytes if work else 0)
+        assert internal(hip, f32)(ta, 0, m, N, m, -1.0, dA.ptr + s, m + 1, dB.ptr, N, 1.0, dC.ptr, N, ctypes.byref(o),
+                                  None) == 0
+        hip.sync()
+        got = dC.to_host()
+        assert np.isfinite(got).all()
+        assert (np.abs(got[:, cols] - want) <= bound).all(), work
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("m,K", [(1, 1), (65, 40), (129, 700), (200, 4099), (600, 3000)])
+def test_mirrored_gram(hip, f32, m, K):
+    """Symmetric products of which the tiles on and below the diagonal are formed and mirrored."""
+    dt, u = (np.float32, 2.0 ** -24) if f32 else (np.float64, 2.0 ** -53)
+    banner(f"mirrored gram m={m} K={K} f32={f32}")
+    X = np.random.default_rng(m + K).standard_normal((m, K)).astype(dt)
+    X64 = X.astype(np.float64)
+    dX = hip.DeviceArray.from_host(X)
+    for work in (False, True):
+        dC = hip.DeviceArray.from_host(np.full((m, m), np.nan, dt))
+        ws = hip.workspace(hip.lib.exc_gemm_workspace(m, m, K)) if work else None
+        o = GemmOpts(0, 1, 1, ws.ptr if work else None, ws.nbytes if work else 0)
+        assert internal(hip, f32)(0, 1, m, m, K, 1.0, dX.ptr, K, dX.ptr, K, 0.0, dC.ptr, m, ctypes.byref(o), None) == 0
+        hip.sync()
+        got = dC.to_host()
+        assert np.array_equal(got, got.T)
+        assert (np.abs(got - X64 @ X64.T) <= (2 * K + 4) * u * (np.abs(X64) @ np.abs(X64).T)).all()
+
+
+def test_triangular_gemm_refuses_what_it_has_no_kernel_for(hip):
+    A = hip.DeviceArray.from_host(np.eye(8))
+    C = hip.DeviceArray.from_host(np.zeros((8, 8)))
+    for tb, lower in ((1, 0), (0, 1)):
+        o = GemmOpts(LOWER, lower, 0, None, 0)
+        assert internal(hip, False)(0, tb, 8, 8, 8, 1.0, A.ptr, 8, A.ptr, 8, 0.0, C.ptr, 8, ctypes.byref(o), None) == -1
+    assert not C.to_host().any()
+
+
+@pytest.mark.parametrize("kchunk", [0, 64, 100])
+def test_grouped_products(hip, kchunk):
+    """Grouped products in FP64, whole and in chunks of K: A B with triangular A of odd orders (NaN in the other
+    triangle), and mirrored A A^T of blocks with one column and with none (whose product is zero)."""
+    banner(f"grouped products kchunk={kchunk}")
+    rng, u = np.random.default_rng(5), 2.0 ** -53
+    grouped = internal(hip, False, grouped=True)
+    size = getattr(hip.lib, "_Z26exc_gemm_grouped_workspaceiiPK14ExcGemmProbleml")
+    size.argtypes, size.restype = [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_long], ctypes.c_size_t
+
+    def run(tb, probs):
+        arr = (GemmProblem * len(probs))(*probs)
+        ws = hip.workspace(size(8, len(probs), arr, kchunk))
+        assert grouped(8, tb, len(probs), arr, 1.0, 0.0, kchunk, ws.ptr, ws.nbytes, None) == 0
+        hip.sync()
+
+    keep, probs, want, bounds = [], [], [], []
+    for m, N in ((1, 3), (63, 65), (129, 200), (193, 1), (321, 130)):
+        A, dirty = triangle(rng, m, False, np.float64)
+        B = rng.standard_normal((m, N))
+        d = [hip.DeviceArray.from_host(x) for x in (dirty, B, np.full((m, N), np.nan))]
+        keep.append(d)
+        probs.append(GemmProblem(d[0].ptr, m, d[1].ptr, N, d[2].ptr, N, m, N, m, LOWER, 0, 0, 0))
+        want.append(A @ B)
+        bounds.append((2 * m + 4) * u * (np.abs(A) @ np.abs(B)))
+    run(0, probs)
+    for d, w, b in zip(keep, want, bounds):
+        assert (np.abs(d[2].to_host() - w) <= b).all()
+
+    keep, probs, want, bounds = [], [], [], []
+    for m, K in ((129, 1), (70, 0), (65, 333), (3, 0), (200, 129)):
+        X = rng.standard_normal((m, K))
+        d = [hip.DeviceArray.from_host(X if K else np.zeros((m, 1))), hip.DeviceArray.from_host(np.full((m, m), np.nan))]
+        keep.append(d)
+        probs.append(GemmProblem(d[0].ptr, K, d[0].ptr, K, d[1].ptr, m, m, m, K, 0, 1, 1, 0))
+        want.append(X @ X.T)
+        bounds.append((2 * K + 4) * u * (np.abs(X) @ np.abs(X).T))
+    run(1, probs)
+    for d, w, b in zip(keep, want, bounds):
+        got = d[1].to_host()
+        assert np.array_equal(got, got.T) and (np.abs(got - w) <= b).all()
