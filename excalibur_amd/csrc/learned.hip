@@ -235,26 +235,26 @@ constexpr long kW1 = 0, kB1 = kW1 + (long)kIn * kHid, kW2 = kB1 + kHid, kB2 = kW
 // Caller's float arrays are read 4 at a time with no more than their elements' alignment.
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// H = relu(Z + bias) over the B x 256 layer, four columns per thread.
-__global__ __launch_bounds__(256) void k_bias_relu(long B, const float* __restrict__ Z, const float* __restrict__ bias,
+// Z += bias and H = relu(Z) over the B x 256 layer, four columns per thread.
+__global__ __launch_bounds__(256) void k_bias_relu(long B, float* __restrict__ Z, const float* __restrict__ bias,
                                                    float* __restrict__ H) {
   const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= B * (kHid / 4)) return;
   const int j = (int)(g % (kHid / 4)) * 4;
-  const f4u z = *(const f4u*)(Z + 4 * g);
-  f4u h;
+  f4u z = *(const f4u*)(Z + 4 * g), h;
 #pragma unroll
   for (int q = 0; q < 4; q++) {
-    const float v = z[q] + bias[j + q];
-    h[q] = v > 0.f ? v : 0.f;
+    z[q] += bias[j + q];
+    h[q] = z[q] > 0.f ? z[q] : 0.f;
   }
+  *(f4u*)(Z + 4 * g) = z;
   *(f4u*)(H + 4 * g) = h;
 }
 
 // The second hidden layer's bias and ReLU and the output layer in one pass: a wavefront per row,
 // four columns per lane. (As a matrix product the two output columns fill 1/64 of a tile.)
 constexpr int kHeadRows = 4;  // rows per wavefront
-__global__ __launch_bounds__(256) void k_bias_relu_head(long B, const float* __restrict__ Z,
+__global__ __launch_bounds__(256) void k_bias_relu_head(long B, float* __restrict__ Z,
                                                         const float* __restrict__ p, float* __restrict__ H,
                                                         float* __restrict__ O) {
   const int lane = threadIdx.x & 63, j = 4 * lane;
@@ -267,16 +267,16 @@ __global__ __launch_bounds__(256) void k_bias_relu_head(long B, const float* __r
     b2[q] = p[kB2 + j + q];
   }
   for (long r = r0; r < min(B, r0 + kHeadRows); r++) {
-    const f4u z = *(const f4u*)(Z + r * kHid + j);
-    f4u h;
+    f4u z = *(const f4u*)(Z + r * kHid + j), h;
     float o0 = 0.f, o1 = 0.f;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      const float v = z[q] + b2[q];
-      h[q] = v > 0.f ? v : 0.f;
+      z[q] += b2[q];
+      h[q] = z[q] > 0.f ? z[q] : 0.f;
       o0 += h[q] * w0[q];
       o1 += h[q] * w1[q];
     }
+    *(f4u*)(Z + r * kHid + j) = z;
     *(f4u*)(H + r * kHid + j) = h;
     o0 = wave_sum(o0);
     o1 = wave_sum(o1);
@@ -596,7 +596,8 @@ int exc_mlp_dims(int* d_in, int* hidden, int* d_out) {
   return EXC_OK;
 }
 
-// Activations of a batch: Z1, H1, Z2, H2 (B x 256 each) and O (B x 2), floats.
+// Activations of a batch: Z1, H1, Z2, H2 (B x 256 each) and O (B x 2), floats: the hidden layers before
+// and after their ReLU, biases added. exc_mlp_backward needs H1 and H2 and writes over Z1 and Z2.
 size_t exc_mlp_acts_floats(long B) { return (size_t)B * (4 * kHid + kOut); }
 
 int exc_mlp_forward(long B, const float* d_x, const float* d_p, float* d_acts, float* d_out, void* d_work,

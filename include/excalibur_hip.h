@@ -415,7 +415,9 @@ int exc_bisect_index(int ntg, const int* d_n, const long* d_off, const double* d
 /* The bracket network: in 32 -> 256 -> 256 -> 2, ReLU, parameters in one FP32 array of
  * exc_mlp_param_count() floats (W1 32x256, b1, W2 256x256, b2, W3 256x2, b3; row-major, inputs
  * by rows). Outputs (c, w): the target is c with Laplace scale exp(w). Training in FP32 on the
- * MFMA GEMM: exc_mlp_forward keeps the activations (exc_mlp_acts_floats(B)), exc_mlp_backward
+ * MFMA GEMM: exc_mlp_forward keeps the activations (exc_mlp_acts_floats(B): the first hidden
+ * layer before and after its ReLU, B x 256 each, then the second), exc_mlp_backward reads those after
+ * the ReLU, uses the place of those before it as scratch, and
  * writes the gradient of the mean Laplace negative log-likelihood and the loss, exc_mlp_adam
  * updates. Inference in BF16: exc_mlp_to_bf16 converts the parameters (2 bytes each),
  * exc_mlp_infer_bf16 runs a batch. No counterpart in the reference. */

@@ -79,6 +79,32 @@ def test_network_batch_edges(L, B):
     assert np.max(np.abs(net.infer(X) - want)) <= 3e-2 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("B", [1, 5, 300])
+def test_forward_keeps_the_activations(hip, B):
+    """Z1, H1, Z2, H2: each layer's sums with their bias, and their ReLU. The sums have at most 257 terms;
+    in FP32 an entry is off by at most 259 u times the sum of their magnitudes, the inputs being exact."""
+    from oracle import mlp
+    banner(f"activations batch {B}")
+    rng = np.random.default_rng(B)
+    p = mlp.init(rng).astype(np.float32)
+    p[32 * 256:32 * 256 + 256] = rng.standard_normal(256)  # biases that show
+    p[33 * 256 + 65536:33 * 256 + 65536 + 256] = rng.standard_normal(256)
+    X = rng.uniform(-1, 1, (B, 32)).astype(np.float32)
+    dp, dx = hip.DeviceArray.from_host(p), hip.DeviceArray.from_host(X)
+    da, do = hip.DeviceArray((hip.lib.exc_mlp_acts_floats(B),), np.float32), hip.DeviceArray((B, 2), np.float32)
+    hip.call("exc_mlp_forward", B, dx.ptr, dp.ptr, da.ptr, do.ptr, None, 0, None)
+    hip.sync()
+    Z1, H1, Z2, H2 = da.to_host()[:4 * B * 256].reshape(4, B, 256)
+    W1, b1 = p[:32 * 256].reshape(32, 256).astype(np.float64), p[32 * 256:33 * 256].astype(np.float64)
+    W2 = p[33 * 256:33 * 256 + 65536].reshape(256, 256).astype(np.float64)
+    b2 = p[33 * 256 + 65536:34 * 256 + 65536].astype(np.float64)
+    u = 2.0 ** -24
+    for x, W, b, Z, H in ((X, W1, b1, Z1, H1), (H1, W2, b2, Z2, H2)):
+        x = x.astype(np.float64)
+        assert (np.abs(Z - (x @ W + b)) <= 259 * u * (np.abs(x) @ np.abs(W) + np.abs(b))).all()
+        assert np.array_equal(H, np.where(Z > 0, Z, np.float32(0)))
+
+
 def gk_restated(sig, start, steps):
     """The first steps of Golub-Kahan on diag(sig) in numpy (alpha_j u_j = D v_j - beta_{j-1}
     u_{j-1}, beta_j v_{j+1} = D u_j - alpha_j v_j)."""
