@@ -328,9 +328,10 @@ int exc_bb_bidiagonal_svd(int k, const double* alpha, const double* beta, double
   EXC_REQUIRE(k >= 1 && top_k >= 0 && top_k <= k && alpha && (k == 1 || beta) && sigma &&
                   (top_k == 0 || (bidiagonal_u && bidiagonal_v)),
               EXC_ERR_ARG, "exc_bb_bidiagonal_svd: bad arguments");
-  // One allocation, one upload and (for results that fit in kStaged) one download per call: at k =
-  // 100 the six allocations, their frees and five copies took longer than the kernels (312 us the
-  // call, 278 now).
+  // One allocation and, through a host buffer for what fits in kStaged bytes, one upload and one
+  // download per call: at k = 100 the six allocations, their frees and five copies took longer than the
+  // kernels (312 us the call, 278 now). Longer arrays are copied as they lie: the buffer stays small
+  // whatever the caller passes.
   constexpr size_t kStaged = (size_t)1 << 20;
   const size_t K = (size_t)k, out = K * (size_t)top_k, head = 2 * K;
   const size_t results = ((size_t)top_k + 2 * out) * sizeof(double);
@@ -343,10 +344,16 @@ int exc_bb_bidiagonal_svd(int k, const double* alpha, const double* beta, double
   double* ds = da + head;
   double* du = ds + top_k;
   double* dv = du + out;
-  std::vector<double> h(head, 0.0);
-  std::copy(alpha, alpha + K, h.begin());
-  if (k > 1) std::copy(beta, beta + K - 1, h.begin() + K);
-  EXC_CHECK_HIP(hipMemcpy(da, h.data(), head * sizeof(double), hipMemcpyHostToDevice));
+  std::vector<double> h;
+  if (head * sizeof(double) <= kStaged) {
+    h.assign(head, 0.0);
+    std::copy(alpha, alpha + K, h.begin());
+    if (k > 1) std::copy(beta, beta + K - 1, h.begin() + K);
+    EXC_CHECK_HIP(hipMemcpy(da, h.data(), head * sizeof(double), hipMemcpyHostToDevice));
+  } else {
+    EXC_CHECK_HIP(hipMemcpy(da, alpha, K * sizeof(double), hipMemcpyHostToDevice));
+    EXC_CHECK_HIP(hipMemcpy(da + K, beta, (K - 1) * sizeof(double), hipMemcpyHostToDevice));
+  }
   int rc = exc_bidiag_svd(k, da, da + K, du, dv, ds, top_k, nullptr, dev + at_work, wb, nullptr);
   if (rc) return rc;
   if (results <= kStaged) {

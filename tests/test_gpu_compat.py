@@ -103,3 +103,24 @@ def test_virtual_mask_branch_bit_exact(bb, oracle, mask):
     got = x.copy()
     bb.block_shift_mask(3, 10001, 32, got, mask, False, 123)
     assert np.array_equal(got, want)
+
+
+def test_bidiagonal_svd_of_long_arrays(bb, hip):
+    """Arrays beyond the host staging buffer: the values of the device entry point bit for bit, and no copy
+    of the arrays in host memory (2 x 32 MB here) beside the caller's."""
+    import resource
+    banner("bidiagonal svd of long arrays")
+    n = 1 << 22
+    a, b = np.full(n, 2.0), np.full(n - 1, 0.5)  # equal rows: bounds are near, the search is short
+    bb.bidiagonal_bisection_twisted_svd(1000, a[:1000], b[:999], 0)  # the runtime's own buffers
+    before = resource.getrusage(resource.RUSAGE_SELF).ru_maxrss
+    rss = int(open("/proc/self/statm").read().split()[1]) * resource.getpagesize() // 1024
+    bb.bidiagonal_bisection_twisted_svd(n, a, b, 0)
+    after = resource.getrusage(resource.RUSAGE_SELF).ru_maxrss
+    assert after - max(before, rss) < 32 << 10
+    n = 65537
+    a, b = random_bidiagonal(np.random.default_rng(3), n, "positive")
+    u, v, s = bb.bidiagonal_bisection_twisted_svd(n, a, b, 1)
+    sg, ug, vg, _, rc = hip.bidiag_svd(a, b, 1)
+    assert rc == 0
+    assert np.array_equal(s, sg) and np.array_equal(u, ug) and np.array_equal(v, vg)
