@@ -84,10 +84,11 @@ def test_virtual_matrix_mask_bit_exact(hip, oracle, m, n, is_left):
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("is_left", [True, False])
 @pytest.mark.parametrize("K,lines", [(2, 1), (127, 771), (128, 385), (130, 1540), (1025, 3), (1026, 387), (2048, 5),
-                                     (2051, 2), (4096, 3), (4099, 2), (9001, 2)])
+                                     (2051, 2), (4096, 3), (4099, 2), (9001, 2), (1026, 771), (2051, 771), (4099, 771)])
 def test_givens_shape_edges(hip, K, lines, is_left, f32):
-    """Line counts around the strips of 1, 2, 4 and 8 lines and pair counts around the threads of one
-    wavefront, one pair per thread, two, and more than the registers hold; bit for bit."""
+    """Line counts around the strips of 1, 2 and (in FP32) 4 lines and pair counts around the threads of one
+    wavefront, one pair per thread, two, and more than the registers hold, each with narrow and wide strips;
+    bit for bit."""
     banner(f"givens K={K} lines={lines} left={is_left} f32={f32}")
     dt = np.float32 if f32 else np.float64
     x = np.random.default_rng(K + lines).standard_normal((K, lines) if is_left else (lines, K)).astype(dt)
