@@ -72,20 +72,6 @@ struct Quad {
   __device__ int col(int b) const { return 16 * b + li; }
 };
 
-// acc <- the nr x nc tile of A at (r0, c0), zero outside.
-__device__ __forceinline__ void acc_load(d4 (&acc)[4][4], const Quad& q, const double* A, long lda, long r0, long c0, int nr,
-                         int nc) {
-#pragma unroll
-  for (int a = 0; a < 4; a++)
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int r = q.row(a, v), c = q.col(b);
-        acc[a][b][v] = (r < nr && c < nc) ? A[(r0 + r) * lda + c0 + c] : 0.0;
-      }
-}
-
 // S (LDS, 64 x 65) <- acc
 __device__ __forceinline__ void acc_to_lds(const d4 (&acc)[4][4], const Quad& q, double* S) {
 #pragma unroll
@@ -114,14 +100,6 @@ __device__ __forceinline__ void tile_to_lds(double* T, const double* A, long lda
   }
 }
 
-// T (LDS) <- the transpose of the nr x nc tile of A at (r0, c0), zero outside.
-__device__ __forceinline__ void tile_to_lds_t(double* T, const double* A, long lda, long r0, long c0, int nr, int nc) {
-  for (int e = threadIdx.x; e < TB * TB; e += TNT) {
-    const int r = e >> 6, c = e & 63;
-    T[c * LD + r] = (r < nr && c < nc) ? A[(r0 + r) * lda + c0 + c] : 0.0;
-  }
-}
-
 // The nr x nc tile of A at (r0, c0) <- S (LDS); lower_zero writes zeros above the diagonal.
 // Coherent stores: other workgroups read the finished tile.
 __device__ __forceinline__ void lds_to_tile(const double* S, double* A, long lda, long r0, long c0, int nr, int nc, bool lower_zero) {
@@ -131,8 +109,7 @@ __device__ __forceinline__ void lds_to_tile(const double* S, double* A, long lda
   }
 }
 
-// acc -= X Y^T (TRANS_Y) or X Y, X and Y 64 x 64 in LDS.
-template <bool TRANS_Y>
+// acc -= X Y, X and Y 64 x 64 in LDS.
 __device__ __forceinline__ void acc_update(d4 (&acc)[4][4], const Quad& q, const double* X, const double* Y) {
 #pragma unroll 2
   for (int kk = 0; kk < TB; kk += 4) {
@@ -140,8 +117,7 @@ __device__ __forceinline__ void acc_update(d4 (&acc)[4][4], const Quad& q, const
 #pragma unroll
     for (int a = 0; a < 4; a++) xa[a] = -X[(16 * a + q.li) * LD + kk + q.lk];
 #pragma unroll
-    for (int b = 0; b < 4; b++)
-      yb[b] = TRANS_Y ? Y[(16 * b + q.li) * LD + kk + q.lk] : Y[(kk + q.lk) * LD + 16 * b + q.li];
+    for (int b = 0; b < 4; b++) yb[b] = Y[(kk + q.lk) * LD + 16 * b + q.li];
 #pragma unroll
     for (int a = 0; a < 4; a++)
 #pragma unroll
@@ -174,7 +150,7 @@ __device__ inline void wave_sync() {
 // Every element receives the same fused multiply-adds in the same order as a column-by-column
 // right-looking factorization.
 //
-// The routine runs once per diagonal tile on one wavefront, so every instruction is fetched cold:
+// The routine runs once per diagonal tile of a workgroup, so every instruction is fetched cold:
 // a fully unrolled form (tens of KB of straight-line code) was bound by instruction fetch, not
 // arithmetic. So only a panel of PW columns is unrolled (inside it the pivot and the multipliers
 // L[k][j] reach the other lanes by v_readlane, no LDS, no barrier); the panel loop is not. The
@@ -306,11 +282,10 @@ __device__ __forceinline__ void getf2_loop(double* S, int kb, double* sgn, bool 
   }
 }
 
-// Off-diagonal tile solves against the final diagonal tile, read from HBM with wave-uniform
-// addresses (the flag's acquire made it visible): ROWS: lane = row r of S, S[r] <- S[r] op(D)^-1
-// (LOWER_T: op(D) = L^T, Cholesky; else U, LU); else lane = column c, S[:, c] <- L^-1 S[:, c]
-// with L the unit lower part of D (LU) or (MODE 3) the lower triangle of the tile the caller
-// staged in T (triangular inverse).
+// Off-diagonal tile solves against the diagonal tile D, on one wavefront. Modes 0 and 1: lane = row r of S,
+// S[r] <- S[r] op(D)^-1 with op(D) = L^T (Cholesky) or U (LU); modes 2 and 3: lane = column c,
+// S[:, c] <- L^-1 S[:, c] with L the unit lower part of D (LU) or its lower triangle (triangular inverse).
+// Mode 0 reads D from HBM at Dg; in the others the caller staged it in T.
 template <int MODE>  // 0: rows, L^T; 1: rows, U; 2: columns, unit L; 3: columns, L
 __device__ __forceinline__ void tile_solve(double* S, double* T, const double* Dg, long lda, int kd) {
   // The diagonal tile was finished by another workgroup. Except in the Cholesky mode the caller
@@ -367,10 +342,10 @@ __host__ __device__ inline int chol_index(int i, int j, int nb) { return j * nb 
 // The one-wavefront tile spends most of a diagonal step outside the factorization itself: the last
 // 64 x 64 x 64 update (256 MFMAs), staging the tiles it needs and storing the finished tile. Here
 // wavefront w holds rows 16w .. 16w + 15 of the tile (four 16 x 16 MFMA blocks), so the updates,
-// the staging and the stores split four ways; the in-register factorization and the solve, chains
-// of dependent operations on 64 rows, stay on wavefront 0. Every block receives the same MFMAs in
-// the same order as in the one-wavefront form, and the factorization and solve are the same code,
-// so the factor is bit-identical.
+// the staging, the stores and the updates inside a diagonal tile split four ways; the panels of its
+// factorization and the solve, chains of dependent operations on 64 rows, stay on wavefront 0. Every
+// element receives the same operations in the same order as in the one-wavefront form, so the factor
+// is bit-identical.
 constexpr int TNT4 = 256;
 
 // element v of lane l of block b of wavefront w: row 16w + (l / 16) + 4v, column 16b + l % 16
@@ -536,7 +511,7 @@ __global__ __launch_bounds__(TNT) void k_trinv_tiles_batched(int n, const double
     tile_to_lds(P, L, ldl, r0, (long)k * TB, nr, kc);   // L(i, k)
     tile_to_lds(Q, Xo, ldx, (long)k * TB, c0, kc, nc);  // X(k, j), finished by another workgroup
     __syncthreads();
-    acc_update<false>(acc, q, P, Q);
+    acc_update(acc, q, P, Q);
     __syncthreads();
   }
   acc_to_lds(acc, q, S);
@@ -584,7 +559,7 @@ __device__ __forceinline__ void acc_update4_nn(d4 (&acc)[4], const Quad4& q, con
 }
 
 // Four wavefronts per tile, as in the Cholesky: updates, staging and stores split four ways, the
-// factorization and the solve on wavefront 0. Order 1000: 1.52 ms with one wavefront and the
+// factorization's panels and the solve on wavefront 0. Order 1000: 1.52 ms with one wavefront and the
 // unrolled factorization, 0.87 ms now.
 __global__ __launch_bounds__(TNT4) void k_lu_tiles(int n, double* __restrict__ A, long lda, int nb,
                                                    double* __restrict__ sgn, int square_last,
