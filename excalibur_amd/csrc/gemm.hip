@@ -8,8 +8,9 @@
 // x 2000 (156 alone, 149 the library); with scalar loads behind branches, whose merged registers
 // waited for every load at once, 55 and 46.6, 111 and 105. Options used by the factorizations: split-K
 // (partial tiles summed in a fixed order by a second kernel, so results do not depend on
-// scheduling), skipping the zero K range of a triangular operand, and computing only the lower
-// tiles of a symmetric product (mirrored into the upper half by the reduction).
+// scheduling), skipping the zero K range of a triangular op(A), and computing only the lower tiles of a
+// symmetric product (mirrored into the upper half by a kernel of its own, in grouped products by the
+// reduction).
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -317,8 +318,8 @@ struct Slab {
 // same with a triangular op(A), whose mask costs registers (the FP64 128 x 128 kernel of A B reloads a
 // few in its loop). The MFMAs alone take
 // 1.73 / 0.43 us in FP64 and 0.86 / 0.22 us in FP32. The FP64 tile is split over eight wavefronts
-// (65.9 TFLOP/s at order 4096, 63.7 with four of 64 x 64, whose 256 registers leave two wavefronts
-// per SIMD); in FP32 four reach 129.5 at order 8192, eight 122.4. kMaxSum: terms of one running sum
+// (four of 64 x 64, whose 256 registers leave two wavefronts per SIMD, are 3 % slower at order 4096); in
+// FP32 eight are 5 % slower than four at order 8192. kMaxSum: terms of one running sum
 // (its rounding error grows with them) beyond which K is split as far as the workspace allows and,
 // in FP64 (kMaxSumFills), as far as two workgroups per CU (and a plan that stays above it counts 10 % more).
 template <typename T>

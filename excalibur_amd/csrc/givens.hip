@@ -14,8 +14,8 @@
 // stored line-fastest, a pair's two elements are one LDS word of up to 16 bytes each, and the plan
 // entry is read once per strip, straight into registers and two passes ahead of its use (it was
 // staged in LDS and read again for every line). A strip that one wavefront covers needs no barrier:
-// a wavefront's LDS operations complete in order. Both sides of a 1000 x 1000 FP64 mask: 139 -> 57
-// us, 2000 x 2000 FP32: 360 -> 103, 100 x 100: 64 -> 19 (HBM would take 3.3, 6.7 and 0.05 us).
+// a wavefront's LDS operations complete in order. Both sides of a 1000 x 1000 FP64 mask: 139 -> 52
+// us, 2000 x 2000 FP32: 358 -> 97, 100 x 100: 64 -> 19 (HBM would take 3.3, 6.7 and 0.05 us).
 #include <algorithm>
 #include <type_traits>
 
@@ -182,8 +182,8 @@ __global__ __launch_bounds__(kMaxThreads) void k_givens_batched(T* const* __rest
 // Shape of a sweep: threads (a pair each, two above 512 pairs so that a thread's LDS accesses
 // overlap) and the lines of a strip: as many as make a 16-byte word, while the strips still cover
 // three quarters of the CUs and fit in LDS. (With 32-byte words the 1000 x 1000 mask has one strip
-// per CU and nothing runs while it waits at its barriers: 72 us against 57; with 256 threads of two
-// pairs each instead of 512 of one, 83.)
+// per CU and nothing runs while it waits at its barriers: 26 % slower; with 256 threads of two pairs
+// each instead of 512 of one, 46 %.)
 struct Sweep {
   int threads, np, l;
 };

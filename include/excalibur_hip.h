@@ -142,7 +142,9 @@ int exc_block_shift_mask(double* d_x, long m, long n, long passes, int mask, int
 /* C = alpha op(A) op(B) + beta C, row-major, op = transpose when trans_* != 0. FP64 on
  * v_mfma_f64_16x16x4_f64 (the reference's cblas_dgemm calls, client.cpp:1018, 1179, 1190);
  * FP32 on v_mfma_f32_16x16x4_f32 for the mixed-precision form. d_work (nullable) enables
- * split-K for short-and-deep products; exc_gemm_workspace() bounds what it may use. */
+ * split-K for short-and-deep products, up to as many partial results as work_bytes holds: the number of
+ * splits, and with it the rounding, depends on its size. exc_gemm_workspace() is 8 FP64 or 16 FP32
+ * partials. */
 size_t exc_gemm_workspace(long M, long N, long K);
 int exc_dgemm(int trans_a, int trans_b, long M, long N, long K, double alpha, const double* d_a, long lda,
               const double* d_b, long ldb, double beta, double* d_c, long ldc, void* d_work, size_t work_bytes,
@@ -371,15 +373,16 @@ int exc_givens_apply_batched(int nb, double* const* d_xs, long m, long n, const 
  * block X_b (m x cols[b] row-major FP64, cols[b] >= m; host array of device pointers h_x) R_b^T
  * (m x m lower, positive diagonal) into h_rt[b] and, when h_qt is given, Q_b^T (m x cols[b]) into
  * h_qt[b]. A shifted CholeskyQR whose first pass runs in FP32 on the MFMA (all blocks' Gram
- * matrices in one grouped launch, its K chunk chosen by the library's autotuner), refined by FP64 passes (grouped launches); the m x m factorizations run one
- * workgroup per block in one launch. h_stats (nullable, 3 nb doubles): per block the FP32 shift,
+ * matrices in one grouped launch, its K chunk chosen by the library's autotuner), refined by FP64
+ * passes (grouped launches); the m x m factorizations of all blocks run in one launch, a workgroup per
+ * 64 x 64 tile. h_stats (nullable, 3 nb doubles): per block the FP32 shift,
  * max |Z Z^T - I| before the last FP64 pass and the number of FP64 passes. Synchronizes. No
  * counterpart in the reference, which runs one peer per process. */
 size_t exc_batched_local_qr_workspace(int nb, int m, const long* h_cols);
 int exc_batched_local_qr(int nb, int m, const long* h_cols, const double* const* h_x, double* const* h_rt,
                          double* const* h_qt, double* h_stats, void* d_work, size_t work_bytes, exc_stream_t stream);
 /* The grouped GEMM autotuner's choices so far (JSON list of {dtype, problems, sum_k, kchunk, grid,
- * ms}). */
+ * ms}; grid: workgroups). */
 int exc_gemm_grouped_tuning(char* buf, size_t cap);
 
 /* ---------------------------------------------------------------- learned bisection brackets */
